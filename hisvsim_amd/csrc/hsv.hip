@@ -54,8 +54,8 @@ struct hsv_state {
   hipStream_t stream = nullptr;
   void* gate_buf = nullptr;        // device copy of the current part's gates
   size_t gate_buf_bytes = 0;
-  double* partial = nullptr;       // device reduction partials
-  std::vector<double> host_partial;
+  double* partial = nullptr;       // device reduction partials (the chain's folded renormalisation; made at its first use)
+  double* host_partial = nullptr;  // the read-outs' partials, pinned host memory that the kernels write
   // Event pairs around each timed launch (a pool reused across collections).
   std::vector<std::pair<hipEvent_t, hipEvent_t>> events;
   size_t events_used = 0;
@@ -644,15 +644,13 @@ int launch_tile_part(hsv_state* s, const std::vector<Lowered>& Ls, uint64_t part
 }
 
 template <typename R, int MODE>
-int reduce_t(hsv_state* a, hsv_state* b, int qubit, double* out0, double* out1) {
+int reduce_t(hsv_state* a, hsv_state* b, double* out0, double* out1) {
   auto* pa = amp_as<R>(a);
   auto* pb = b ? amp_as<R>(b) : nullptr;
   int blocks = kRedBlocks;
   if (MODE == RD_CHUNK) blocks = (int)std::min<uint64_t>(kRedBlocks, a->len);
-  hipLaunchKernelGGL((k_reduce<R, MODE>), blocks, kRedBlock, 0, a->stream, pa, pb, a->len, qubit, a->partial);
+  hipLaunchKernelGGL((k_reduce<R, MODE>), blocks, kRedBlock, 0, a->stream, pa, pb, a->len, a->host_partial);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(a->host_partial.data(), a->partial, sizeof(double) * 2 * blocks, hipMemcpyDeviceToHost,
-                        a->stream));
   HIPCHK(hipStreamSynchronize(a->stream));
   if (MODE == RD_CHUNK) return blocks;
   double s0 = 0, s1 = 0;
@@ -666,8 +664,49 @@ int reduce_t(hsv_state* a, hsv_state* b, int qubit, double* out0, double* out1) 
 }
 
 template <int MODE>
-int reduce(hsv_state* a, hsv_state* b, int qubit, double* o0, double* o1) {
-  return a->dtype == HSV_C128 ? reduce_t<double, MODE>(a, b, qubit, o0, o1) : reduce_t<float, MODE>(a, b, qubit, o0, o1);
+int reduce(hsv_state* a, hsv_state* b, double* o0, double* o1) {
+  return a->dtype == HSV_C128 ? reduce_t<double, MODE>(a, b, o0, o1) : reduce_t<float, MODE>(a, b, o0, o1);
+}
+
+// Workgroups of a one-state read-out over `count` items (a power of two):
+// four items per thread until the chip is full (sum_items).
+int sum_grid(uint64_t count) {
+  return (int)std::max<uint64_t>(1, std::min<uint64_t>(kSumBlocks, count / (4 * kRedBlock)));
+}
+int sum_partials(hsv_state* s, int grid, double* out) {
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(s->stream));
+  double t = 0;
+  for (int i = 0; i < grid; ++i) t += s->host_partial[2 * i];
+  *out = t;
+  return HSV_OK;
+}
+
+// sum |a_i|^2 over the amplitudes with bit `qubit` zero; all with qubit < 0
+template <typename R>
+int mass0_t(hsv_state* s, int qubit, double* out) {
+  // units of the half that is read (qubit 0 of complex64 is inside a unit)
+  const uint64_t count = (s->len >> Unit<R>::LOG) >> (qubit >= Unit<R>::LOG);
+  const int grid = sum_grid(count);
+  hipLaunchKernelGGL((k_mass0<R>), grid, kRedBlock, 0, s->stream, amp_as<R>(s), count, qubit, s->host_partial);
+  return sum_partials(s, grid, out);
+}
+int mass0(hsv_state* s, int qubit, double* out) {
+  return s->dtype == HSV_C128 ? mass0_t<double>(s, qubit, out) : mass0_t<float>(s, qubit, out);
+}
+
+// the sum of a Pauli string without its factor (see k_pauli_z, k_pauli_x)
+template <typename R>
+int pauli_t(hsv_state* s, uint64_t x, uint64_t z, double* out) {
+  const uint64_t units = s->len >> Unit<R>::LOG;
+  const uint64_t count = (x >> Unit<R>::LOG) ? units / 2 : units;
+  const int grid = sum_grid(count);
+  if (x)
+    hipLaunchKernelGGL((k_pauli_x<R>), grid, kRedBlock, 0, s->stream, amp_as<R>(s), count, x, z,
+                       __builtin_popcountll(x & z) & 1, s->host_partial);
+  else
+    hipLaunchKernelGGL((k_pauli_z<R>), grid, kRedBlock, 0, s->stream, amp_as<R>(s), count, z, s->host_partial);
+  return sum_partials(s, grid, out);
 }
 
 int lower_all(const hsv_gate* gates, int num_gates, std::vector<Lowered>* out, const hsv_state* s) {
@@ -715,6 +754,11 @@ static int permute_in_place(hsv_state* s, const int* new_slot, bool renorm = fal
     moves2 = moves2 || s2[q] != q;
   }
   renorm = renorm && moves1 && moves2;
+  if (renorm && !s->partial &&
+      hipMalloc(reinterpret_cast<void**>(&s->partial), sizeof(double) * 2 * kRedBlocks) != hipSuccess) {
+    s->partial = nullptr;
+    return fail(HSV_ERR_ALLOC, "cannot allocate reduction scratch");
+  }
   if (int rc = begin_timed(s)) return rc;
   for (const std::vector<int>* sp : {&s1, &s2}) {
     const std::vector<int>& sig = *sp;
@@ -884,10 +928,8 @@ int hsv_create(int num_qubits, int dtype, hsv_state** out) {
   int dev = 0;
   HIPCHK(hipGetDevice(&dev));
   s->device = dev;
-  hipDeviceProp_t prop;
-  HIPCHK(hipGetDeviceProperties(&prop, dev));
-  s->max_lds = (int)prop.sharedMemPerBlock;
-  s->num_cu = prop.multiProcessorCount;
+  HIPCHK(hipDeviceGetAttribute(&s->max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+  HIPCHK(hipDeviceGetAttribute(&s->num_cu, hipDeviceAttributeMultiprocessorCount, dev));
   if (hipStreamCreate(&s->stream) != hipSuccess) { delete s; return fail(HSV_ERR_DEVICE, "hipStreamCreate failed"); }
   if (hipMalloc(&s->amp, s->len * s->elem()) != hipSuccess) {
     hipStreamDestroy(s->stream);
@@ -895,13 +937,12 @@ int hsv_create(int num_qubits, int dtype, hsv_state** out) {
     return fail(HSV_ERR_ALLOC, "cannot allocate " + std::to_string(s->len * (dtype == HSV_C128 ? 16 : 8)) +
                                    " bytes of device memory for the state");
   }
-  if (hipMalloc(reinterpret_cast<void**>(&s->partial), sizeof(double) * 2 * kRedBlocks) != hipSuccess) {
+  if (hipHostMalloc(reinterpret_cast<void**>(&s->host_partial), sizeof(double) * 2 * kSumBlocks, 0) != hipSuccess) {
     hipFree(s->amp);
     hipStreamDestroy(s->stream);
     delete s;
     return fail(HSV_ERR_ALLOC, "cannot allocate reduction scratch");
   }
-  s->host_partial.resize(2 * kRedBlocks);
   *out = s;
   return hsv_reset(s);
 }
@@ -910,7 +951,8 @@ int hsv_destroy(hsv_state* s) {
   if (!s) return HSV_OK;
   hipStreamSynchronize(s->stream);
   hipFree(s->amp);
-  hipFree(s->partial);
+  if (s->partial) (void)hipFree(s->partial);
+  (void)hipHostFree(s->host_partial);
   if (s->gate_buf) hipFree(s->gate_buf);
   if (s->fused_scratch.ptr) hipFree(s->fused_scratch.ptr);
   for (auto& e : s->events) {
@@ -1227,28 +1269,28 @@ int hsv_write(hsv_state* s, uint64_t offset, uint64_t count, const double* host_
 
 int hsv_norm2(hsv_state* s, double* out) {
   if (!s || !out) return fail(HSV_ERR_ARG, "null argument");
-  return reduce<RD_NORM2>(s, nullptr, 0, out, nullptr);
+  return mass0(s, -1, out);
 }
 
 int hsv_inner(hsv_state* a, hsv_state* b, double* out2) {
   if (!a || !b || !out2) return fail(HSV_ERR_ARG, "null argument");
   if (a->n != b->n || a->dtype != b->dtype) return fail(HSV_ERR_ARG, "states differ in size or dtype");
   HIPCHK(hipStreamSynchronize(b->stream));
-  return reduce<RD_INNER>(a, b, 0, &out2[0], &out2[1]);
+  return reduce<RD_INNER>(a, b, &out2[0], &out2[1]);
 }
 
 int hsv_max_abs_diff(hsv_state* a, hsv_state* b, double* out) {
   if (!a || !out) return fail(HSV_ERR_ARG, "null argument");
   if (b && (a->n != b->n || a->dtype != b->dtype)) return fail(HSV_ERR_ARG, "states differ in size or dtype");
   if (b) HIPCHK(hipStreamSynchronize(b->stream));
-  return reduce<RD_MAXDIFF>(a, b, 0, out, nullptr);
+  return reduce<RD_MAXDIFF>(a, b, out, nullptr);
 }
 
 int hsv_probability(hsv_state* s, int qubit, int value, double* out) {
   if (!s || !out || qubit < 0 || qubit >= s->n || (value != 0 && value != 1))
     return fail(HSV_ERR_ARG, "bad qubit or value");
   double p0 = 0;
-  if (int rc = reduce<RD_PROB0>(s, nullptr, qubit, &p0, nullptr)) return rc;
+  if (int rc = mass0(s, qubit, &p0)) return rc;
   *out = value == 0 ? p0 : 1.0 - p0;
   return HSV_OK;
 }
@@ -1257,7 +1299,7 @@ int hsv_renormalize(hsv_state* s, double* norm2_before) {
   if (!s) return fail(HSV_ERR_ARG, "null handle");
   s->basis0 = false;
   double n2 = 0;
-  if (int rc = reduce<RD_NORM2>(s, nullptr, 0, &n2, nullptr)) return rc;
+  if (int rc = mass0(s, -1, &n2)) return rc;
   if (norm2_before) *norm2_before = n2;
   if (!(n2 > 0.0)) return fail(HSV_ERR_ARG, "cannot renormalise a zero state");
   const double scale = 1.0 / std::sqrt(n2);
@@ -1279,13 +1321,11 @@ int hsv_project(hsv_state* s, uint64_t qubit_mask, uint64_t values, double* p_ou
   const int blocks = kRedBlocks;
   if (s->dtype == HSV_C128)
     hipLaunchKernelGGL((k_mass<double>), blocks, kRedBlock, 0, s->stream, amp_as<double>(s), s->len, qubit_mask,
-                       values, s->partial);
+                       values, s->host_partial);
   else
     hipLaunchKernelGGL((k_mass<float>), blocks, kRedBlock, 0, s->stream, amp_as<float>(s), s->len, qubit_mask,
-                       values, s->partial);
+                       values, s->host_partial);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(s->host_partial.data(), s->partial, sizeof(double) * 2 * blocks, hipMemcpyDeviceToHost,
-                        s->stream));
   HIPCHK(hipStreamSynchronize(s->stream));
   double p = 0;
   for (int i = 0; i < blocks; ++i) p += s->host_partial[2 * i];
@@ -1306,29 +1346,14 @@ int hsv_project(hsv_state* s, uint64_t qubit_mask, uint64_t values, double* p_ou
 int hsv_expect_pauli(hsv_state* s, uint64_t x_mask, uint64_t z_mask, double* out2) {
   if (!s || !out2) return fail(HSV_ERR_ARG, "null argument");
   if ((x_mask | z_mask) >> s->n) return fail(HSV_ERR_ARG, "Pauli mask names a qubit beyond the state");
-  const int blocks = kRedBlocks;
-  if (s->dtype == HSV_C128)
-    hipLaunchKernelGGL((k_pauli<double>), blocks, kRedBlock, 0, s->stream, amp_as<double>(s), s->len, x_mask,
-                       z_mask, s->partial);
-  else
-    hipLaunchKernelGGL((k_pauli<float>), blocks, kRedBlock, 0, s->stream, amp_as<float>(s), s->len, x_mask,
-                       z_mask, s->partial);
-  HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(s->host_partial.data(), s->partial, sizeof(double) * 2 * blocks, hipMemcpyDeviceToHost,
-                        s->stream));
-  HIPCHK(hipStreamSynchronize(s->stream));
-  double re = 0, im = 0;
-  for (int i = 0; i < blocks; ++i) {
-    re += s->host_partial[2 * i];
-    im += s->host_partial[2 * i + 1];
-  }
-  // multiply by i^ny, ny = number of Y factors
-  switch (__builtin_popcountll(x_mask & z_mask) & 3) {
-    case 0: out2[0] = re; out2[1] = im; break;
-    case 1: out2[0] = -im; out2[1] = re; break;
-    case 2: out2[0] = -re; out2[1] = -im; break;
-    default: out2[0] = im; out2[1] = -re; break;
-  }
+  double t = 0;
+  if (int rc = s->dtype == HSV_C128 ? pauli_t<double>(s, x_mask, z_mask, &t) : pauli_t<float>(s, x_mask, z_mask, &t))
+    return rc;
+  // with X or Y: 2 t (ny even) or 2i t (ny odd), ny = number of Y factors,
+  // times i^ny: real, 2 t for ny = 0, 3 and -2 t for ny = 1, 2 (mod 4)
+  const int ny = __builtin_popcountll(x_mask & z_mask) & 3;
+  out2[0] = !x_mask ? t : (ny == 0 || ny == 3) ? 2 * t : -2 * t;
+  out2[1] = 0.0;
   return HSV_OK;
 }
 
@@ -1343,8 +1368,8 @@ int hsv_measure(hsv_state* s, const int* qubits, int num_qubits, const double* u
   std::sort(u.begin(), u.end());
   // Probability mass per contiguous chunk, then the reference's sequential
   // walk (state_vector.hpp:946-972) inside the chunks the samples land in.
-  int blocks = s->dtype == HSV_C128 ? reduce_t<double, RD_CHUNK>(s, nullptr, 0, nullptr, nullptr)
-                                    : reduce_t<float, RD_CHUNK>(s, nullptr, 0, nullptr, nullptr);
+  int blocks = s->dtype == HSV_C128 ? reduce_t<double, RD_CHUNK>(s, nullptr, nullptr, nullptr)
+                                    : reduce_t<float, RD_CHUNK>(s, nullptr, nullptr, nullptr);
   if (blocks < 0) return blocks;
   const uint64_t chunk = s->len / blocks;
   std::vector<double> amps(2 * chunk);

@@ -290,14 +290,17 @@ __global__ __launch_bounds__(BS) void k_part(typename VecT<R>::type* __restrict_
 }
 
 // ---- reductions (FP64 accumulation, fixed grid -> deterministic) -----------
-enum { RD_NORM2 = 0, RD_INNER = 1, RD_MAXDIFF = 2, RD_PROB0 = 3, RD_CHUNK = 4 };
+// Every reduction writes one pair of doubles per block to `partial`, which is
+// pinned host memory: the host adds them after the stream's synchronisation,
+// with no copy in between (a copy of the partials took 15 us of a read-out).
+enum { RD_INNER = 1, RD_MAXDIFF = 2, RD_CHUNK = 4 };
 constexpr int kRedBlocks = 1024;
 constexpr int kRedBlock = 256;
 
 template <typename R, int MODE>
 __global__ __launch_bounds__(kRedBlock) void k_reduce(const typename VecT<R>::type* __restrict__ a,
                                                       const typename VecT<R>::type* __restrict__ b,
-                                                      uint64_t len, int qubit, double* __restrict__ partial) {
+                                                      uint64_t len, double* __restrict__ partial) {
   double s0 = 0.0, s1 = 0.0;
   if constexpr (MODE == RD_CHUNK) {
     const uint64_t chunk = len / gridDim.x;
@@ -310,11 +313,7 @@ __global__ __launch_bounds__(kRedBlock) void k_reduce(const typename VecT<R>::ty
     const uint64_t stride = uint64_t(gridDim.x) * kRedBlock;
     for (uint64_t i = uint64_t(blockIdx.x) * kRedBlock + threadIdx.x; i < len; i += stride) {
       const double x = a[i].x, y = a[i].y;
-      if constexpr (MODE == RD_NORM2) {
-        s0 += x * x + y * y;
-      } else if constexpr (MODE == RD_PROB0) {
-        if (!((i >> qubit) & 1)) s0 += x * x + y * y;
-      } else if constexpr (MODE == RD_INNER) {
+      if constexpr (MODE == RD_INNER) {
         const double u = b[i].x, v = b[i].y;
         s0 += x * u + y * v;   // Re(conj(a) b)
         s1 += x * v - y * u;   // Im(conj(a) b)
@@ -345,37 +344,133 @@ __global__ __launch_bounds__(kRedBlock) void k_reduce(const typename VecT<R>::ty
   }
 }
 
-// <psi|P|psi> for a Pauli string: P|j> = i^ny (-1)^popc(j & z) |j ^ x>, so the
-// sum is i^ny * sum_j conj(a[j ^ x]) a[j] (-1)^popc(j & z); the host applies
-// i^ny. Same fixed grid and partials layout as k_reduce.
+// The one-state read-outs below go through the state in 16-byte units (one
+// complex128 or two complex64 amplitudes), four loads in flight per thread on
+// a grid that fills the chip (kSumBlocks workgroups, 8 per CU), and load only
+// what the result depends on. They are bound by HBM: a two-qubit
+// XX or YY term of a 28-qubit complex64 state (2.1 GB) takes 366 us (5.9
+// TB/s; with one thread per amplitude, every pair read twice, 610), a ZZ term
+// 398; P(0) of a 31-qubit complex128 state (17 GB of its 34) 3.7 ms against
+// 4.8 with the whole state's loop.
+constexpr int kSumBlocks = 2048;
+
 template <typename R>
-__global__ __launch_bounds__(kRedBlock) void k_pauli(const typename VecT<R>::type* __restrict__ a, uint64_t len,
-                                                     uint64_t xmask, uint64_t zmask, double* __restrict__ partial) {
-  double s0 = 0.0, s1 = 0.0;
+struct Unit {
+  static constexpr int N = 16 / (2 * sizeof(R));
+  static constexpr int LOG = N - 1;
+  typename VecT<R>::type a[N];
+  __device__ __forceinline__ double mass(int b) const {
+    return double(a[b].x) * double(a[b].x) + double(a[b].y) * double(a[b].y);
+  }
+};
+template <typename R>
+__device__ __forceinline__ Unit<R> load_unit(const typename VecT<R>::type* a, uint64_t u) {
+  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(Unit<R>, reinterpret_cast<const u4*>(a)[u]);
+}
+
+// w with a zero bit inserted at position pv (none when pv < 0)
+__device__ __forceinline__ uint64_t insert_zero(uint64_t w, int pv) {
+  if (pv < 0) return w;
+  const uint64_t lo = w & ((1ull << pv) - 1);
+  return ((w ^ lo) << 1) | lo;
+}
+
+// f(w) summed over w < count, as partial[2 * block]. count and the grid are
+// powers of two, so with 4 * 256 * grid <= count every thread has the same
+// number of groups of four; smaller counts run on one block.
+template <typename F>
+__device__ __forceinline__ void sum_items(uint64_t count, double* __restrict__ partial, F f) {
   const uint64_t stride = uint64_t(gridDim.x) * kRedBlock;
-  for (uint64_t j = uint64_t(blockIdx.x) * kRedBlock + threadIdx.x; j < len; j += stride) {
-    const double x = a[j].x, y = a[j].y;
-    const uint64_t k = j ^ xmask;
-    const double u = a[k].x, v = a[k].y;
-    const double sg = (__popcll(j & zmask) & 1) ? -1.0 : 1.0;
-    s0 += sg * (u * x + v * y);   // Re(conj(a_k) a_j)
-    s1 += sg * (u * y - v * x);   // Im(conj(a_k) a_j)
-  }
-  __shared__ double r0[kRedBlock], r1[kRedBlock];
-  r0[threadIdx.x] = s0;
-  r1[threadIdx.x] = s1;
-  __syncthreads();
-  for (int h = kRedBlock / 2; h > 0; h >>= 1) {
-    if (threadIdx.x < h) {
-      r0[threadIdx.x] += r0[threadIdx.x + h];
-      r1[threadIdx.x] += r1[threadIdx.x + h];
+  uint64_t w = uint64_t(blockIdx.x) * kRedBlock + threadIdx.x;
+  double s[4] = {0.0, 0.0, 0.0, 0.0};
+  if (count >= 4 * stride) {
+    for (; w < count; w += 4 * stride) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) s[j] += f(w + j * stride);
     }
-    __syncthreads();
+  } else {
+    for (; w < count; w += stride) s[0] += f(w);
   }
+  double t = (s[0] + s[1]) + (s[2] + s[3]);
+  for (int m = 32; m >= 1; m >>= 1) t += __shfl_xor(t, m);
+  __shared__ double r[kRedBlock / 64];
+  if ((threadIdx.x & 63) == 0) r[threadIdx.x >> 6] = t;
+  __syncthreads();
   if (threadIdx.x == 0) {
-    partial[2 * blockIdx.x] = r0[0];
-    partial[2 * blockIdx.x + 1] = r1[0];
+    partial[2 * blockIdx.x] = (r[0] + r[1]) + (r[2] + r[3]);
+    partial[2 * blockIdx.x + 1] = 0.0;
   }
+}
+
+// sum |a_i|^2 over the amplitudes with bit `qubit` zero (all with qubit < 0):
+// only that half of the state is read.
+template <typename R>
+__global__ __launch_bounds__(kRedBlock) void k_mass0(const typename VecT<R>::type* __restrict__ a, uint64_t count,
+                                                     int qubit, double* __restrict__ partial) {
+  const int pv = qubit - Unit<R>::LOG;  // the qubit's bit of the unit index
+  const bool inside = Unit<R>::N == 2 && qubit == 0;
+  sum_items(count, partial, [&](uint64_t w) {
+    const Unit<R> x = load_unit<R>(a, insert_zero(w, qubit < 0 ? -1 : pv));
+    double p = x.mass(0);
+    if constexpr (Unit<R>::N == 2) p += inside ? 0.0 : x.mass(1);
+    return p;
+  });
+}
+
+// <psi|P|psi> for a Pauli string: P|j> = i^ny (-1)^popc(j & z) |j ^ x>, so the
+// sum is i^ny * sum_j conj(a[j ^ x]) a[j] (-1)^popc(j & z). Without X or Y
+// (x = 0) that is sum_j |a[j]|^2 (-1)^popc(j & z): k_pauli_z. Otherwise the
+// terms of j and j ^ x are conjugates of each other up to the sign (-1)^ny,
+// so each pair is read once and gives twice the real part (ny even) or 2i
+// times the imaginary part (ny odd) of conj(a[j ^ x]) a[j]: k_pauli_x sums
+// that part over the j with the highest bit of x zero, and the host applies
+// the factor.
+template <typename R>
+__global__ __launch_bounds__(kRedBlock) void k_pauli_z(const typename VecT<R>::type* __restrict__ a, uint64_t count,
+                                                       uint64_t zmask, double* __restrict__ partial) {
+  sum_items(count, partial, [&](uint64_t u) {
+    const Unit<R> x = load_unit<R>(a, u);
+    double p = x.mass(0);
+    if constexpr (Unit<R>::N == 2) p += (zmask & 1) ? -x.mass(1) : x.mass(1);
+    return (__popcll(u & (zmask >> Unit<R>::LOG)) & 1) ? -p : p;
+  });
+}
+
+template <typename V>
+__device__ __forceinline__ double conj_part(V ak, V aj, bool imag) {
+  const double u = ak.x, v = ak.y, x = aj.x, y = aj.y;
+  return imag ? u * y - v * x : u * x + v * y;
+}
+
+template <typename R>
+__global__ __launch_bounds__(kRedBlock) void k_pauli_x(const typename VecT<R>::type* __restrict__ a, uint64_t count,
+                                                       uint64_t xmask, uint64_t zmask, int imag,
+                                                       double* __restrict__ partial) {
+  const uint64_t xu = xmask >> Unit<R>::LOG, zu = zmask >> Unit<R>::LOG;
+  if (xu == 0) {  // x = 1 on complex64: both partners in one unit
+    sum_items(count, partial, [&](uint64_t u) {
+      const Unit<R> p = load_unit<R>(a, u);
+      const double t = conj_part(p.a[Unit<R>::N - 1], p.a[0], imag);
+      return (__popcll(u & zu) & 1) ? -t : t;
+    });
+    return;
+  }
+  const int pv = 63 - __clzll(xu);
+  sum_items(count, partial, [&](uint64_t w) {
+    const uint64_t u = insert_zero(w, pv);
+    const Unit<R> p = load_unit<R>(a, u), q = load_unit<R>(a, u ^ xu);
+    double t;
+    if constexpr (Unit<R>::N == 2) {
+      const bool sw = xmask & 1;
+      const double t0 = conj_part(sw ? q.a[1] : q.a[0], p.a[0], imag);
+      const double t1 = conj_part(sw ? q.a[0] : q.a[1], p.a[1], imag);
+      t = t0 + ((zmask & 1) ? -t1 : t1);
+    } else {
+      t = conj_part(q.a[0], p.a[0], imag);
+    }
+    return (__popcll(u & zu) & 1) ? -t : t;
+  });
 }
 
 // Probability mass of the amplitudes with (i & mask) == value.

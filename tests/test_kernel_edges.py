@@ -27,3 +27,39 @@ def test_mlp_contractions_at_tile_edges(in_features, hidden, n):
     assert abs(loss - rl) <= 1e-4 * rl
     assert np.abs(g - rg).max() <= 1e-4 * max(1.0, np.abs(rg).max())
     m.close()
+
+
+def _stored(n, dtype, seed):
+    rng = np.random.default_rng(seed)
+    a = rng.normal(size=2 ** n) + 1j * rng.normal(size=2 ** n)
+    a /= np.linalg.norm(a)
+    return a if dtype == "complex128" else a.astype(np.complex64).astype(complex)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+@pytest.mark.parametrize("n", [1, 2, 3, 9, 10, 11, 13, 20])
+def test_read_outs_at_unit_and_grid_edges(n, dtype):
+    """Norm, P(0) of every qubit and Pauli strings (no X, X on the lowest
+    qubit alone, on the highest alone, random) where a state is less than a
+    16-byte unit's block, one block, several. At most 64 roundings of partial
+    sums below 1 in a row: 1e-14, and the sums in numpy as much again."""
+    from hisvsim_amd import capi
+    from oracle.oracle import pauli_expectation
+    a = _stored(n, dtype, n)
+    p = np.abs(a) ** 2
+    i = np.arange(2 ** n)
+    rng = np.random.default_rng(n + 50)
+    full = 2 ** n - 1
+    strings = [(0, 1), (0, full), (1, 0), (1, 1), (1, full), (1 << (n - 1), 0), (full, full)]
+    strings += [(int(rng.integers(0, 2 ** n)), int(rng.integers(0, 2 ** n))) for _ in range(12)]
+    with capi.State(n, dtype) as s:
+        s.write(a)
+        assert abs(s.norm2() - p.sum()) <= 1e-13
+        for q in range(n):
+            p0 = p[(i >> q) & 1 == 0].sum()
+            assert abs(s.probability(q, 0) - p0) <= 1e-13
+            assert abs(s.probability(q, 1) - (1 - p0)) <= 1e-13
+        for x, z in strings:
+            want = pauli_expectation(a, x, z)
+            assert abs(s.expectation((x, z)) - want.real) <= 1e-13, (x, z)
