@@ -10,6 +10,7 @@
 #include <array>
 #include <atomic>
 #include <chrono>
+#include <cmath>
 #include <mutex>
 #include <cstring>
 #include <string>
@@ -84,6 +85,11 @@ struct hsv_state {
   // that may change it): the chain then skips the tiles that are still zero.
   bool basis0 = false;
   DeviceScratch fused_scratch;       // fused unitary + offset tables
+  // hsv_measure on the device (made at its first use): the walked chunks'
+  // sub-block sums; the lists and answers that its kernels read and write in
+  // pinned host memory
+  uint64_t* walk_sub = nullptr;
+  void* walk_host = nullptr;
   size_t elem() const { return dtype == HSV_C128 ? 16 : 8; }
 };
 
@@ -709,6 +715,271 @@ int pauli_t(hsv_state* s, uint64_t x, uint64_t z, double* out) {
   return sum_partials(s, grid, out);
 }
 
+// The measurement walk: the reference's sequential walk over cumulative
+// probabilities (state_vector.hpp:946-972) inside the chunks the samples land
+// in, the other chunks passed by their mass. States of kWalkHostLen
+// amplitudes or less are read back whole and walked here; on wider ones the
+// chunks' serial sums and the samples' places come from the device (see
+// k_walk_sums), bit for bit the walk's, and only the sub-blocks that its
+// integers do not cover (the first one from cum = 0, a change of binade, an
+// exact tie) are read back and walked here. A chunk read back and walked
+// costs about 12 us and 2 ns an amplitude, the device's two launches and
+// waits about 60 us: kWalkDeviceUs is where they meet. Shots of the whole
+// register of a complex128 state, every walked chunk read back and walked
+// here -> this: 1000 shots at 24 qubits (i.i.d. amplitudes) 22 -> 0.4 ms; on a
+// product state at 18 / 28 qubits 10 shots 0.21 -> 0.09 / 2.3 -> 1.2 ms, 1000
+// shots 3.2 -> 0.14 / 11.4 -> 1.2 ms.
+constexpr double kWalkDeviceUs = 60.0;
+constexpr uint64_t kWalkHostLen = 1ull << 14;
+
+struct Walk {
+  hsv_state* s;
+  const int* qubits;
+  int num_qubits;
+  const std::vector<double>& u;  // sorted
+  int32_t* out;
+  uint64_t chunk;                // amplitudes per chunk
+  int sp = 0;                    // samples placed
+  double cum = 0;
+  std::vector<double> amps = {};
+  std::vector<uint64_t> fetched = {};   // sub-blocks of fetch_len amplitudes whose masses are at hand
+  uint64_t fetch_len = 0;
+  const double* fetched_mass = nullptr;
+  std::vector<WalkFind> finds = {};
+  std::vector<int> find_sample = {};
+
+  int samples() const { return (int)u.size(); }
+  void place(int sample, uint64_t pos) {
+    for (int j = 0; j < num_qubits; ++j) out[sample * num_qubits + j] = (int32_t)((pos >> qubits[j]) & 1);
+  }
+  void step(double p, uint64_t pos) {
+    while (sp < samples() && u[sp] < cum + p) place(sp++, pos);
+    cum += p;
+  }
+  // the walk over `len` amplitudes from `base`, at `a`, fetched or read back
+  int serial(uint64_t base, uint64_t len, const double* a = nullptr) {
+    for (size_t f = 0; !a && f < fetched.size(); ++f) {
+      if (fetched[f] != base || len != fetch_len) continue;
+      for (uint64_t i = 0; i < len && sp < samples(); ++i) step(fetched_mass[f * len + i], base + i);
+      return HSV_OK;
+    }
+    if (!a) {
+      amps.resize(2 * len);
+      if (int rc = hsv_read(s, base, len, amps.data())) return rc;
+      a = amps.data();
+    }
+    for (uint64_t i = 0; i < len && sp < samples(); ++i) {
+      const double x = a[2 * i], y = a[2 * i + 1];
+      step(x * x + y * y, base + i);
+    }
+    return HSV_OK;
+  }
+  // whether the walk's next `sum0` / `sum1` ulps (lower / upper binade of the
+  // row's scale) stay inside one binade; the samples in that stretch are
+  // listed for k_walk_find and cum moves to its end
+  bool stretch(const WalkChunk& W, uint64_t sum0, uint64_t sum1, uint64_t base, int row) {
+    if (!(cum > 0.0) || (sum0 & kWalkFlag)) return false;
+    for (int sel = 0; sel < 2; ++sel) {
+      const double scale = sel ? 0.5 * W.scale : W.scale, c = cum * scale;
+      if (!(c >= 4503599627370496.0 && c < 9007199254740992.0)) continue;  // 2^52 .. 2^53: cum's binade
+      const uint64_t c0 = (uint64_t)c, end = c0 + (sel ? sum1 : sum0);
+      if (end > (1ull << 53)) return false;
+      const double cum_end = (double)end / scale;
+      for (; sp < samples() && u[sp] < cum_end; ++sp) {
+        const double t = std::floor(u[sp] * scale);
+        finds.push_back(WalkFind{base, c0, t < 0.0 ? 0 : (uint64_t)t + 1, scale, row, sel});
+        find_sample.push_back(sp);
+      }
+      cum = cum_end;
+      return true;
+    }
+    return false;
+  }
+
+  template <typename R>
+  int find(int nsub) {
+    auto* list = reinterpret_cast<WalkFind*>(static_cast<unsigned char*>(s->walk_host) + kFindOff);
+    auto* pos = reinterpret_cast<uint64_t*>(static_cast<unsigned char*>(s->walk_host) + kPosOff);
+    for (size_t f0 = 0; f0 < finds.size(); f0 += kWalkFindBatch) {
+      const int cnt = (int)std::min<size_t>(kWalkFindBatch, finds.size() - f0);
+      std::copy(finds.begin() + f0, finds.begin() + f0 + cnt, list);
+      std::fill(pos, pos + cnt, ~0ull);
+      hipLaunchKernelGGL((k_walk_find<R>), cnt, 256, 0, s->stream, amp_as<R>(s), chunk / nsub, nsub, list, s->walk_sub,
+                         pos);
+      HIPCHK(hipGetLastError());
+      HIPCHK(hipStreamSynchronize(s->stream));
+      for (int i = 0; i < cnt; ++i) {
+        if (pos[i] >= s->len) return fail(HSV_ERR_DEVICE, "measurement walk: a sample was not found");
+        place(find_sample[f0 + i], pos[i]);
+      }
+    }
+    return HSV_OK;
+  }
+
+  template <typename R>
+  int device(const std::vector<double>& mass) {
+    const int blocks = (int)mass.size();
+    // the chunks the walk is expected to go through, by the masses alone
+    std::vector<int> walked;
+    std::vector<double> start;
+    {
+      int q = 0;
+      double c = 0;
+      for (int b = 0; b < blocks && q < samples(); ++b) {
+        const double end = c + mass[b];
+        if (u[q] < end) {
+          walked.push_back(b);
+          start.push_back(c);
+          while (q < samples() && u[q] < end) ++q;
+        }
+        c = end;
+      }
+    }
+    std::vector<int> row0(blocks, 0), rows_of(blocks, 0);
+    std::vector<uint64_t> total;  // per row, both binades
+    int nrows = 0, nsub = 1;
+    const WalkChunk* rows_in = nullptr;
+    const uint64_t* sums = nullptr;
+    if (double(walked.size()) * (12.0 + 0.002 * double(chunk)) > kWalkDeviceUs) {
+      if (!s->walk_sub &&
+          hipMalloc(reinterpret_cast<void**>(&s->walk_sub), sizeof(uint64_t) * 2 * kWalkSums) != hipSuccess) {
+        s->walk_sub = nullptr;
+        return fail(HSV_ERR_ALLOC, "cannot allocate the measurement's sums");
+      }
+      if (!s->walk_host && hipHostMalloc(&s->walk_host, kHostBytes, 0) != hipSuccess) {
+        s->walk_host = nullptr;
+        return fail(HSV_ERR_ALLOC, "cannot allocate the measurement's lists");
+      }
+      auto* rows = static_cast<WalkChunk*>(s->walk_host);
+      auto* sums_out = reinterpret_cast<uint64_t*>(static_cast<unsigned char*>(s->walk_host) + kSumOff);
+      rows_in = rows;
+      sums = sums_out;
+      // rows of two binades each, from the one of the chunk's start (a little
+      // below it: the start is known to rounding) to the one of its end, the
+      // upper eight where they are more
+      for (size_t w = 0; w < walked.size(); ++w) {
+        const int b = walked[w];
+        const double end = (start[w] + mass[b]) * (1.0 + 1e-9);
+        if (!(end < 1e300 && end > 1e-200)) continue;
+        int e0 = 0, e1 = 0;
+        std::frexp(end, &e1);
+        std::frexp(start[w] * (1.0 - 1e-9), &e0);  // start in [2^(e0-1), 2^e0)
+        e0 = start[w] > 0.0 ? std::max(e0, e1 - 7) : e1 - 7;
+        row0[b] = nrows;
+        for (int e = e0; e <= e1 && nrows < kWalkRows; e += 2) {
+          // below 2^62 ulps (at most 8 binades), so that no sum overflows
+          rows[nrows++] = WalkChunk{(uint64_t)b, std::ldexp(1.0, 53 - e)};
+        }
+        rows_of[b] = nrows - row0[b];
+      }
+      while (nsub < kWalkSub && chunk / nsub > 64 && 2 * nsub * nrows <= kWalkSums) nsub *= 2;
+      if (nrows) {
+        hipLaunchKernelGGL((k_walk_sums<R>), dim3(nrows, (nsub + 3) / 4), 256, 0, s->stream, amp_as<R>(s), chunk, nsub,
+                           rows, s->walk_sub, sums_out);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipStreamSynchronize(s->stream));
+        total.resize(2 * nrows);
+        for (int r = 0; r < nrows; ++r) {
+          uint64_t t0 = 0, t1 = 0, flags = 0;
+          for (const uint64_t* p = sums + size_t(r) * nsub * 2; p < sums + size_t(r + 1) * nsub * 2; p += 2) {
+            flags |= p[0] & kWalkFlag;
+            t0 += p[0] & ~kWalkFlag;
+            t1 += p[1];
+          }
+          total[2 * r] = t0 | flags;
+          total[2 * r + 1] = t1;
+        }
+      }
+    }
+    // the walk; expected: only the sub-blocks that it will have to go through
+    // here, cum moved past them by their sums
+    std::vector<uint64_t> need;
+    const uint64_t sb = chunk / nsub;
+    auto walk = [&](bool expected) -> int {
+      sp = 0;
+      cum = 0;
+      finds.clear();
+      find_sample.clear();
+      for (int b = 0; b < blocks && sp < samples(); ++b) {
+        if (!(u[sp] < cum + mass[b])) { cum += mass[b]; continue; }
+        const uint64_t base = uint64_t(b) * chunk;
+        const int r0 = row0[b], nr = rows_of[b];
+        if (!nr) {
+          if (!expected) {
+            if (int rc = serial(base, chunk)) return rc;
+            continue;
+          }
+          cum += mass[b];
+          while (sp < samples() && u[sp] < cum) ++sp;
+          continue;
+        }
+        if (nr == 1 && stretch(rows_in[r0], total[2 * r0], total[2 * r0 + 1], base, r0)) continue;
+        int read_back = 0;
+        for (int j = 0; j < nsub && sp < samples(); ++j) {
+          const uint64_t* sum = sums + (size_t(r0) * nsub + j) * 2;
+          bool done = false;
+          for (int r = 0; r < nr && !done; ++r)
+            done = stretch(rows_in[r0 + r], sum[size_t(r) * nsub * 2], sum[size_t(r) * nsub * 2 + 1], base + j * sb, -1);
+          if (done) continue;
+          // after a few sub-blocks the rest of the chunk in one read (ties
+          // throughout, say)
+          const bool rest = ++read_back > 3;
+          if (!expected) {
+            if (int rc = serial(base + j * sb, rest ? chunk - j * sb : sb)) return rc;
+          } else if (!rest) {
+            need.push_back(base + j * sb);
+            cum += (double)(sum[0] & ~kWalkFlag) / rows_in[r0].scale;
+            while (sp < samples() && u[sp] < cum) ++sp;
+          }
+          if (rest) break;
+        }
+      }
+      return HSV_OK;
+    };
+    if (nrows) {
+      if (int rc = walk(true)) return rc;
+      fetch_len = sb;
+      need.resize(std::min<size_t>(need.size(), std::min<uint64_t>(kWalkFetch, kWalkFetched / sb)));
+      if (!need.empty()) {
+        auto* bases = reinterpret_cast<uint64_t*>(static_cast<unsigned char*>(s->walk_host) + kPosOff);
+        auto* got = reinterpret_cast<double*>(static_cast<unsigned char*>(s->walk_host) + kFetchOff);
+        std::copy(need.begin(), need.end(), bases);
+        const int grid = (int)std::min<uint64_t>((sb + 255) / 256, 64);
+        hipLaunchKernelGGL((k_walk_fetch<R>), dim3(grid, (unsigned)need.size()), 256, 0, s->stream, amp_as<R>(s), sb,
+                           bases, got);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipStreamSynchronize(s->stream));
+        fetched = need;
+        fetched_mass = got;
+      }
+    }
+    if (int rc = walk(false)) return rc;
+    return find<R>(nsub);
+  }
+
+  int run(int blocks) {
+    std::vector<double> mass(blocks);
+    for (int b = 0; b < blocks; ++b) mass[b] = s->host_partial[2 * b];
+    if (s->len > kWalkHostLen) return s->dtype == HSV_C128 ? device<double>(mass) : device<float>(mass);
+    std::vector<double> a(2 * s->len);
+    if (int rc = hsv_read(s, 0, s->len, a.data())) return rc;
+    for (int b = 0; b < blocks && sp < samples(); ++b) {
+      if (!(u[sp] < cum + mass[b])) { cum += mass[b]; continue; }
+      if (int rc = serial(uint64_t(b) * chunk, chunk, a.data() + 2 * uint64_t(b) * chunk)) return rc;
+    }
+    return HSV_OK;
+  }
+
+  // walk_host: the rows of k_walk_sums, their sums, the samples of one
+  // k_walk_find launch, their places (before that the sub-blocks to fetch), the
+  // fetched masses
+  static constexpr size_t kSumOff = sizeof(WalkChunk) * kWalkRows;
+  static constexpr size_t kFindOff = kSumOff + sizeof(uint64_t) * 2 * kWalkSums;
+  static constexpr size_t kPosOff = kFindOff + sizeof(WalkFind) * kWalkFindBatch;
+  static constexpr size_t kFetchOff = kPosOff + sizeof(uint64_t) * kWalkFindBatch;
+  static constexpr size_t kHostBytes = kFetchOff + sizeof(double) * kWalkFetched;
+};
+
 int lower_all(const hsv_gate* gates, int num_gates, std::vector<Lowered>* out, const hsv_state* s) {
   out->resize(num_gates);
   for (int i = 0; i < num_gates; ++i) {
@@ -953,6 +1224,8 @@ int hsv_destroy(hsv_state* s) {
   hipFree(s->amp);
   if (s->partial) (void)hipFree(s->partial);
   (void)hipHostFree(s->host_partial);
+  if (s->walk_sub) (void)hipFree(s->walk_sub);
+  if (s->walk_host) (void)hipHostFree(s->walk_host);
   if (s->gate_buf) hipFree(s->gate_buf);
   if (s->fused_scratch.ptr) hipFree(s->fused_scratch.ptr);
   for (auto& e : s->events) {
@@ -1366,31 +1639,13 @@ int hsv_measure(hsv_state* s, const int* qubits, int num_qubits, const double* u
   if (!num_samples) return HSV_OK;
   std::vector<double> u(uniforms, uniforms + num_samples);
   std::sort(u.begin(), u.end());
-  // Probability mass per contiguous chunk, then the reference's sequential
-  // walk (state_vector.hpp:946-972) inside the chunks the samples land in.
-  int blocks = s->dtype == HSV_C128 ? reduce_t<double, RD_CHUNK>(s, nullptr, nullptr, nullptr)
-                                    : reduce_t<float, RD_CHUNK>(s, nullptr, nullptr, nullptr);
+  // Probability mass per contiguous chunk, then the walk.
+  const int blocks = s->dtype == HSV_C128 ? reduce_t<double, RD_CHUNK>(s, nullptr, nullptr, nullptr)
+                                          : reduce_t<float, RD_CHUNK>(s, nullptr, nullptr, nullptr);
   if (blocks < 0) return blocks;
-  const uint64_t chunk = s->len / blocks;
-  std::vector<double> amps(2 * chunk);
-  double cum = 0;
-  int sp = 0;
-  for (int c = 0; c < blocks && sp < num_samples; ++c) {
-    const double mass = s->host_partial[2 * c];
-    if (!(u[sp] < cum + mass)) { cum += mass; continue; }
-    if (int rc = hsv_read(s, uint64_t(c) * chunk, chunk, amps.data())) return rc;
-    for (uint64_t i = 0; i < chunk && sp < num_samples; ++i) {
-      const double x = amps[2 * i], y = amps[2 * i + 1];
-      const double p = x * x + y * y;
-      const uint64_t pos = uint64_t(c) * chunk + i;
-      while (sp < num_samples && u[sp] < cum + p) {
-        for (int j = 0; j < num_qubits; ++j) out[sp * num_qubits + j] = (int32_t)((pos >> qubits[j]) & 1);
-        ++sp;
-      }
-      cum += p;
-    }
-  }
-  for (; sp < num_samples; ++sp)  // mass exhausted: the reference reports all ones (:973-980)
+  Walk W{s, qubits, num_qubits, u, out, s->len / blocks};
+  if (int rc = W.run(blocks)) return rc;
+  for (int sp = W.sp; sp < num_samples; ++sp)  // mass exhausted: the reference reports all ones (:973-980)
     for (int j = 0; j < num_qubits; ++j) out[sp * num_qubits + j] = 1;
   return HSV_OK;
 }

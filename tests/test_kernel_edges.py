@@ -63,3 +63,50 @@ def test_read_outs_at_unit_and_grid_edges(n, dtype):
         for x, z in strings:
             want = pauli_expectation(a, x, z)
             assert abs(s.expectation((x, z)) - want.real) <= 1e-13, (x, z)
+
+
+def _walk_states():
+    """(name, n, dtype, amplitudes) where the measurement walk's integer sums
+    can go wrong: one wavefront's chunk and several, changes of binade at and
+    inside chunks, exact ties, empty chunks, all mass in one amplitude."""
+    out = []
+    for n, dtype in ((14, "complex128"), (15, "complex128"), (15, "complex64"), (16, "complex128"),
+                     (18, "complex64"), (20, "complex128")):
+        out.append(("gaussian", n, dtype, _stored(n, dtype, n)))
+    out.append(("uniform", 16, "complex128", np.full(2 ** 16, 2.0 ** -8, complex)))
+    a = np.zeros(2 ** 15, complex)
+    a[0], a[1:] = np.sqrt(0.5), 2.0 ** -27     # each |a|^2 half an ulp of the sum so far
+    out.append(("ties", 15, "complex128", a))
+    a = _stored(17, "complex128", 3)
+    a[: 2 ** 15] = 0
+    a[2 ** 16: 2 ** 16 + 2 ** 14] = 0
+    out.append(("gaps", 17, "complex128", a))
+    a = _stored(16, "complex128", 4) * 2.0 ** -12
+    a[40000] = 1.0
+    out.append(("peak", 16, "complex128", a))
+    out.append(("large", 16, "complex128", _stored(16, "complex128", 5) * 3.0))   # norm^2 = 9
+    return out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,n,dtype,a", _walk_states(), ids=lambda v: v if isinstance(v, str) else "")
+def test_measurement_walk_is_the_serial_sum(name, n, dtype, a):
+    """Uniforms on and just below the serial FP64 sum, in every chunk (so that
+    every chunk with mass is walked and the sum is serial from 0): the outcome
+    is the first amplitude whose sum exceeds the uniform, to the last bit."""
+    from hisvsim_amd import capi
+    p = a.real * a.real + a.imag * a.imag
+    cum = np.cumsum(p)
+    rng = np.random.default_rng(n)
+    chunk = max(1, 2 ** n // 1024)
+    at = (np.arange(0, 2 ** n, chunk)[:, None] + rng.integers(0, chunk, (2 ** n // chunk, 3))).ravel()
+    edge = np.concatenate([np.arange(chunk - 1, 2 ** n, chunk), at])
+    u = np.sort(np.concatenate([cum[edge], np.nextafter(cum[edge], 0.0), [0.0, -0.5, cum[-1] * 1.01]]))
+    # a chunk without a uniform below its end would be passed by its mass
+    want = np.searchsorted(cum, u, side="right")
+    with capi.State(n, dtype) as s:
+        s.write(a)
+        got = s.measure(list(range(n)), u) @ (1 << np.arange(n))
+    inside = want < 2 ** n
+    assert np.array_equal(got[inside], want[inside])
+    assert np.all(got[~inside] == 2 ** n - 1)
