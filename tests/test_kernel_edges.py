@@ -110,3 +110,36 @@ def test_measurement_walk_is_the_serial_sum(name, n, dtype, a):
     inside = want < 2 ** n
     assert np.array_equal(got[inside], want[inside])
     assert np.all(got[~inside] == 2 ** n - 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(13, 512), (12, 256), (8, 128), (11, 512)])
+def test_qaoa_passes_at_chunk_edges(orc, shape):
+    """Instances of one chunk (whole in LDS, 13 qubits in registers), just
+    wider (a high chunk over all but a few qubits), with every split of a
+    13-qubit chunk into low and high qubits up to the widest the shape takes;
+    no layer to four; angles on both sides of |cos b| = |sin b| (odd and even
+    numbers of layers past it) and at 0, pi/2 and pi. <C> and the state
+    against the CPU oracle: complex64 states, the bars of the batch's tests."""
+    from hisvsim_amd.qaoa import Instance, QAOABatch, circuit, cut_values, random_3regular
+    bits, threads = shape
+    rng = np.random.default_rng(bits)
+    insts = []
+    for n in sorted({2, 3, 4, bits - 1, bits, bits + 1, bits + 2, bits + 4, min(bits + 6, 17), 13, 14}):
+        edges = random_3regular(n, rng) if n >= 4 else [(0, n - 1)]
+        for p in range(5):
+            betas = [float(x) for x in rng.uniform(0, np.pi, p)]
+            insts.append(Instance(n, edges, [float(x) for x in rng.uniform(0, np.pi, p)], betas))
+        insts.append(Instance(n, edges, [0.3, 0.9, 1.7], [0.0, np.pi / 2, np.pi]))
+    with QAOABatch(insts) as b:
+        b.tune("chunk_bits", bits)
+        b.tune("threads", threads)
+        for _ in range(2):
+            got = b.run()
+        for i, inst in enumerate(insts):
+            amps = np.zeros(2 ** inst.n, complex)
+            amps[0] = 1
+            orc.apply_gates(amps, circuit(inst))
+            want = float(np.sum(np.abs(amps) ** 2 * cut_values(inst.n, inst.edges)))
+            assert abs(got[i] - want) <= 1e-5 * max(1.0, abs(want)), (inst.n, inst.p)
+            assert np.abs(b.state(i) - amps).max() <= 2e-6, (inst.n, inst.p)
