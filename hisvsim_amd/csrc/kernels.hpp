@@ -1275,7 +1275,7 @@ __device__ __forceinline__ uint32_t tile_thread_bits(uint32_t regmask) {
 // NTH threads: per segment, each thread reads the 2^RB values of its
 // register layout (RB = KT - log2 NTH), applies the segment's gates (rounds
 // or gate records) and writes them back in place.
-__device__ __forceinline__ uint32_t tile_sw(uint32_t t) { return t ^ (((t >> 4) ^ (t >> 8)) & 15u); }
+__host__ __device__ __forceinline__ uint32_t tile_sw(uint32_t t) { return t ^ (((t >> 4) ^ (t >> 8)) & 15u); }
 constexpr int tile_log2(int x) { return x <= 1 ? 0 : 1 + tile_log2(x >> 1); }
 
 template <typename R, int KT, int NTH>

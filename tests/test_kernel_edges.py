@@ -143,3 +143,67 @@ def test_qaoa_passes_at_chunk_edges(orc, shape):
             want = float(np.sum(np.abs(amps) ** 2 * cut_values(inst.n, inst.edges)))
             assert abs(got[i] - want) <= 1e-5 * max(1.0, abs(want)), (inst.n, inst.p)
             assert np.abs(b.state(i) - amps).max() <= 2e-6, (inst.n, inst.p)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+@pytest.mark.parametrize("n,qubits", [(12, (0,)), (12, (5, 7, 8, 9, 10, 11)), (12, (0, 1, 2, 3, 4, 5, 6)),
+                                      (13, (0, 4, 8, 12)), (13, (1, 5, 9, 2, 12)), (14, (3, 7, 11, 12, 13)),
+                                      (15, (8, 9, 10, 11, 12, 13, 14)), (16, (0, 2, 6, 10, 13, 14, 15))])
+def test_fused_f64_steps_match_the_gates(n, qubits, dtype):
+    """The FP64 fused path as 4-qubit steps on a tile (part qubits below, in
+    and above the tile's low slots, all bank classes as rows, the smallest
+    state), and where it stays one dense product (a gate on five qubits, more
+    steps than the product is worth), against the gates one by one: 1e-12,
+    complex64 states at their rounding of one pass, 2^-24 times the largest
+    amplitude a few times over."""
+    from hisvsim_amd import capi
+    from hisvsim_amd.circuit import Gate
+    rng = np.random.default_rng(n * 100 + len(qubits))
+    a = _stored(n, dtype, 7)
+    lists = []
+    for count in (1, 4, 12, 40):
+        gs = []
+        for _ in range(count):
+            q = [int(x) for x in rng.permutation(qubits)]
+            th = [float(x) for x in rng.uniform(0, 6, 3)]
+            gs.append(Gate("U3", (q[0],), (), tuple(th)))
+            if len(q) > 1:
+                gs += [Gate("Z", (q[1],), (q[0],)), Gate("R1", (q[0],), (q[1],), (th[0],)),
+                       Gate("RZZ", (q[0], q[1]), (), (th[1],)), Gate("SWAP", (q[1], q[0]))]
+            if len(q) > 3:
+                gs.append(Gate("RY", (q[3],), (q[0], q[1], q[2]), (th[2],)))
+        lists.append(gs)
+    if len(qubits) > 4:
+        lists.append(lists[1] + [Gate("X", (qubits[0],), tuple(qubits[1:5]))])
+    tol = 1e-12 if dtype == "complex128" else 2.0 ** -20 * np.abs(a).max()
+    with capi.State(n, dtype) as s, capi.State(n, "complex128") as r:
+        for gs in lists:
+            s.write(a)
+            s.apply_fused(gs, "f64")
+            r.write(a)
+            r.apply_gates(gs)
+            assert np.abs(s.read() - r.read()).max() <= tol
+
+
+@pytest.mark.gpu
+def test_fused_f64_unitarity_is_the_parts():
+    """Accepted and refused as before: a gate that is not unitary followed by
+    its inverse is a unitary part; alone it is none."""
+    from hisvsim_amd import capi
+    from hisvsim_amd.circuit import Gate
+    n, m = 13, np.array([[2.0, 0.5], [0.25, 1.0]])
+    g = Gate("C1", (3,), (), tuple(m.ravel()))
+    inv = Gate("C1", (3,), (), tuple(np.linalg.inv(m).ravel()))
+    far = [Gate("H", (q,)) for q in (3, 4, 5, 6, 7)]
+    a = _stored(n, "complex128", 1)
+    with capi.State(n) as s:
+        s.write(a)
+        s.apply_fused([g] + [inv], "f64")
+        assert np.abs(s.read() - a).max() <= 1e-12
+        with pytest.raises(capi.HsvError) as e:
+            s.apply_fused([g] + far, "f64")
+        assert e.value.code == -6
+        with pytest.raises(capi.HsvError) as e:
+            s.apply_fused([Gate("H", (q,)) for q in range(8)], "f64")
+        assert e.value.code == -5
