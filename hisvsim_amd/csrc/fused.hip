@@ -15,7 +15,9 @@
 //
 //  * HSV_FUSED_F64: v_mfma_f64_16x16x4_f64, FP64 products and accumulation;
 //    most parts as 4-qubit steps on a tile (k_fused_tile, below).
-//  * HSV_FUSED_F32SPLIT: v_mfma_f32_16x16x4_f32 on hi/lo FP32 splits of U and
+//  * HSV_FUSED_F32SPLIT: the same FP64 steps where they are the faster way
+//    (15 parts of 6 qubits at 25 qubits 9.6 -> 4.3 ms with their read-outs), and
+//    the more exact one; other parts v_mfma_f32_16x16x4_f32 on hi/lo FP32 splits of U and
 //    X (x = hi + lo, hi = fp32(x), lo = fp32(x - hi)); each real product is
 //    hi*hi + hi*lo + lo*hi, accumulated in FP32; the result is stored back in
 //    the state's precision.
@@ -1411,12 +1413,14 @@ int part_apply_bf(void* amp, int n, int dtype, hipStream_t stream, DeviceScratch
 
 // The FP64 path on tiles (k_fused_tile). *taken = false, and nothing done, when
 // the dense kernel is to run: a gate on more than 4 qubits, more steps than
-// the dense product has flops for (2^(K - 4)), a state below a tile, or steps
+// the dense product is worth (2^(K - 4) in FP64, which it has the same flops
+// as; half as many again against the FP32-split product, whose three FP32
+// products a flop take 1.5 times FP64's time), a state below a tile, or steps
 // whose unitarity does not by itself bound the part's (a gate and its inverse
 // that are not unitary, say): U^H U - I of a product of S embedded steps is at
 // most 16 S times the steps' own in its largest entry.
 int fused_apply_tile64(void* amp, int n, int dtype, hipStream_t stream, DeviceScratch* scratch,
-                       const std::vector<Lowered>& gates, int tile_order, bool* taken, std::string* err) {
+                       const std::vector<Lowered>& gates, bool split, int tile_order, bool* taken, std::string* err) {
   *taken = false;
   std::vector<uint64_t> qm;
   std::vector<const Lowered*> gl;
@@ -1435,7 +1439,7 @@ int fused_apply_tile64(void* amp, int n, int dtype, hipStream_t stream, DeviceSc
   if (n < 12 || n > 34 || K > 7 || qm.empty()) return HSV_OK;
   const std::vector<std::vector<int>> groups = step_groups(qm, 4, 16);
   const int ns = (int)groups.size();
-  if (ns == 0 || ns > std::min(kTileStepsMax, 1 << (K - 4))) return HSV_OK;
+  if (ns == 0 || ns > std::min(kTileStepsMax, (split ? 3 : 2) << (K - 4) >> 1)) return HSV_OK;
   uint64_t tmask = pmask;
   for (int b = 0; b < n && __builtin_popcountll(tmask) < 12; ++b) tmask |= 1ull << b;
   int slot[12];
@@ -1665,7 +1669,7 @@ int fused_apply(void* amp, int n, int dtype, hipStream_t stream, int num_cu, Dev
     if (__builtin_popcountll(pmask) > 7)
       return part_apply_bf(amp, n, dtype, stream, scratch, gates, pmask, nullptr, nullptr, ~0ull, bf, err, 2);
   }
-  if (mode == HSV_FUSED_F64) {
+  if (mode == HSV_FUSED_F64 || mode == HSV_FUSED_F32SPLIT) {
     // identities count towards a part's 7 qubits
     uint64_t mask = 0;
     for (const Lowered& L : gates) {
@@ -1674,7 +1678,7 @@ int fused_apply(void* amp, int n, int dtype, hipStream_t stream, int num_cu, Dev
     }
     bool taken = false;
     if (__builtin_popcountll(mask) <= 7)
-      if (int rc = fused_apply_tile64(amp, n, dtype, stream, scratch, gates, bf.tile_order, &taken, err)) return rc;
+      if (int rc = fused_apply_tile64(amp, n, dtype, stream, scratch, gates, mode == HSV_FUSED_F32SPLIT, bf.tile_order, &taken, err)) return rc;
     if (taken) return HSV_OK;
   }
   std::vector<int> Q;

@@ -65,7 +65,8 @@ typedef struct hsv_gate {
 /* Fused-part precision modes. */
 enum hsv_fused_mode {
   HSV_FUSED_F64 = 0,        /* FP64 matrix cores (v_mfma_f64)            */
-  HSV_FUSED_F32SPLIT = 1,   /* FP32 matrix cores, hi/lo split products   */
+  HSV_FUSED_F32SPLIT = 1,   /* FP32 matrix cores, hi/lo split products;
+                               FP64 steps where those are faster         */
   HSV_FUSED_BF16SPLIT = 2,  /* BF16 matrix cores, hi/lo split products
                                accumulated in FP32; parts of 5..14 qubits */
   HSV_FUSED_BF16X3 = 3,     /* BF16 matrix cores, three-piece split (six
