@@ -1420,7 +1420,8 @@ int part_apply_bf(void* amp, int n, int dtype, hipStream_t stream, DeviceScratch
 // that are not unitary, say): U^H U - I of a product of S embedded steps is at
 // most 16 S times the steps' own in its largest entry.
 int fused_apply_tile64(void* amp, int n, int dtype, hipStream_t stream, DeviceScratch* scratch,
-                       const std::vector<Lowered>& gates, bool split, int tile_order, bool* taken, std::string* err) {
+                       const std::vector<Lowered>& gates, bool split, uint64_t live, int tile_order, bool* taken,
+                       std::string* err) {
   *taken = false;
   std::vector<uint64_t> qm;
   std::vector<const Lowered*> gl;
@@ -1508,8 +1509,8 @@ int fused_apply_tile64(void* amp, int n, int dtype, hipStream_t stream, DeviceSc
     return HSV_ERR_DEVICE;
   }
   const uint64_t all = (n == 64) ? ~0ull : ((1ull << n) - 1);
-  const uint64_t outer = all & ~tmask, top = top_slots(outer, tile_order);
-  const unsigned ntiles = 1u << (n - 12);
+  const uint64_t outer = all & ~tmask & live, top = top_slots(outer, tile_order);
+  const unsigned ntiles = 1u << __builtin_popcountll(outer);
   const auto* dev = static_cast<const unsigned char*>(scratch->ptr);
   const auto* da = reinterpret_cast<const TileAddr*>(dev);
   const auto* ds = reinterpret_cast<const TileStep*>(dev + step_off);
@@ -1531,8 +1532,8 @@ int fused_apply_tile64(void* amp, int n, int dtype, hipStream_t stream, DeviceSc
 // variant: 0 / 1 = column-block kernel (1: swizzled row order), 2 = tile form
 // (needs n >= 12; falls back to 1 below that).
 int fused_apply_bf(void* amp, int n, int dtype, hipStream_t stream, int num_cu, DeviceScratch* scratch,
-                   const std::vector<int>& Q, const std::vector<cd>& Um, int variant, int tpw, int tile_order,
-                   std::string* err) {
+                   const std::vector<int>& Q, const std::vector<cd>& Um, uint64_t live, int variant, int tpw,
+                   int tile_order, std::string* err) {
   const int K = (int)Q.size();
   const int D = 1 << K;
   if (K < 5 || K > 7) {
@@ -1576,8 +1577,8 @@ int fused_apply_bf(void* amp, int n, int dtype, hipStream_t stream, int num_cu, 
       *err = "fused upload failed";
       return HSV_ERR_DEVICE;
     }
-    const uint64_t ntiles = 1ull << (n - 12);
-    const uint64_t outer = all & ~qmask & ~cmask;
+    const uint64_t outer = all & ~qmask & ~cmask & live;
+    const uint64_t ntiles = 1ull << __builtin_popcountll(outer);
     const int grid = (int)((ntiles + tpw - 1) / tpw);
     const uint64_t top = top_slots(outer, tile_order);
     const bool c128 = dtype == HSV_C128;
@@ -1607,8 +1608,8 @@ int fused_apply_bf(void* amp, int n, int dtype, hipStream_t stream, int num_cu, 
     return HSV_ERR_DEVICE;
   }
   BfArgs f{};
-  f.outer_mask = all & ~qmask & ~tmask;
-  f.nblocks = 1ull << (n - K - 4);
+  f.outer_mask = all & ~qmask & ~tmask & live;
+  f.nblocks = 1ull << __builtin_popcountll(f.outer_mask);
   const uint64_t waves = kBfThreads / 64;
   const int grid = (int)std::min<uint64_t>((f.nblocks + waves - 1) / waves, uint64_t(num_cu) * 2);
   int rc = HSV_OK;
@@ -1642,7 +1643,7 @@ int fused_part_bf_layout(void* amp, int n, int dtype, hipStream_t stream, Device
 }
 
 int fused_apply(void* amp, int n, int dtype, hipStream_t stream, int num_cu, DeviceScratch* scratch,
-                const std::vector<Lowered>& gates, int mode, std::string* err, const BfTune& bf) {
+                const std::vector<Lowered>& gates, int mode, uint64_t live, std::string* err, const BfTune& bf) {
   if (mode != HSV_FUSED_F64 && mode != HSV_FUSED_F32SPLIT && mode != HSV_FUSED_BF16SPLIT &&
       mode != HSV_FUSED_BF16X3) {
     *err = "unknown fused mode";
@@ -1657,7 +1658,7 @@ int fused_apply(void* amp, int n, int dtype, hipStream_t stream, int num_cu, Dev
       for (int i = 0; i < L.nt; ++i) pmask |= 1ull << L.t[i];
       for (int i = 0; i < L.nc; ++i) pmask |= 1ull << L.c[i];
     }
-    return part_apply_bf(amp, n, dtype, stream, scratch, gates, pmask, nullptr, nullptr, ~0ull, bf, err, 3);
+    return part_apply_bf(amp, n, dtype, stream, scratch, gates, pmask, nullptr, nullptr, live, bf, err, 3);
   }
   if (mode == HSV_FUSED_BF16SPLIT) {
     uint64_t pmask = 0;
@@ -1667,7 +1668,7 @@ int fused_apply(void* amp, int n, int dtype, hipStream_t stream, int num_cu, Dev
       for (int i = 0; i < L.nc; ++i) pmask |= 1ull << L.c[i];
     }
     if (__builtin_popcountll(pmask) > 7)
-      return part_apply_bf(amp, n, dtype, stream, scratch, gates, pmask, nullptr, nullptr, ~0ull, bf, err, 2);
+      return part_apply_bf(amp, n, dtype, stream, scratch, gates, pmask, nullptr, nullptr, live, bf, err, 2);
   }
   if (mode == HSV_FUSED_F64 || mode == HSV_FUSED_F32SPLIT) {
     // identities count towards a part's 7 qubits
@@ -1678,7 +1679,7 @@ int fused_apply(void* amp, int n, int dtype, hipStream_t stream, int num_cu, Dev
     }
     bool taken = false;
     if (__builtin_popcountll(mask) <= 7)
-      if (int rc = fused_apply_tile64(amp, n, dtype, stream, scratch, gates, mode == HSV_FUSED_F32SPLIT, bf.tile_order, &taken, err)) return rc;
+      if (int rc = fused_apply_tile64(amp, n, dtype, stream, scratch, gates, mode == HSV_FUSED_F32SPLIT, live, bf.tile_order, &taken, err)) return rc;
     if (taken) return HSV_OK;
   }
   std::vector<int> Q;
@@ -1697,7 +1698,7 @@ int fused_apply(void* amp, int n, int dtype, hipStream_t stream, int num_cu, Dev
     return HSV_ERR_LIMIT;
   }
   if (mode == HSV_FUSED_BF16SPLIT)
-    return fused_apply_bf(amp, n, dtype, stream, num_cu, scratch, Q, Um, bf.variant, std::max(bf.tile_tpw, 1),
+    return fused_apply_bf(amp, n, dtype, stream, num_cu, scratch, Q, Um, live, bf.variant, std::max(bf.tile_tpw, 1),
                           bf.tile_order, err);
   int NC = 2048 / (16 * D);
   while (NC > 1 && 4 + __builtin_ctz(NC) > free_bits) NC >>= 1;
@@ -1710,8 +1711,8 @@ int fused_apply(void* amp, int n, int dtype, hipStream_t stream, int num_cu, Dev
     if (!(qmask >> b & 1)) { tmask |= 1ull << b; ++got; }
   const uint64_t all = (n == 64) ? ~0ull : ((1ull << n) - 1);
   FusedArgs f{};
-  f.outer_mask = all & ~qmask & ~tmask;
-  f.ntiles = 1ull << (n - K - logC);
+  f.outer_mask = all & ~qmask & ~tmask & live;
+  f.ntiles = 1ull << __builtin_popcountll(f.outer_mask);
   f.C = C;
   f.logC = logC;
   f.NC = NC;

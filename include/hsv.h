@@ -96,7 +96,11 @@ int hsv_apply_gate(hsv_state* s, const hsv_gate* g);
 /* Replaces gather_and_execute_on (py_wrapper.cpp:156 -> execute.hpp:171-316,
  * with the live gather/execute/scatter body of execute.hpp:318-470): all
  * gates of one part applied in one pass, the part's sub-state staged in LDS.
- * opt_slots adds qubits 0..3 to the part (execute.hpp:184-199). */
+ * opt_slots adds qubits 0..3 to the part (execute.hpp:184-199).
+ * A handle knows which qubits gates have acted on since it was |0...0>
+ * (hsv_create, hsv_reset; all of them after hsv_write): the others are |0>
+ * everywhere, and every gate path skips the part of the state that is
+ * therefore zero. */
 int hsv_apply_part(hsv_state* s, const hsv_gate* gates, int num_gates, int opt_slots);
 
 /* Not in the reference: the part's gates fused on the host into one
@@ -126,9 +130,8 @@ int hsv_apply_fused(hsv_state* s, const hsv_gate* gates, int num_gates, int mode
  * are exact. Argument errors are
  * found before any pass; a part that fails later (a gate on more than 5
  * qubits) leaves the parts before it applied, in the standard layout.
- * Right after hsv_create or hsv_reset (state |0...0>), a qubit that no
- * earlier part has touched is |0> everywhere, so the first passes skip the
- * tiles with a 1 in such a qubit. */
+ * A qubit that no gate has touched since the state was |0...0> is |0>
+ * everywhere, so the first passes skip the tiles with a 1 in such a qubit. */
 int hsv_apply_fused_chain(hsv_state* s, const hsv_gate* gates, int num_gates, const int* part_sizes,
                           int num_parts, const int* lows, int mode);
 

@@ -207,3 +207,70 @@ def test_fused_f64_unitarity_is_the_parts():
         with pytest.raises(capi.HsvError) as e:
             s.apply_fused([Gate("H", (q,)) for q in range(8)], "f64")
         assert e.value.code == -5
+
+
+def _some_gates(rng, qubits, count):
+    from hisvsim_amd.circuit import Gate
+    gs = []
+    for _ in range(count):
+        q = [int(x) for x in rng.permutation(qubits)]
+        th = [float(x) for x in rng.uniform(0, 6, 3)]
+        gs.append(Gate("U3", (q[0],), (), tuple(th)))
+        if len(q) > 1:
+            gs += [Gate("X", (q[1],), (q[0],)), Gate("RZZ", (q[0], q[1]), (), (th[1],)), Gate("SWAP", (q[1], q[0]))]
+    return gs
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("seed", range(12))
+def test_passes_skip_only_what_is_zero(seed):
+    """From |0...0>, whatever acts in between on whatever qubits (gates, parts
+    on each kernel, fused parts, chains, permutations, projections,
+    renormalisations, reads, writes of a range, resets): the state equals the
+    one of the same calls on a state that was written, where nothing is known
+    to be zero. 1e-12 (the FP64 paths; the chain runs the same passes on
+    both, so its rounding is the same or that of zeros)."""
+    from hisvsim_amd import capi
+    n, rng = 15, np.random.default_rng(seed)
+    zero = np.zeros(2 ** n, complex)
+    zero[0] = 1
+    with capi.State(n) as a, capi.State(n) as b:
+        for _ in range(14):
+            b.write(b.read())        # forgets what b knows
+            pick = [int(x) for x in rng.permutation(n)[:int(rng.integers(1, 6))]]
+            op = rng.choice(["gates", "part", "reg", "lds", "f64", "f32split", "chain", "permute", "project",
+                             "renormalize", "write", "reset", "measure"],
+                            p=[.2, .15, .08, .07, .1, .06, .08, .1, .03, .03, .03, .04, .03])
+            gs = _some_gates(rng, pick, int(rng.integers(1, 4)))
+            perm = [int(x) for x in rng.permutation(n)]
+            at = int(rng.integers(0, 2 ** n - 4))
+            u = rng.random(5)
+            for s in (a, b):
+                s.tune("part_kernel", {"reg": 1, "lds": 0}.get(op, 2))
+                if op == "gates":
+                    s.apply_gates(gs)
+                elif op in ("part", "reg", "lds"):
+                    s.apply_part(gs, 0)
+                elif op in ("f64", "f32split"):
+                    s.apply_fused(gs, "f64")
+                elif op == "chain":
+                    s.apply_fused_chain([gs], [list(range(5))], "bf16x3")
+                elif op == "permute":
+                    s.permute_qubits(perm)
+                elif op == "project":
+                    q = pick[0]
+                    s.project([q], [0 if s.probability(q, 0) > 0.4 else 1])
+                elif op == "renormalize":
+                    s.renormalize()
+                elif op == "write":
+                    s.write(np.full(3, 0.01 + 0.02j), at)
+                elif op == "reset":
+                    s.reset()
+                else:
+                    s.measure(list(range(n)), u)
+            tol = 1e-12 if op != "chain" else 1e-6
+            x, y = a.read(), b.read()
+            assert np.abs(x - y).max() <= tol, op
+            if op == "chain":        # past a chain both go on from the same amplitudes
+                a.reset()
+                b.reset()
