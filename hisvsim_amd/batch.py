@@ -41,7 +41,7 @@ class CircuitBatch:
             offs.append(offs[-1] + len(g))
         self._offs = offs
         go = (ctypes.c_int * len(offs))(*offs)
-        arr = capi.gate_array([g for _, gs in self.instances for g in gs])
+        arr = self._records = capi.gate_array([g for _, gs in self.instances for g in gs])
         self._h = ctypes.c_void_p()
         dt = {"complex128": capi.HSV_C128, "complex64": capi.HSV_C64}[dtype]
         capi._check(capi.lib().hsv_batch_create(len(self.instances), nq, go, arr, dt, ctypes.byref(self._h)))
@@ -66,7 +66,9 @@ class CircuitBatch:
     def set_gates(self, gate_lists: Sequence[Sequence[Gate]]) -> None:
         """New gates with the same types and qubits, instance by instance."""
         flat = [g for gs in gate_lists for g in gs]
-        capi._check(capi.lib().hsv_batch_set_gates(self._h, capi.gate_array(flat)))
+        if len(flat) < self._offs[-1]:
+            raise ValueError("fewer gates than the batch has")
+        capi._check(capi.lib().hsv_batch_set_gates(self._h, capi.gate_array(flat, self._records)))
         self.instances = [(n, list(g)) for (n, _), g in zip(self.instances, gate_lists)]
 
     def run(self) -> None:

@@ -69,10 +69,35 @@ def to_hsv_gate(g) -> hsv_gate:
     return d
 
 
-def gate_array(gates: Sequence) -> ctypes.Array:
-    arr = (hsv_gate * max(1, len(gates)))()
-    for i, g in enumerate(gates):
-        arr[i] = to_hsv_gate(g)
+_native = None
+
+
+def _module():
+    """The pybind module, whose native conversion of gate lists gate_array
+    and State.apply_gates use; False without it."""
+    global _native
+    if _native is None:
+        try:
+            from . import load_module
+            _native = load_module()
+        except ImportError:
+            _native = False
+    return _native
+
+
+def _fill(arr: ctypes.Array, gates: Sequence) -> bool:
+    """Whether the module filled `arr` (whatever it held) from `gates` (plain
+    Gate lists; see fill_gates in csrc/py_wrapper.cpp)."""
+    m = _module()
+    return bool(m) and m._fill_gates(gates, Gate, GATE_TYPES, ctypes.addressof(arr), len(arr))
+
+
+def gate_array(gates: Sequence, into: ctypes.Array | None = None) -> ctypes.Array:
+    """The gates' records; `into`: an array of at least their number to use."""
+    arr = (hsv_gate * max(1, len(gates)))() if into is None or len(into) < len(gates) else into
+    if not _fill(arr, gates):
+        for i, g in enumerate(gates):
+            arr[i] = to_hsv_gate(g)
     return arr
 
 
@@ -290,6 +315,11 @@ class State:
         _check(lib().hsv_apply_gate(self._h, ctypes.byref(d)))
 
     def apply_gates(self, gates: Iterable) -> None:
+        if isinstance(gates, (list, tuple)):
+            arr = (hsv_gate * max(1, len(gates)))()
+            if _fill(arr, gates):
+                _check(_module()._apply_gates(self._h.value or 0, ctypes.addressof(arr), len(gates)))
+                return
         for g in gates:
             self.apply_gate(g)
 

@@ -56,11 +56,11 @@ struct BSeg {
   uint64_t chunk_mask;  // instance qubits held in a chunk
   uint64_t outer_mask;  // the others (one chunk per assignment of them)
   int bits;             // popcount(chunk_mask)
-  int gate_first;       // first PartGate record
+  int gate_first;       // its gates, in rec_gate
   int gate_count;
   int tseg_first;       // chunks with a tile plan: its first register segment
   int tseg_count;       // -1: the gates sweep the chunk in LDS one by one
-  int pad;
+  int part_first;       // then its first PartGate record
 };
 
 // A chunk of KT qubits runs the FP64 tile kernel's register segments
@@ -178,7 +178,7 @@ __global__ __launch_bounds__(BS) void k_batch_stage(typename VecT<R>::type* __re
     for (uint32_t j = threadIdx.x; j < nin; j += BS) lds[j] = st[base + tlo[j & 63] + thi[j >> 6]];
     __syncthreads();
     for (int g = 0; g < S.gate_count; ++g) {
-      part_gate_lds<R, BS>(lds, gates[S.gate_first + g]);
+      part_gate_lds<R, BS>(lds, gates[S.part_first + g]);
       __syncthreads();
     }
     for (uint32_t j = threadIdx.x; j < nin; j += BS) st[base + tlo[j & 63] + thi[j >> 6]] = lds[j];
@@ -270,6 +270,10 @@ struct hsv_batch {
   std::vector<int> nq;
   std::vector<int> gate_off;          // num + 1
   std::vector<hsv_gate> gates;        // as given
+  // set_gates' working memory, kept between calls: the gates lowered, the next
+  // ones, the LDS sweeps' records
+  std::vector<Lowered> lowered, next;
+  std::vector<PartGate> recs;
   std::vector<uint64_t> starts;       // first amplitude per instance
   uint64_t total = 0;
   int L = 12;                         // chunk bits (tuned)
@@ -280,8 +284,8 @@ struct hsv_batch {
   void* state = nullptr;
   // plan (rebuilt when L changes): segments, their gate records, stage lists
   std::vector<BSeg> segs;
-  std::vector<int> rec_gate;          // source gate of each PartGate record
-  std::vector<std::vector<int>> rec_inner;  // qubit -> chunk bit of each record's segment
+  std::vector<int> rec_gate;          // the segments' gates, segment by segment
+  std::vector<std::vector<int>> seg_inner;  // per segment: qubit -> chunk bit
   std::vector<StageList> stages;
   BSeg* d_segs = nullptr;
   PartGate* d_gates = nullptr;
@@ -290,6 +294,14 @@ struct hsv_batch {
   void* d_tile = nullptr;
   size_t tile_bytes = 0;
   size_t tile_nseg = 0, tile_nround = 0, tile_ngate = 0, tile_nmat = 0;
+  // host copy of the tile plans' gate records and matrices and where each
+  // record comes from, so that new parameters only rewrite the numbers
+  std::vector<RegGate> tile_gates;
+  std::vector<int> tile_m2idx, tile_source;
+  std::vector<double> tile_mat2;
+  std::vector<char> tile_sign;        // per record: planned as a sign flip
+  struct TileRange { int seg, first, count; };
+  std::vector<TileRange> tile_ranges; // per segment with a plan: its records
   void* d_lists = nullptr;
   std::vector<size_t> list_off;
   uint64_t* d_starts = nullptr;
@@ -323,15 +335,21 @@ void drop_plan(hsv_batch* b) {
   b->d_lists = nullptr;
   b->d_tile = nullptr;
   b->tile_bytes = 0;
+  b->tile_gates.clear();
+  b->tile_m2idx.clear();
+  b->tile_source.clear();
+  b->tile_mat2.clear();
+  b->tile_sign.clear();
+  b->tile_ranges.clear();
   b->segs.clear();
   b->rec_gate.clear();
-  b->rec_inner.clear();
+  b->seg_inner.clear();
   b->stages.clear();
 }
 
-// Lowers every gate, cuts each instance into segments and builds the gate
-// records; fails on a bad gate before anything is uploaded.
-int plan(hsv_batch* b, std::vector<PartGate>* recs) {
+// Lowers every gate and cuts each instance into segments; fails on a bad gate
+// before anything is uploaded.
+int plan(hsv_batch* b) {
   std::vector<std::vector<int>> inst_segs(b->num);
   for (int i = 0; i < b->num; ++i) {
     const int n = b->nq[i];
@@ -382,14 +400,11 @@ int plan(hsv_batch* b, std::vector<PartGate>* recs) {
       S.chunk_mask = chunk;
       S.outer_mask = all & ~chunk;
       S.bits = L;
-      S.gate_first = (int)recs->size();
-      for (int g : taken) {
-        if (Ls[g].kind == K_IDENT) continue;
-        recs->push_back(part_gate_of(Ls[g], L, inner));
-        b->rec_gate.push_back(g0 + g);
-        b->rec_inner.emplace_back(inner, inner + 64);
-      }
-      S.gate_count = (int)recs->size() - S.gate_first;
+      S.gate_first = (int)b->rec_gate.size();
+      for (int g : taken)
+        if (Ls[g].kind != K_IDENT) b->rec_gate.push_back(g0 + g);
+      S.gate_count = (int)b->rec_gate.size() - S.gate_first;
+      b->seg_inner.emplace_back(inner, inner + 64);
       inst_segs[i].push_back((int)b->segs.size());
       b->segs.push_back(S);
       rem = keep;
@@ -420,9 +435,19 @@ struct TileArrays {
   std::vector<RegSeg> segs;
   std::vector<TileRound> rounds;
   std::vector<RegGate> gates;
-  std::vector<int> m2idx;
+  std::vector<int> m2idx, source;
   std::vector<double> mat2;
+  std::vector<char> sign;
+  std::vector<hsv_batch::TileRange> ranges;
 };
+
+// The gates of segment S, lowered.
+std::vector<Lowered> segment_gates(const hsv_batch* b, const BSeg& S, const std::vector<Lowered>& all) {
+  std::vector<Lowered> Ls;
+  Ls.reserve(S.gate_count);
+  for (int r = S.gate_first; r < S.gate_first + S.gate_count; ++r) Ls.push_back(all[b->rec_gate[r]]);
+  return Ls;
+}
 
 void build_tiles(hsv_batch* b, const std::vector<Lowered>& all, std::vector<BSeg>* segs, TileArrays* A) {
   int tb = 0;
@@ -434,10 +459,9 @@ void build_tiles(hsv_batch* b, const std::vector<Lowered>& all, std::vector<BSeg
     // the widths k_batch_stage instantiates (tile_chunk_ok)
     const bool ok = S.bits >= 8 && S.bits <= (b->dtype == HSV_C128 ? 12 : 13) && RB >= 2 && RB <= 5 && b->nt >= 128;
     if (!ok || S.gate_count == 0) continue;
-    std::vector<Lowered> Ls;
-    for (int r = S.gate_first; r < S.gate_first + S.gate_count; ++r) Ls.push_back(all[b->rec_gate[r]]);
+    const std::vector<Lowered> Ls = segment_gates(b, S, all);
     TilePlan TP;
-    if (build_tile_plan(Ls, b->rec_inner[S.gate_first].data(), S.bits, RB, &TP) != HSV_OK) continue;
+    if (build_tile_plan(Ls, b->seg_inner[&S - segs->data()].data(), S.bits, RB, &TP) != HSV_OK) continue;
     const int rb = (int)A->rounds.size(), gb = (int)A->gates.size(), mb = (int)(A->mat2.size() / 32);
     S.tseg_first = (int)A->segs.size();
     S.tseg_count = (int)TP.segs.size();
@@ -451,7 +475,11 @@ void build_tiles(hsv_batch* b, const std::vector<Lowered>& all, std::vector<BSeg
       Q.sfirst += gb;
       A->rounds.push_back(Q);
     }
+    A->ranges.push_back({(int)(&S - segs->data()), gb, (int)TP.gates.size()});
+    const std::vector<Lowered> fused = fuse_one_qubit_runs(Ls);
     for (size_t i = 0; i < TP.gates.size(); ++i) {
+      A->source.push_back(TP.source[i]);
+      A->sign.push_back(tile_sign_flip(fused[TP.source[i]]));
       A->gates.push_back(TP.gates[i]);
       A->m2idx.push_back(TP.m2idx[i] >= 0 ? TP.m2idx[i] + mb : -1);
     }
@@ -485,9 +513,61 @@ int upload_tiles(hsv_batch* b, const TileArrays& A) {
     hg[i].m2 = A.m2idx[i] >= 0 ? reinterpret_cast<const double*>(dev + mat_off) + 32 * size_t(A.m2idx[i]) : nullptr;
   }
   if (!A.mat2.empty()) std::memcpy(host.data() + mat_off, A.mat2.data(), A.mat2.size() * sizeof(double));
+  b->tile_gates.assign(hg, hg + A.gates.size());
+  b->tile_m2idx = A.m2idx;
+  b->tile_source = A.source;
+  b->tile_mat2 = A.mat2;
+  b->tile_sign = A.sign;
+  b->tile_ranges = A.ranges;
   BCHK(hipMemcpyAsync(b->d_tile, host.data(), bytes, hipMemcpyHostToDevice, b->stream));
   BCHK(hipStreamSynchronize(b->stream));
   return HSV_OK;
+}
+
+// New matrices in the tile plans' records, the gates' kinds as planned;
+// *same = false (and nothing uploaded) when a phase gate became or stopped
+// being a sign flip: such a plan is another one.
+int refresh_tiles(hsv_batch* b, const std::vector<Lowered>& all, bool* same) {
+  *same = true;
+  for (const auto& R : b->tile_ranges) {
+    const std::vector<Lowered> fused = fuse_one_qubit_runs(segment_gates(b, b->segs[R.seg], all));
+    for (int i = R.first; i < R.first + R.count; ++i) {
+      const Lowered& L = fused[b->tile_source[i]];
+      if (tile_sign_flip(L) != (b->tile_sign[i] != 0)) {
+        *same = false;
+        return HSV_OK;
+      }
+      double m[32];
+      for (int j = 0; j < 16; ++j) {
+        m[2 * j] = L.m[j].real();
+        m[2 * j + 1] = L.m[j].imag();
+      }
+      std::memcpy(b->tile_gates[i].m, m, sizeof(b->tile_gates[i].m));
+      if (b->tile_m2idx[i] >= 0) std::memcpy(b->tile_mat2.data() + 32 * size_t(b->tile_m2idx[i]), m, sizeof(m));
+    }
+  }
+  const size_t gate_off = b->tile_nseg * sizeof(RegSeg) + b->tile_nround * sizeof(TileRound);
+  const size_t mat_off = gate_off + b->tile_gates.size() * sizeof(RegGate);
+  auto* dev = static_cast<unsigned char*>(b->d_tile);
+  if (!b->tile_gates.empty())
+    BCHK(hipMemcpyAsync(dev + gate_off, b->tile_gates.data(), b->tile_gates.size() * sizeof(RegGate),
+                        hipMemcpyHostToDevice, b->stream));
+  if (!b->tile_mat2.empty())
+    BCHK(hipMemcpyAsync(dev + mat_off, b->tile_mat2.data(), b->tile_mat2.size() * sizeof(double),
+                        hipMemcpyHostToDevice, b->stream));
+  BCHK(hipStreamSynchronize(b->stream));
+  return HSV_OK;
+}
+
+// The LDS sweeps' records: the gates of the segments without a tile plan.
+void part_records(const hsv_batch* b, const std::vector<Lowered>& all, std::vector<PartGate>* recs) {
+  recs->clear();
+  for (size_t i = 0; i < b->segs.size(); ++i) {
+    const BSeg& S = b->segs[i];
+    if (S.tseg_count >= 0) continue;
+    for (int r = S.gate_first; r < S.gate_first + S.gate_count; ++r)
+      recs->push_back(part_gate_of(all[b->rec_gate[r]], S.bits, b->seg_inner[i].data()));
+  }
 }
 
 template <typename T>
@@ -533,11 +613,11 @@ void launch_stage_nt(hsv_batch* b, const StageList& st, const int* ids, const ui
 
 int build(hsv_batch* b) {
   drop_plan(b);
-  std::vector<PartGate> recs;
-  if (int rc = plan(b, &recs)) {
+  if (int rc = plan(b)) {
     drop_plan(b);
     return rc;
   }
+  std::vector<PartGate> recs;
   {
     std::vector<Lowered> all(b->gates.size());
     for (size_t g = 0; g < b->gates.size(); ++g) {
@@ -547,6 +627,12 @@ int build(hsv_batch* b) {
     TileArrays A;
     build_tiles(b, all, &b->segs, &A);
     if (int rc = upload_tiles(b, A)) return rc;
+    int first = 0;
+    for (BSeg& S : b->segs) {
+      S.part_first = first;
+      if (S.tseg_count < 0) first += S.gate_count;
+    }
+    part_records(b, all, &recs);
   }
   BCHK(hipMalloc(reinterpret_cast<void**>(&b->d_segs), std::max<size_t>(b->segs.size(), 1) * sizeof(BSeg)));
   BCHK(hipMalloc(reinterpret_cast<void**>(&b->d_gates), std::max<size_t>(recs.size(), 1) * sizeof(PartGate)));
@@ -657,8 +743,7 @@ int hsv_batch_create(int num_instances, const int* num_qubits, const int* gate_o
   BCHK(hipMemcpy(b->d_nq, b->nq.data(), sizeof(int) * num_instances, hipMemcpyHostToDevice));
   BCHK(hipEventCreate(&b->e0));
   BCHK(hipEventCreate(&b->e1));
-  std::vector<PartGate> recs;
-  if (int rc = plan(b, &recs)) {   // report bad gates at creation
+  if (int rc = plan(b)) {   // report bad gates at creation
     drop_plan(b);
     hsv_batch_destroy(b);
     return rc;
@@ -691,46 +776,36 @@ int hsv_batch_set_gates(hsv_batch* b, const hsv_gate* gates) {
   for (size_t g = 0; g < b->gates.size(); ++g)
     if (!same_structure(b->gates[g], gates[g]))
       return bfail(HSV_ERR_ARG, "gate " + std::to_string(g) + " differs in type or qubits from the batch's");
-  std::vector<Lowered> Ls(b->gates.size());
-  for (size_t g = 0; g < b->gates.size(); ++g) {
-    std::string err;
-    if (int rc = lower(gates[g], &Ls[g], &err)) return bfail(rc, "gate " + std::to_string(g) + ": " + err);
-  }
-  std::vector<Lowered> old(b->gates.size());
+  const size_t count = b->gates.size();
   bool same_kinds = true;
-  for (size_t g = 0; g < b->gates.size(); ++g) {
+  {
     std::string err;
-    same_kinds = same_kinds && lower(b->gates[g], &old[g], &err) == HSV_OK && old[g].kind == Ls[g].kind;
+    b->next.resize(count);
+    for (size_t g = 0; g < count; ++g)
+      if (int rc = lower(gates[g], &b->next[g], &err)) return bfail(rc, "gate " + std::to_string(g) + ": " + err);
+    if (b->lowered.size() != count) {
+      b->lowered.resize(count);
+      for (size_t g = 0; g < count; ++g) (void)lower(b->gates[g], &b->lowered[g], &err);
+    }
+    for (size_t g = 0; g < count; ++g) same_kinds = same_kinds && b->lowered[g].kind == b->next[g].kind;
+    b->lowered.swap(b->next);
   }
-  std::copy(gates, gates + b->gates.size(), b->gates.begin());
+  std::copy(gates, gates + count, b->gates.begin());
   if (!same_kinds) drop_plan(b);  // a caller-supplied matrix changed class: plan again
   if (!b->exec) return HSV_OK;    // the next run plans with the new gates
   // same geometry, new matrices: rewrite the records in place, keep the graph
-  std::vector<PartGate> recs(b->rec_gate.size());
-  for (size_t r = 0; r < recs.size(); ++r) {
-    const int g = b->rec_gate[r];
-    int inst = 0;
-    while (b->gate_off[inst + 1] <= g) ++inst;
-    recs[r] = part_gate_of(Ls[g], std::min(b->nq[inst], b->L), b->rec_inner[r].data());
-  }
-  // the tile plans: the same layout of segments and rounds keeps the graph
-  // (new matrices in place); a different one (a phase gate that became or
-  // stopped being a sign flip) plans again at the next run
-  std::vector<BSeg> segs = b->segs;
-  TileArrays A;
-  build_tiles(b, Ls, &segs, &A);
-  bool same_tiles = A.segs.size() == b->tile_nseg && A.rounds.size() == b->tile_nround &&
-                    A.gates.size() == b->tile_ngate && A.mat2.size() == b->tile_nmat;
-  for (size_t i = 0; same_tiles && i < segs.size(); ++i)
-    same_tiles = segs[i].tseg_first == b->segs[i].tseg_first && segs[i].tseg_count == b->segs[i].tseg_count;
+  // (in the tile plans, or plan again at the next run)
+  bool same_tiles = true;
+  if (int rc = refresh_tiles(b, b->lowered, &same_tiles)) return rc;
   if (!same_tiles) {
     drop_plan(b);
     return HSV_OK;
   }
-  if (int rc = upload_tiles(b, A)) return rc;
-  if (!recs.empty())
-    BCHK(hipMemcpyAsync(b->d_gates, recs.data(), recs.size() * sizeof(PartGate), hipMemcpyHostToDevice, b->stream));
-  BCHK(hipStreamSynchronize(b->stream));
+  part_records(b, b->lowered, &b->recs);
+  if (!b->recs.empty()) {
+    BCHK(hipMemcpyAsync(b->d_gates, b->recs.data(), b->recs.size() * sizeof(PartGate), hipMemcpyHostToDevice, b->stream));
+    BCHK(hipStreamSynchronize(b->stream));
+  }
   return HSV_OK;
 }
 

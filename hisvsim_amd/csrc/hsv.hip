@@ -532,6 +532,8 @@ std::vector<Lowered> hsv::fuse_one_qubit_runs(const std::vector<Lowered>& Ls) {
   return out;
 }
 
+bool hsv::tile_sign_flip(const Lowered& L) { return L.kind == K_PHASE1 && L.m[0] == cd{-1.0, 0.0}; }
+
 // The FP64 tile kernel's plan of one part (shared with the circuit batch):
 // the part's one-qubit runs fused (fuse_one_qubit_runs), then the register
 // kernel's layout segments over the tile's KT bits with RB register bits;
@@ -594,6 +596,7 @@ int hsv::build_tile_plan(const std::vector<Lowered>& Ls_in, const int* inner_of,
   T->segs = std::move(P.segs);
   T->gates = std::move(P.gates);
   T->m2idx = std::move(P.m2idx);
+  T->source = std::move(P.order);
   T->mat2 = std::move(P.mat2);
   return HSV_OK;
 }

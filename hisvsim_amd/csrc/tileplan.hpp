@@ -14,6 +14,7 @@ struct TilePlan {
   std::vector<TileRound> rounds;
   std::vector<RegGate> gates;      // m2 left unset: the uploader points it at mat2
   std::vector<int> m2idx;          // per gate: its matrix in mat2, or -1
+  std::vector<int> source;         // per gate: its place among the fused gates (fuse_one_qubit_runs)
   std::vector<double> mat2;        // 32 doubles per dense two-qubit gate
 };
 
@@ -23,6 +24,9 @@ struct TilePlan {
 // one-qubit gates on one qubit are first multiplied into one gate.
 // HSV_ERR_LIMIT when a segment's layout does not hold RB register bits.
 int build_tile_plan(const std::vector<Lowered>& Ls, const int* inner_of, int KT, int RB, TilePlan* T);
+
+// Whether a gate counts as a sign flip (Z, CZ, ...) in a plan's fast segments.
+bool tile_sign_flip(const Lowered& L);
 
 // The fusion build_tile_plan applies: each run of uncontrolled one-qubit
 // gates on one qubit (no other gate on that qubit in between) becomes one

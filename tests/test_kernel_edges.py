@@ -274,3 +274,68 @@ def test_passes_skip_only_what_is_zero(seed):
             if op == "chain":        # past a chain both go on from the same amplitudes
                 a.reset()
                 b.reset()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+@pytest.mark.parametrize("threads", [64, 256, 512])
+def test_new_parameters_equal_a_new_batch(threads, dtype):
+    """set_gates with plain new angles, with a phase that becomes and stops
+    being a sign flip and with matrices that change their kind, on instances
+    with tile plans and with LDS sweeps: bit for bit the states of a batch
+    made with those gates."""
+    from hisvsim_amd.batch import CircuitBatch, ansatz
+    from hisvsim_amd.circuit import Gate
+    sizes = [3, 6, 8, 10, 11, 12, 14]
+
+    def gates(seed, phase, swap):
+        rng = np.random.default_rng(seed)
+        out = []
+        for n in sizes:
+            m = np.array([[0, 1], [1, 0]]) if swap else np.diag([1, np.exp(0.3j)])
+            mid = [Gate("MATRIX", (1,), (), (1, 0, 0, complex(np.cos(phase), np.sin(phase)) if phase else -1.0)),
+                   Gate("MATRIX", (n - 1,), (0,), tuple(complex(x) for x in m.ravel())),
+                   Gate("RZZ", (0, n - 1), (), (float(rng.uniform(0, 6)),)), Gate("C1", (2,), (), (1, 0, 0, 1j))]
+            out.append(ansatz(n, 2, rng.uniform(0, 6, 4 * n)) + mid + ansatz(n, 2, rng.uniform(0, 6, 4 * n)))
+        return out
+
+    first = gates(1, 0.7, False)
+    with CircuitBatch(list(zip(sizes, first)), dtype) as b:
+        b.tune("threads", threads)
+        b.run()
+        for seed, phase, swap in ((2, 0.9, False), (3, 0, False), (4, 0, True), (5, 1.1, True), (6, 0.2, False)):
+            new = gates(seed, phase, swap)
+            b.set_gates(new)
+            b.run()
+            with CircuitBatch(list(zip(sizes, new)), dtype) as c:
+                c.tune("threads", threads)
+                c.run()
+                for i in range(len(sizes)):
+                    assert np.array_equal(b.state(i), c.state(i)), (seed, sizes[i])
+
+
+@pytest.mark.parametrize("gates", [
+    [("X", (1,), (), ())], [("U3", (3,), (), (1.5, 2, np.float64(0.3)))], [("C1", (0,), (1, 2), (1j, 2, 3.5, 1 + 2j))],
+    [("RXFRAC", (2,), (), (3, 4))], [("MATRIX", (0, 1), (), tuple(range(16)))], [("H", [4], [True], [])],
+    [("x", (1,), (2,), ())], [("RZ", (np.int64(1),), (), (0.5,))], [("RX", (1,), (), (np.complex64(1),))], []])
+def test_native_gate_records_equal_the_python_ones(gates):
+    """capi.gate_array (native where the list is plain, Python where not),
+    also into a used array, against to_hsv_gate."""
+    from hisvsim_amd import capi
+    from hisvsim_amd.circuit import Gate
+    gs = [Gate(*g) for g in gates]
+    used = capi.gate_array([Gate("C1", (9,), (7, 8), (1j, 2j, 3j, 4j))] * 3)
+    for arr in (capi.gate_array(gs), capi.gate_array(tuple(gs), used)):
+        for g, d in zip(gs, arr):
+            assert bytes(d) == bytes(capi.to_hsv_gate(g))
+
+
+@pytest.mark.parametrize("gate", [("NOTAGATE", (0,), (), ()), ("X", tuple(range(6)), (), ()), ("X", ("a",), (), ()),
+                                  ("RXFRAC", (0,), (), (1j, 2)), ("U3", (0,), (), tuple(range(17)))])
+def test_native_gate_records_refuse_what_python_refuses(gate):
+    from hisvsim_amd import capi
+    from hisvsim_amd.circuit import Gate
+    with pytest.raises(Exception) as want:
+        capi.to_hsv_gate(Gate(*gate))
+    with pytest.raises(type(want.value)):
+        capi.gate_array([Gate("X", (0,)), Gate(*gate)])
