@@ -113,6 +113,7 @@ SIGNATURES = {
     "hsv_num_qubits": (ctypes.c_int, [_P]),
     "hsv_dtype": (ctypes.c_int, [_P]),
     "hsv_apply_gate": (ctypes.c_int, [_P, _G]),
+    "hsv_apply_gates": (ctypes.c_int, [_P, _G, ctypes.c_int]),
     "hsv_apply_part": (ctypes.c_int, [_P, _G, ctypes.c_int, ctypes.c_int]),
     "hsv_apply_fused": (ctypes.c_int, [_P, _G, ctypes.c_int, ctypes.c_int]),
     "hsv_apply_fused_chain": (ctypes.c_int, [_P, _G, ctypes.c_int, _I, ctypes.c_int, _I, ctypes.c_int]),
@@ -318,7 +319,7 @@ class State:
         if isinstance(gates, (list, tuple)):
             arr = (hsv_gate * max(1, len(gates)))()
             if _fill(arr, gates):
-                _check(_module()._apply_gates(self._h.value or 0, ctypes.addressof(arr), len(gates)))
+                _check(lib().hsv_apply_gates(self._h, arr, len(gates)))
                 return
         for g in gates:
             self.apply_gate(g)

@@ -56,7 +56,7 @@ struct hsv_state {
   void* gate_buf = nullptr;        // device copy of the current part's gates
   size_t gate_buf_bytes = 0;
   double* partial = nullptr;       // device reduction partials (the chain's folded renormalisation; made at its first use)
-  double* host_partial = nullptr;  // the read-outs' partials, pinned host memory that the kernels write
+  double* host_partial = nullptr;  // the read-outs' partials, pinned host memory that the kernels write (made at the first)
   // Event pairs around each timed launch (a pool reused across collections).
   std::vector<std::pair<hipEvent_t, hipEvent_t>> events;
   size_t events_used = 0;
@@ -239,18 +239,17 @@ int ensure_gate_buf(hsv_state* s, size_t bytes) {
   return HSV_OK;
 }
 
-template <typename R>
-int launch_part_t(hsv_state* s, const std::vector<Lowered>& Ls, uint64_t part_mask, uint64_t live) {
-  const int k = __builtin_popcountll(part_mask);
-  int inner_of[64];
-  for (int b = 0, r = 0; b < 64; ++b) inner_of[b] = (part_mask >> b & 1) ? r++ : -1;
+// The LDS sweeps' records of the gates that do something, over a sub-state of
+// k bits, qubit q at bit map(q).
+template <typename Map>
+std::vector<PartGate> part_gates(const std::vector<Lowered>& Ls, int k, Map map) {
   std::vector<PartGate> pg;
   pg.reserve(Ls.size());
   for (const Lowered& L : Ls) {
     if (L.kind == K_IDENT) continue;
     PartGate G{};
     uint64_t set, o1, o2, nw;
-    sweep_geometry(L, k, [&](int q) { return inner_of[q]; }, &G.nfixed, G.fixed, &set, &o1, &o2, &nw);
+    sweep_geometry(L, k, map, &G.nfixed, G.fixed, &set, &o1, &o2, &nw);
     G.kind = L.kind;
     G.setmask = (uint32_t)set;
     G.off1 = (uint32_t)o1;
@@ -259,6 +258,36 @@ int launch_part_t(hsv_state* s, const std::vector<Lowered>& Ls, uint64_t part_ma
     pack_matrix(L, G.m);
     pg.push_back(G);
   }
+  return pg;
+}
+
+// hsv_apply_gates on a state that fits one workgroup's LDS.
+template <typename R>
+int launch_gate_list_t(hsv_state* s, const std::vector<Lowered>& Ls) {
+  for (const Lowered& L : Ls) touch(s, L);
+  const uint64_t live = s->support & (s->len - 1);
+  if (!live) return HSV_OK;  // identities only
+  const int nbits = 64 - __builtin_clzll(live);
+  const std::vector<PartGate> pg = part_gates(Ls, nbits, [](int q) { return q; });
+  const size_t bytes = pg.size() * sizeof(PartGate);
+  if (int rc = ensure_gate_buf(s, bytes)) return rc;
+  if (bytes) HIPCHK(hipMemcpyAsync(s->gate_buf, pg.data(), bytes, hipMemcpyHostToDevice, s->stream));
+  const size_t lds = (size_t(1) << nbits) * sizeof(typename VecT<R>::type);
+  auto kern = &k_gate_list<R>;
+  if (lds + sizeof(PartGate) * kListChunk > 65536)
+    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  hipLaunchKernelGGL(kern, 1, kListThreads, lds, s->stream, amp_as<R>(s), 1u << nbits,
+                     static_cast<const PartGate*>(s->gate_buf), (int)pg.size());
+  HIPCHK(hipGetLastError());
+  return HSV_OK;
+}
+
+template <typename R>
+int launch_part_t(hsv_state* s, const std::vector<Lowered>& Ls, uint64_t part_mask, uint64_t live) {
+  const int k = __builtin_popcountll(part_mask);
+  int inner_of[64];
+  for (int b = 0, r = 0; b < 64; ++b) inner_of[b] = (part_mask >> b & 1) ? r++ : -1;
+  const std::vector<PartGate> pg = part_gates(Ls, k, [&](int q) { return inner_of[q]; });
   const size_t bytes = pg.size() * sizeof(PartGate);
   if (int rc = ensure_gate_buf(s, bytes)) return rc;
   if (bytes) HIPCHK(hipMemcpyAsync(s->gate_buf, pg.data(), bytes, hipMemcpyHostToDevice, s->stream));
@@ -674,8 +703,18 @@ int launch_tile_part(hsv_state* s, const std::vector<Lowered>& Ls, uint64_t part
                                  : launch_tile_part_t<R, KT - 1, 256>(s, Ls, part_mask, live);
 }
 
+int ensure_host_partial(hsv_state* s) {
+  if (s->host_partial) return HSV_OK;
+  if (hipHostMalloc(reinterpret_cast<void**>(&s->host_partial), sizeof(double) * 2 * kSumBlocks, 0) != hipSuccess) {
+    s->host_partial = nullptr;
+    return fail(HSV_ERR_ALLOC, "cannot allocate reduction scratch");
+  }
+  return HSV_OK;
+}
+
 template <typename R, int MODE>
 int reduce_t(hsv_state* a, hsv_state* b, double* out0, double* out1) {
+  if (int rc = ensure_host_partial(a)) return rc;
   auto* pa = amp_as<R>(a);
   auto* pb = b ? amp_as<R>(b) : nullptr;
   int blocks = kRedBlocks;
@@ -704,11 +743,11 @@ int reduce(hsv_state* a, hsv_state* b, double* o0, double* o1) {
 int sum_grid(uint64_t count) {
   return (int)std::max<uint64_t>(1, std::min<uint64_t>(kSumBlocks, count / (4 * kRedBlock)));
 }
-int sum_partials(hsv_state* s, int grid, double* out) {
+int sum_partials(hsv_state* s, int grid, const double* partial, double* out) {
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(s->stream));
   double t = 0;
-  for (int i = 0; i < grid; ++i) t += s->host_partial[2 * i];
+  for (int i = 0; i < grid; ++i) t += partial[2 * i];
   *out = t;
   return HSV_OK;
 }
@@ -718,9 +757,18 @@ template <typename R>
 int mass0_t(hsv_state* s, int qubit, double* out) {
   // units of the half that is read (qubit 0 of complex64 is inside a unit)
   const uint64_t count = (s->len >> Unit<R>::LOG) >> (qubit >= Unit<R>::LOG);
-  const int grid = sum_grid(count);
+  int grid = sum_grid(count);
+  if (!s->host_partial && s->fused_scratch.fixed) {
+    // within the no-allocation chain: its device partials, copied
+    grid = std::min(grid, kRedBlocks);
+    double host[2 * kRedBlocks];
+    hipLaunchKernelGGL((k_mass0<R>), grid, kRedBlock, 0, s->stream, amp_as<R>(s), count, qubit, s->partial);
+    HIPCHK(hipMemcpyAsync(host, s->partial, sizeof(double) * 2 * grid, hipMemcpyDeviceToHost, s->stream));
+    return sum_partials(s, grid, host, out);
+  }
+  if (int rc = ensure_host_partial(s)) return rc;
   hipLaunchKernelGGL((k_mass0<R>), grid, kRedBlock, 0, s->stream, amp_as<R>(s), count, qubit, s->host_partial);
-  return sum_partials(s, grid, out);
+  return sum_partials(s, grid, s->host_partial, out);
 }
 int mass0(hsv_state* s, int qubit, double* out) {
   return s->dtype == HSV_C128 ? mass0_t<double>(s, qubit, out) : mass0_t<float>(s, qubit, out);
@@ -732,12 +780,13 @@ int pauli_t(hsv_state* s, uint64_t x, uint64_t z, double* out) {
   const uint64_t units = s->len >> Unit<R>::LOG;
   const uint64_t count = (x >> Unit<R>::LOG) ? units / 2 : units;
   const int grid = sum_grid(count);
+  if (int rc = ensure_host_partial(s)) return rc;
   if (x)
     hipLaunchKernelGGL((k_pauli_x<R>), grid, kRedBlock, 0, s->stream, amp_as<R>(s), count, x, z,
                        __builtin_popcountll(x & z) & 1, s->host_partial);
   else
     hipLaunchKernelGGL((k_pauli_z<R>), grid, kRedBlock, 0, s->stream, amp_as<R>(s), count, z, s->host_partial);
-  return sum_partials(s, grid, out);
+  return sum_partials(s, grid, s->host_partial, out);
 }
 
 // The measurement walk: the reference's sequential walk over cumulative
@@ -1233,12 +1282,6 @@ int hsv_create(int num_qubits, int dtype, hsv_state** out) {
     return fail(HSV_ERR_ALLOC, "cannot allocate " + std::to_string(s->len * (dtype == HSV_C128 ? 16 : 8)) +
                                    " bytes of device memory for the state");
   }
-  if (hipHostMalloc(reinterpret_cast<void**>(&s->host_partial), sizeof(double) * 2 * kSumBlocks, 0) != hipSuccess) {
-    hipFree(s->amp);
-    hipStreamDestroy(s->stream);
-    delete s;
-    return fail(HSV_ERR_ALLOC, "cannot allocate reduction scratch");
-  }
   *out = s;
   return hsv_reset(s);
 }
@@ -1248,7 +1291,7 @@ int hsv_destroy(hsv_state* s) {
   hipStreamSynchronize(s->stream);
   hipFree(s->amp);
   if (s->partial) (void)hipFree(s->partial);
-  (void)hipHostFree(s->host_partial);
+  if (s->host_partial) (void)hipHostFree(s->host_partial);
   if (s->walk_sub) (void)hipFree(s->walk_sub);
   if (s->walk_host) (void)hipHostFree(s->walk_host);
   if (s->gate_buf) hipFree(s->gate_buf);
@@ -1286,6 +1329,34 @@ int hsv_apply_gate(hsv_state* s, const hsv_gate* g) {
   if (int rc = launch_gate(s, L)) return rc;
   g_gate_count++;
   return end_timed(s);
+}
+
+// Lists of kListMin gates or more on a state that one workgroup's LDS holds
+// run as one launch; a launch of its own costs a gate about 4 us there, the
+// list's upload as much as three of them. Not while launches are timed: each
+// gate then has its pair of events.
+int hsv_apply_gates(hsv_state* s, const hsv_gate* gates, int num_gates) {
+  if (!s || num_gates < 0 || (num_gates > 0 && !gates)) return fail(HSV_ERR_ARG, "bad arguments");
+  constexpr int kListMin = 6;
+  if (num_gates < kListMin || s->timing || s->len * s->elem() > 65536) {
+    for (int i = 0; i < num_gates; ++i)
+      if (int rc = hsv_apply_gate(s, gates + i)) return rc;
+    return HSV_OK;
+  }
+  // up to the first gate that hsv_apply_gate would refuse
+  std::vector<Lowered> Ls;
+  Ls.reserve(num_gates);
+  int bad = HSV_OK;
+  std::string why;
+  for (int i = 0; i < num_gates && !bad; ++i) {
+    Lowered L;
+    bad = lower(gates[i], &L, &why);
+    if (!bad && L.kind != K_IDENT && (bad = check_gate_qubits(s, L))) why = g_err;
+    if (!bad) Ls.push_back(L);
+  }
+  if (int rc = s->dtype == HSV_C128 ? launch_gate_list_t<double>(s, Ls) : launch_gate_list_t<float>(s, Ls)) return rc;
+  g_gate_count += (long long)Ls.size();
+  return bad ? fail(bad, why) : HSV_OK;
 }
 
 int hsv_apply_part(hsv_state* s, const hsv_gate* gates, int num_gates, int opt_slots) {
@@ -1622,6 +1693,7 @@ int hsv_project(hsv_state* s, uint64_t qubit_mask, uint64_t values, double* p_ou
   if (!s) return fail(HSV_ERR_ARG, "null handle");
   if (qubit_mask >> s->n) return fail(HSV_ERR_ARG, "qubit mask names a qubit beyond the state");
   if (values & ~qubit_mask) return fail(HSV_ERR_ARG, "values has bits outside qubit_mask");
+  if (int rc = ensure_host_partial(s)) return rc;
   const int blocks = kRedBlocks;
   if (s->dtype == HSV_C128)
     hipLaunchKernelGGL((k_mass<double>), blocks, kRedBlock, 0, s->stream, amp_as<double>(s), s->len, qubit_mask,

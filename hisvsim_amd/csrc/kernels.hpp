@@ -20,9 +20,13 @@ template <> struct VecT<float> { using type = float2; };
 template <typename V, typename R>
 __device__ __forceinline__ V cmk(R x, R y) { V v; v.x = x; v.y = y; return v; }
 
+// a*b with its FMAs written out (which of a sum's two products is rounded
+// first is the compiler's choice otherwise, and differs from kernel to
+// kernel): every kernel that applies a gate's matrix so gives the same bits.
 template <typename V, typename R>
 __device__ __forceinline__ V cmul(V a, R bx, R by) {
-  return cmk<V, R>(a.x * bx - a.y * by, a.x * by + a.y * bx);
+  if constexpr (sizeof(R) == 8) return cmk<V, R>(fma(a.x, bx, -(a.y * by)), fma(a.y, bx, a.x * by));
+  return cmk<V, R>(fma(a.x, bx, -(a.y * by)), fma(a.x, by, a.y * bx));
 }
 // acc + a*b as two FMA chains (4 FMAs; `acc += a*b - c*d` written naively
 // compiles to mul + fma + add per component).
@@ -287,6 +291,36 @@ __global__ __launch_bounds__(BS) void k_part(typename VecT<R>::type* __restrict_
     }
     for (uint32_t j = threadIdx.x; j < nin; j += BS) a[base + tlo[j & 63] + thi[j >> 6]] = lds[j];
   }
+}
+
+// A list of gates on a state that one workgroup's LDS holds (hsv_apply_gates):
+// the gate sweeps' arithmetic, a barrier between gates, one launch for all of
+// them. Bound by latency (the barrier and the LDS round trip of each gate);
+// the records come through LDS too, kListChunk at a time, so no gate waits for
+// global memory. 60 gates on 10 qubits take 38
+// us, as 60 launches 120 us of kernels alone and 250 with the gaps between them.
+constexpr int kListChunk = 64;
+constexpr int kListThreads = 512;
+template <typename R>
+__global__ __launch_bounds__(kListThreads) void k_gate_list(typename VecT<R>::type* __restrict__ a, uint32_t len,
+                                                            const PartGate* __restrict__ gates, int ngates) {
+  using V = typename VecT<R>::type;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  V* lds = reinterpret_cast<V*>(smem_raw);
+  __shared__ PartGate rec[kListChunk];
+  for (uint32_t j = threadIdx.x; j < len; j += kListThreads) lds[j] = a[j];
+  for (int g0 = 0; g0 < ngates; g0 += kListChunk) {
+    const int cnt = min(kListChunk, ngates - g0);
+    const uint32_t* src = reinterpret_cast<const uint32_t*>(gates + g0);
+    uint32_t* dst = reinterpret_cast<uint32_t*>(rec);
+    for (int i = threadIdx.x; i < cnt * (int)(sizeof(PartGate) / 4); i += kListThreads) dst[i] = src[i];
+    __syncthreads();  // the records (and, at first, the state) are in LDS
+    for (int g = 0; g < cnt; ++g) {
+      part_gate_lds<R, kListThreads>(lds, rec[g]);
+      __syncthreads();
+    }
+  }
+  for (uint32_t j = threadIdx.x; j < len; j += kListThreads) a[j] = lds[j];
 }
 
 // ---- reductions (FP64 accumulation, fixed grid -> deterministic) -----------

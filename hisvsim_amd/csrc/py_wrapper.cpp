@@ -371,22 +371,12 @@ bool fill_gates(py::handle gates, py::handle gate_type, py::handle types, uintpt
   return true;
 }
 
-// hsv_apply_gate for each record, up to the first that fails.
-int apply_gates(uintptr_t state, uintptr_t gates, size_t count) {
-  py::gil_scoped_release release;
-  const hsv_gate* g = reinterpret_cast<const hsv_gate*>(gates);
-  for (size_t i = 0; i < count; ++i)
-    if (int rc = hsv_apply_gate(reinterpret_cast<hsv_state*>(state), g + i)) return rc;
-  return HSV_OK;
-}
-
 }  // namespace
 
 PYBIND11_MODULE(svsimulator_py_wrapper, m) {
   m.doc() = "MI355X hierarchical state-vector simulator (HiSVSIM svsimulator_py_wrapper API over libhsv)";
 
   m.def("_fill_gates", &fill_gates);
-  m.def("_apply_gates", &apply_gates);
 
   py::class_<AggregateGate_0>(m, "AggregateGate_0").def(py::init<const std::string&>());
   py::class_<AggregateGate_1>(m, "AggregateGate_1").def(py::init<const std::string&, cd>());

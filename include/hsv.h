@@ -92,6 +92,11 @@ int hsv_dtype(const hsv_state* s);
 /* Replaces BoundGate::apply -> apply_gate -> StateVector::apply
  * (state_vector.hpp:1349, 1202-1320, 402-510): one pass over the state. */
 int hsv_apply_gate(hsv_state* s, const hsv_gate* g);
+/* hsv_apply_gate for each gate in order, up to the first that fails (the
+ * reference's per-gate loop, qasm_assembler_standalone.py:1377-1617). One
+ * launch for the list where the state fits a workgroup's LDS (12 qubits, 13 in
+ * complex64); the same results. */
+int hsv_apply_gates(hsv_state* s, const hsv_gate* gates, int num_gates);
 
 /* Replaces gather_and_execute_on (py_wrapper.cpp:156 -> execute.hpp:171-316,
  * with the live gather/execute/scatter body of execute.hpp:318-470): all

@@ -339,3 +339,46 @@ def test_native_gate_records_refuse_what_python_refuses(gate):
         capi.to_hsv_gate(Gate(*gate))
     with pytest.raises(type(want.value)):
         capi.gate_array([Gate("X", (0,)), Gate(*gate)])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+@pytest.mark.parametrize("n", [1, 2, 5, 9, 12, 13, 14])
+def test_gate_lists_equal_the_gates_one_by_one(n, dtype):
+    """Lists below and above the length that takes one launch, longer than
+    the kernel's chunk of records, on states below, at and beyond a
+    workgroup's LDS, from |0...0> (qubits untouched so far above the touched
+    ones) and from a written state: the same bits as gate by gate."""
+    from hisvsim_amd import capi
+    rng = np.random.default_rng(n)
+    a = _stored(n, dtype, n)
+    low = list(range(max(1, n - 2)))
+    with capi.State(n, dtype) as s, capi.State(n, dtype) as r:
+        for qubits, count, start in ((low, 1, None), (low, 30, None), (list(range(n)), 2, a), (list(range(n)), 40, a)):
+            gs = _some_gates(rng, qubits, count)
+            for x in (s, r):
+                x.reset()
+                if start is not None:
+                    x.write(start)
+            s.apply_gates(gs)
+            for g in gs:
+                r.apply_gate(g)
+            assert np.array_equal(s.read(), r.read())
+
+
+@pytest.mark.gpu
+def test_gate_list_stops_at_the_gate_that_fails():
+    from hisvsim_amd import capi
+    from hisvsim_amd.circuit import Gate
+    gs = [Gate("H", (q,)) for q in range(5)] + [Gate("I", (2,)), Gate("X", (1,), (1,)), Gate("H", (0,))]
+    with capi.State(6) as s, capi.State(6) as r:
+        for bad in (gs, gs[:6] + [Gate("X", (6,))] + gs[:3]):
+            s.reset()
+            r.reset()
+            r.apply_gates(gs[:5])
+            before = capi.counters()["gates"]
+            with pytest.raises(capi.HsvError) as e:
+                s.apply_gates(bad)
+            assert e.value.code == -1
+            assert capi.counters()["gates"] == before + 6
+            assert np.array_equal(s.read(), r.read())
