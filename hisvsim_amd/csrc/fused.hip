@@ -930,6 +930,290 @@ __global__ __launch_bounds__(part_bf_threads(KT, STREAM_U)) __attribute__((amdgp
   }
 }
 
+// ---- step grouping on the device ---------------------------------------------
+// step_groups (partition.cpp), the beam search over the k-subsets of a wide
+// part's qubits that cuts its gates into the fewest fused steps, for all parts
+// of a call at once, with the same choices (extensions in the order of gates
+// left, state, subset; equal sets of gates left kept once). On the host it
+// takes 2 to 5 ms a part, several times the pass itself below 29 qubits. Each
+// level of the search is two launches: k_plan_score scores every (part, state,
+// subset), a wave 64 subsets of one state, over the whole chip; k_plan_select,
+// one workgroup per part and a wave per state, keeps the level's best. Bound by
+// the serial chain of levels and, in it, of kept extensions: for the 10 parts
+// of a 27-qubit QFT (12 levels) 8 to 15 us a score and 40 to 80 us a
+// selection, 0.9 ms in all. With one wave going through all states' extensions
+// and absorbing them again a selection took 200 to 700 us; all levels in one
+// workgroup per part, on 10 of the 256 CUs, 2.5 ms. The whole pass at 27
+// qubits: 34.1 -> 13.8 ms, at 16 qubits 3.0 ms.
+constexpr int kPlanGates = 128;   // gates of a part, at most (two 64-bit masks)
+constexpr int kPlanQubits = 14;
+constexpr int kPlanSubsets = 2002;  // C(14, 5)
+constexpr int kPlanStride = 2048;
+constexpr int kPlanWidth = 16;
+constexpr int kPlanLevels = 24;     // steps of a part, at most
+constexpr int kPlanThreads = 256;
+constexpr size_t kPlanParts = 64;   // parts searched at once (their states are 37 MB)
+constexpr double kPlanWork = 12500;  // subsets times gates from which the device is asked
+
+struct PlanPart {
+  int num_gates, num_qubits;
+  int masks;    // its first gate mask
+  int out;      // its answer: the number of groups, then their qubit sets (0 groups: not found)
+};
+
+// A part's search, in device memory.
+struct PlanState {
+  uint64_t rem[2][kPlanWidth][2];   // per state of a level: the gates left
+  uint64_t on[kPlanQubits][2];      // the gates on each qubit
+  int states, done;
+  uint32_t seen[8];                 // numbers of gates left that occur in the level
+  uint16_t set[kPlanLevels][kPlanWidth];
+  uint8_t parent[kPlanLevels][kPlanWidth];
+  uint16_t sub[kPlanStride];        // the subsets, lexicographic by ascending elements
+  // gates left after the extension of state b by subset q, at b * kPlanStride
+  // + q (255: it takes none)
+  alignas(16) uint8_t left[kPlanWidth * kPlanStride];
+  uint64_t keep[kPlanWidth * kPlanStride][2];  // the gates it leaves
+};
+
+__host__ __device__ constexpr int binomial(int n, int k) {
+  if (k < 0 || k > n) return 0;
+  int c = 1;
+  for (int i = 0; i < k; ++i) c = c * (n - i) / (i + 1);
+  return c;
+}
+
+// The gates of `rem` (two words) that the blocking scan of the qubit set Q
+// takes: those inside Q that share no qubit with an earlier skipped one. on[x]:
+// the gates on qubit x. The skipped ones grow from the gates that leave Q: on
+// each qubit of Q everything from its first skipped gate on, until no qubit
+// adds any (v | -v: the bits from v's lowest up). WIDE: more than 64 gates.
+template <bool WIDE>
+__device__ __forceinline__ void plan_absorb(uint64_t rem0, uint64_t rem1, const uint64_t (*on)[2], int n, uint32_t Q,
+                                            uint64_t* take0, uint64_t* take1) {
+  uint64_t s0 = 0, s1 = 0;
+  for (int x = 0; x < n; ++x) {
+    const uint64_t out = (Q >> x & 1) ? 0 : ~0ull;
+    s0 |= on[x][0] & out;
+    if constexpr (WIDE) s1 |= on[x][1] & out;
+  }
+  s0 &= rem0;
+  s1 &= rem1;
+  uint64_t q0[5], q1[5];
+  uint32_t rest = Q;
+#pragma unroll
+  for (int i = 0; i < 5; ++i) {  // fewer than five: qubit 0's gates of none
+    const int x = rest ? __builtin_ctz(rest) : 0;
+    q0[i] = rest ? on[x][0] & rem0 : 0;
+    q1[i] = WIDE && rest ? on[x][1] & rem1 : 0;
+    rest &= rest - 1;
+  }
+  for (;;) {
+    uint64_t a0 = s0, a1 = s1;
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+      const uint64_t v0 = a0 & q0[i], n0 = 0 - v0;
+      a0 |= q0[i] & (v0 | n0);
+      if constexpr (WIDE) {
+        const uint64_t v1 = a1 & q1[i];
+        a1 |= q1[i] & (v0 ? ~0ull : v1 | (0 - v1));
+      }
+    }
+    const bool more = a0 != s0 || (WIDE && a1 != s1);
+    s0 = a0;
+    s1 = a1;
+    if (!__ballot(more)) break;
+  }
+  *take0 = rem0 & ~s0;
+  *take1 = WIDE ? rem1 & ~s1 : 0;
+}
+
+__device__ __forceinline__ uint64_t uniform64(uint64_t x) {
+  return uint64_t(uint32_t(__builtin_amdgcn_readfirstlane((int)uint32_t(x)))) |
+         uint64_t(uint32_t(__builtin_amdgcn_readfirstlane((int)uint32_t(x >> 32)))) << 32;
+}
+
+__global__ __launch_bounds__(kPlanThreads) void k_plan_start(const PlanPart* __restrict__ parts,
+                                                             const uint16_t* __restrict__ masks, int k,
+                                                             PlanState* __restrict__ states, uint16_t* __restrict__ out) {
+  const PlanPart P = parts[blockIdx.x];
+  PlanState& S = states[blockIdx.x];
+  const int n = P.num_qubits, kk = k < n ? k : n, ns = binomial(n, kk), ng = P.num_gates;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (int q = threadIdx.x; q < ns; q += kPlanThreads) {
+    int r = q, x = 0;
+    uint32_t c = 0;
+    for (int i = 0; i < kk; ++i, ++x) {
+      for (int b; r >= (b = binomial(n - 1 - x, kk - 1 - i)); ++x) r -= b;
+      c |= 1u << x;
+    }
+    S.sub[q] = (uint16_t)c;
+  }
+  for (int x = wave; x < 2 * n; x += kPlanThreads / 64) {
+    const int i = 64 * (x & 1) + lane;
+    const uint64_t g = __ballot(i < ng && (masks[P.masks + i] >> (x >> 1) & 1));
+    if (lane == 0) S.on[x >> 1][x & 1] = g;
+  }
+  if (threadIdx.x < 8) S.seen[threadIdx.x] = 0;
+  if (threadIdx.x == 0) {
+    S.rem[0][0][0] = ng >= 64 ? ~0ull : (1ull << ng) - 1;
+    S.rem[0][0][1] = ng <= 64 ? 0 : ng == 128 ? ~0ull : (1ull << (ng - 64)) - 1;
+    S.states = 1;
+    S.done = 0;
+    out[P.out] = 0;
+  }
+}
+
+// Level `level` of part blockIdx.y: state blockIdx.z, 256 subsets a block.
+__global__ __launch_bounds__(kPlanThreads) void k_plan_score(const PlanPart* __restrict__ parts, int k, int level,
+                                                             PlanState* __restrict__ states) {
+  const PlanPart P = parts[blockIdx.y];
+  PlanState& S = states[blockIdx.y];
+  const int b = blockIdx.z, n = P.num_qubits, kk = k < n ? k : n, ns = binomial(n, kk);
+  if (S.done || b >= S.states || (int)blockIdx.x * kPlanThreads >= ns) return;  // uniform
+  __shared__ uint64_t on[kPlanQubits][2];
+  if (threadIdx.x < 2 * n) on[threadIdx.x >> 1][threadIdx.x & 1] = S.on[threadIdx.x >> 1][threadIdx.x & 1];
+  __syncthreads();
+  const int q = blockIdx.x * kPlanThreads + threadIdx.x;
+  const uint64_t r0 = uniform64(S.rem[level & 1][b][0]), r1 = uniform64(S.rem[level & 1][b][1]);
+  const uint32_t Q = q < ns ? S.sub[q] : 0;
+  uint64_t t0, t1;
+  if (r1) plan_absorb<true>(r0, r1, on, n, Q, &t0, &t1);
+  else plan_absorb<false>(r0, r1, on, n, Q, &t0, &t1);
+  const int got = __popcll(t0) + __popcll(t1);
+  const int l = q < ns && got > 0 ? __popcll(r0) + __popcll(r1) - got : 255;
+  S.left[b * kPlanStride + q] = (uint8_t)l;
+  S.keep[b * kPlanStride + q][0] = r0 & ~t0;
+  S.keep[b * kPlanStride + q][1] = r1 & ~t1;
+  // one atomic per word and wave
+  for (int w = 0; w < 8; ++w) {
+    uint32_t bits = (l >> 5) == w ? 1u << (l & 31) : 0;
+    for (int m = 32; m >= 1; m >>= 1) bits |= __shfl_xor(bits, m);
+    if ((threadIdx.x & 63) == 0 && bits) atomicOr(&S.seen[w], bits);
+  }
+}
+
+// Keeps the best kPlanWidth extensions of a level, wave b going through state
+// b's: for each number of gates left, from the lowest, the waves list their
+// state's first distinct extensions (kPlanWidth of them are enough: each one
+// that the states before have already is one of the kept), and the first wave
+// takes them in order, those whose gates left are new.
+constexpr int kPlanSelect = 64 * kPlanWidth;
+__global__ __launch_bounds__(kPlanSelect) void k_plan_select(const PlanPart* __restrict__ parts, int k, int level,
+                                                             PlanState* __restrict__ states,
+                                                             uint16_t* __restrict__ out) {
+  const PlanPart P = parts[blockIdx.x];
+  PlanState& S = states[blockIdx.x];
+  if (S.done) return;  // uniform
+  const int n = P.num_qubits, kk = k < n ? k : n, ns = binomial(n, kk), now = level & 1, nstates = S.states;
+  __shared__ __align__(16) uint8_t left[kPlanWidth * kPlanStride];
+  __shared__ uint64_t list[kPlanWidth][kPlanWidth][2];
+  __shared__ uint16_t list_q[kPlanWidth][kPlanWidth];
+  __shared__ int listed[kPlanWidth], taken_sh;
+  const int rows = (ns + 255) / 256;  // 256-byte rows that were scored, per state
+  for (int i = threadIdx.x; i < nstates * rows * 16; i += kPlanSelect) {
+    const int b = i / (rows * 16), o = b * kPlanStride + (i - b * rows * 16) * 16;
+    *reinterpret_cast<uint4*>(left + o) = *reinterpret_cast<const uint4*>(S.left + o);
+  }
+  uint32_t seen[8];
+#pragma unroll
+  for (int w = 0; w < 8; ++w) seen[w] = S.seen[w];
+  const int lane = threadIdx.x & 63, b = threadIdx.x >> 6;
+  int taken = 0;
+  uint64_t kept0 = 0, kept1 = 0;  // first wave, lane j: the gates left of the j-th kept extension
+  __syncthreads();  // left; every thread has read seen
+  if (threadIdx.x < 8) S.seen[threadIdx.x] = 0;
+  for (int v = 0; v < 255 && taken < kPlanWidth; ++v) {
+    if (!(seen[v >> 5] >> (v & 31) & 1)) continue;  // uniform
+    int mine = 0;
+    uint64_t own0 = 0, own1 = 0;
+    int own_q = 0;
+    for (int q0 = 0; b < nstates && q0 < ns && mine < kPlanWidth; q0 += 256) {
+      // four numbers a lane: which of the 256 are v
+      const uint32_t w = *reinterpret_cast<const uint32_t*>(left + b * kPlanStride + q0 + 4 * lane);
+      const bool any = (w & 255u) == (uint32_t)v || (w >> 8 & 255u) == (uint32_t)v || (w >> 16 & 255u) == (uint32_t)v ||
+                       w >> 24 == (uint32_t)v;
+      const uint64_t quads = __ballot(any);
+      for (int c = 0; c < 4 && mine < kPlanWidth; ++c) {
+        if (!(quads >> (16 * c) & 0xffffu)) continue;
+        const int q = q0 + 64 * c + lane;
+        uint64_t hits = __ballot(left[b * kPlanStride + q] == (uint8_t)v);
+        const uint64_t k0 = S.keep[b * kPlanStride + q][0], k1 = S.keep[b * kPlanStride + q][1];
+        while (hits && mine < kPlanWidth) {
+          const int h = __builtin_ctzll(hits);
+          const uint64_t h0 = uint64_t(uint32_t(__builtin_amdgcn_readlane((int)uint32_t(k0), h))) |
+                              uint64_t(uint32_t(__builtin_amdgcn_readlane((int)uint32_t(k0 >> 32), h))) << 32;
+          const uint64_t h1 = uint64_t(uint32_t(__builtin_amdgcn_readlane((int)uint32_t(k1), h))) |
+                              uint64_t(uint32_t(__builtin_amdgcn_readlane((int)uint32_t(k1 >> 32), h))) << 32;
+          hits &= ~__ballot(k0 == h0 && k1 == h1);  // with it the others that leave the same gates
+          if (__ballot(lane < mine && own0 == h0 && own1 == h1)) continue;
+          if (lane == mine) {
+            own0 = h0;
+            own1 = h1;
+            own_q = q0 + 64 * c + h;
+          }
+          ++mine;
+        }
+      }
+    }
+    if (lane < mine) {
+      list[b][lane][0] = own0;
+      list[b][lane][1] = own1;
+      list_q[b][lane] = (uint16_t)own_q;
+    }
+    if (lane == 0) listed[b] = mine;
+    __syncthreads();
+    if (v == 0) {  // a state without gates left: the search ends with its first
+      if (threadIdx.x == 0) {
+        int x = 0;
+        while (!listed[x]) ++x;
+        uint16_t* o = out + P.out;
+        o[0] = (uint16_t)(level + 1);
+        o[1 + level] = S.sub[list_q[x][0]];
+        for (int at = level - 1; at >= 0; --at) {
+          o[1 + at] = S.set[at][x];
+          x = S.parent[at][x];
+        }
+        S.done = 1;
+      }
+      return;
+    }
+    if (b == 0) {
+      for (int x = 0; x < nstates && taken < kPlanWidth; ++x) {
+        const int cnt = listed[x];
+        const uint64_t k0 = lane < cnt ? list[x][lane][0] : 0, k1 = lane < cnt ? list[x][lane][1] : 0;
+        for (int h = 0; h < cnt && taken < kPlanWidth; ++h) {
+          const uint64_t h0 = uint64_t(uint32_t(__builtin_amdgcn_readlane((int)uint32_t(k0), h))) |
+                              uint64_t(uint32_t(__builtin_amdgcn_readlane((int)uint32_t(k0 >> 32), h))) << 32;
+          const uint64_t h1 = uint64_t(uint32_t(__builtin_amdgcn_readlane((int)uint32_t(k1), h))) |
+                              uint64_t(uint32_t(__builtin_amdgcn_readlane((int)uint32_t(k1 >> 32), h))) << 32;
+          if (__ballot(lane < taken && kept0 == h0 && kept1 == h1)) continue;
+          if (lane == taken) {
+            kept0 = h0;
+            kept1 = h1;
+            S.parent[level][taken] = (uint8_t)x;
+            S.set[level][taken] = S.sub[list_q[x][h]];
+          }
+          ++taken;
+        }
+      }
+      if (lane == 0) taken_sh = taken;
+    }
+    __syncthreads();  // the lists are read
+    taken = taken_sh;
+  }
+  if (b == 0) {
+    if (lane < taken) {
+      S.rem[now ^ 1][lane][0] = kept0;
+      S.rem[now ^ 1][lane][1] = kept1;
+    }
+    if (lane == 0) {
+      S.states = taken;
+      if (!taken) S.done = 1;  // no gate fits: the host reports it
+    }
+  }
+}
+
 namespace {
 
 // the highest `count` slots of an outer mask (the tile kernels' fast slots)
@@ -1110,9 +1394,12 @@ int rank_gf2(uint32_t* v, int n) {
 struct PartSwizzleKey { int cbit[4]; int rbit0; };
 
 void choose_part_swizzle(int KT, const std::vector<PartSwizzleKey>& keys, uint32_t nimg[14]) {
+  int best = -1;
   auto score = [&](const uint32_t* m) {
-    int sc = 0;
+    int sc = 0, open = 3 * (int)keys.size();
     for (const PartSwizzleKey& k : keys) {
+      if (sc + open <= best) return sc;  // cannot become the best any more
+      open -= 3;
       auto low5 = [&](int c) { return ((c < 5) ? (1u << c) : 0u) ^ m[c]; };
       uint32_t a[4], b[5];
       for (int j = 0; j < 4; ++j) { b[j] = low5(k.cbit[j]); a[j] = b[j] & 15u; }
@@ -1124,7 +1411,7 @@ void choose_part_swizzle(int KT, const std::vector<PartSwizzleKey>& keys, uint32
   const int best_possible = 3 * (int)keys.size();
   uint32_t cand[14] = {0};
   std::memcpy(nimg, cand, sizeof(cand));
-  int best = score(cand);
+  best = score(cand);
   uint64_t rng = 0x9E3779B97F4A7C15ull;
   for (int it = 0; it < 2000 && best < best_possible; ++it) {
     for (int c = 0; c < 14; ++c) {
@@ -1162,7 +1449,8 @@ void launch_part_bf(void* amp, const unsigned char* dev, size_t tabs_off, size_t
 // 12- and 13-qubit tiles).
 int part_apply_bf(void* amp, int n, int dtype, hipStream_t stream, DeviceScratch* scratch,
                   const std::vector<Lowered>& gates, uint64_t tile_qubits, const int* phys,
-                  const int* phys_after, uint64_t live_slots, const BfTune& bf, std::string* err, int pieces) {
+                  const int* phys_after, uint64_t live_slots, const BfTune& bf, std::string* err, int pieces,
+                  const std::vector<std::vector<int>>* planned = nullptr) {
   int tpw = bf.part_tpw;
   int ph[64], pa[64], inv[64];
   for (int q = 0; q < n; ++q) ph[q] = phys ? phys[q] : q;
@@ -1232,7 +1520,8 @@ int part_apply_bf(void* amp, int n, int dtype, hipStream_t stream, DeviceScratch
   for (int j = 0; j < KT; ++j) moves = moves || sslot[j] != slot[j];
   if (qm.empty() && !moves) return HSV_OK;  // identities only
   // the steps: groups of <= 5 qubits, as few as a beam of 16 finds
-  std::vector<std::vector<int>> groups = qm.empty() ? std::vector<std::vector<int>>() : step_groups(qm, 5, 16);
+  std::vector<std::vector<int>> groups;
+  if (!qm.empty()) groups = planned && !planned->empty() ? *planned : step_groups(qm, 5, kPlanWidth);
   if (groups.empty() && !qm.empty()) {
     *err = "a gate acts on more than 5 qubits: the wide bf16 fused path cannot take it";
     return HSV_ERR_LIMIT;
@@ -1637,9 +1926,114 @@ int fused_apply_bf(void* amp, int n, int dtype, hipStream_t stream, int num_cu, 
 int fused_part_bf_layout(void* amp, int n, int dtype, hipStream_t stream, DeviceScratch* scratch,
                          const std::vector<Lowered>& gates, uint64_t tile_qubits, const int* phys,
                          const int* phys_after, uint64_t live_slots, const BfTune& bf, std::string* err,
-                         int pieces) {
+                         int pieces, const std::vector<std::vector<int>>* groups) {
   return part_apply_bf(amp, n, dtype, stream, scratch, gates, tile_qubits, phys, phys_after, live_slots, bf, err,
-                       pieces);
+                       pieces, groups);
+}
+
+int fused_plan_steps(hipStream_t stream, DeviceScratch* scratch, void* host, size_t host_bytes,
+                     const std::vector<std::vector<uint64_t>>& masks, int k, std::vector<std::vector<std::vector<int>>>* groups, std::string* err) {
+  groups->assign(masks.size(), {});
+  struct Wanted {
+    size_t part;
+    uint64_t all;
+    std::vector<int> live;  // its gates that act on something
+  };
+  auto* base = static_cast<unsigned char*>(host);
+  size_t p0 = 0;
+  while (p0 < masks.size()) {
+    // as many parts as the buffer takes: headers | gate masks | answers
+    std::vector<Wanted> want;
+    size_t gates = 0;
+    double work = 0;
+    for (; p0 < masks.size(); ++p0) {
+      Wanted w{p0, 0, {}};
+      bool fits = true;
+      for (size_t i = 0; i < masks[p0].size(); ++i) {
+        if (!masks[p0][i]) continue;
+        w.live.push_back((int)i);
+        w.all |= masks[p0][i];
+        fits = fits && __builtin_popcountll(masks[p0][i]) <= k;
+      }
+      const int nq = __builtin_popcountll(w.all);
+      if (!fits || w.live.size() < 2 || w.live.size() > size_t(kPlanGates) || nq > kPlanQubits ||
+          binomial(nq, std::min(k, nq)) > kPlanSubsets)
+        continue;
+      const size_t need = (want.size() + 1) * sizeof(PlanPart) + (gates + w.live.size()) * 4 + (want.size() + 1) * 2;
+      if (need > host_bytes || want.size() == kPlanParts) break;
+      gates += w.live.size();
+      work += double(binomial(nq, std::min(k, nq))) * double(w.live.size());
+      want.push_back(std::move(w));
+    }
+    // the host's search takes about 40 ns a subset and gate, the device's
+    // (launch and wait included) about 0.5 to 1 ms whatever the number of parts
+    if (want.empty() || work < kPlanWork) continue;
+    auto* parts = reinterpret_cast<PlanPart*>(base);
+    auto* gm = reinterpret_cast<uint16_t*>(base + want.size() * sizeof(PlanPart));
+    auto* out = gm + gates;
+    int mo = 0, oo = 0;
+    for (size_t w = 0; w < want.size(); ++w) {
+      parts[w] = PlanPart{(int)want[w].live.size(), __builtin_popcountll(want[w].all), mo, oo};
+      for (int i : want[w].live) {
+        // qubit bits to the part's own, ascending
+        uint32_t c = 0;
+        int j = 0;
+        for (uint64_t a = want[w].all; a; a &= a - 1, ++j)
+          if (masks[want[w].part][i] & a & (~a + 1)) c |= 1u << j;
+        gm[mo++] = (uint16_t)c;
+      }
+      oo += (int)want[w].live.size() + 1;
+    }
+    if (int rc = ensure_scratch(scratch, want.size() * sizeof(PlanState), stream, err)) {
+      if (rc != HSV_ERR_ALLOC) return rc;
+      (void)hipGetLastError();  // no room on the card: the rest is searched on the host
+      err->clear();
+      return HSV_OK;
+    }
+    auto* st = static_cast<PlanState*>(scratch->ptr);
+    const unsigned np = (unsigned)want.size();
+    size_t most = 0;
+    int blocks = 0;
+    for (size_t w = 0; w < want.size(); ++w) {
+      most = std::max(most, want[w].live.size());
+      const int nq = parts[w].num_qubits;
+      blocks = std::max(blocks, (binomial(nq, std::min(k, nq)) + kPlanThreads - 1) / kPlanThreads);
+    }
+    hipLaunchKernelGGL(k_plan_start, np, kPlanThreads, 0, stream, parts, gm, k, st, out);
+    for (int level = 0; level < std::min<int>(kPlanLevels, (int)most); ++level) {
+      hipLaunchKernelGGL(k_plan_score, dim3(blocks, np, level ? kPlanWidth : 1), kPlanThreads, 0, stream, parts, k,
+                         level, st);
+      hipLaunchKernelGGL(k_plan_select, np, kPlanSelect, 0, stream, parts, k, level, st, out);
+    }
+    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(stream) != hipSuccess) {
+      *err = "step grouping failed on the device";
+      return HSV_ERR_DEVICE;
+    }
+    for (size_t w = 0; w < want.size(); ++w) {
+      const uint16_t* o = out + parts[w].out;
+      const uint16_t* m = gm + parts[w].masks;
+      // the sets' blocking scans, one after another (none when not found)
+      std::vector<int> rem(want[w].live.size());
+      for (size_t i = 0; i < rem.size(); ++i) rem[i] = (int)i;
+      for (int g = 0; g < o[0]; ++g) {
+        const uint32_t Q = o[1 + g];
+        uint32_t blocked = 0;
+        std::vector<int> taken, keep;
+        for (int i : rem) {
+          if ((m[i] & blocked) || (m[i] & ~Q)) {
+            blocked |= m[i];
+            keep.push_back(i);
+          } else {
+            taken.push_back(want[w].live[i]);
+          }
+        }
+        (*groups)[want[w].part].push_back(std::move(taken));
+        rem.swap(keep);
+      }
+      if (!rem.empty()) (*groups)[want[w].part].clear();
+    }
+  }
+  return HSV_OK;
 }
 
 int fused_apply(void* amp, int n, int dtype, hipStream_t stream, int num_cu, DeviceScratch* scratch,

@@ -54,11 +54,22 @@ int fused_apply(void* amp, int n, int dtype, hipStream_t stream, int num_cu, Dev
 // nonzero amplitude (the others hold |0> on the whole state, so tiles with
 // such a bit set are zero and are skipped); ~0 when nothing is known.
 // pieces: BF16 pieces per value, 2 (HSV_FUSED_BF16SPLIT) or 3
-// (HSV_FUSED_BF16X3, 12- and 13-qubit tiles).
+// (HSV_FUSED_BF16X3, 12- and 13-qubit tiles). groups: the part's steps (gate
+// indices, identities left out) from fused_plan_steps; null or empty: searched
+// here.
 int fused_part_bf_layout(void* amp, int n, int dtype, hipStream_t stream, DeviceScratch* scratch,
                          const std::vector<Lowered>& gates, uint64_t tile_qubits, const int* phys,
                          const int* phys_after, uint64_t live_slots, const BfTune& bf, std::string* err,
-                         int pieces = 2);
+                         int pieces = 2, const std::vector<std::vector<int>>* groups = nullptr);
+
+// The step groups of several wide parts at once, searched on the device with
+// the choices of step_groups (partition.hpp, width 16): masks[p][i] = the
+// tile bits of part p's i-th gate (0: an identity, in no group). (*groups)[p]
+// stays empty where the host's own search is to run: parts too large for the
+// kernels, gates on more than k qubits, too little work in all to be worth a
+// launch. host: pinned memory that the kernel reads and writes.
+int fused_plan_steps(hipStream_t stream, DeviceScratch* scratch, void* host, size_t host_bytes,
+                     const std::vector<std::vector<uint64_t>>& masks, int k, std::vector<std::vector<std::vector<int>>>* groups, std::string* err);
 
 // The fused unitary itself (for tests and the cost model): qubits of the
 // part (sorted, padded with the lowest free qubits to at least min_qubits)

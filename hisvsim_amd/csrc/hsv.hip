@@ -1543,6 +1543,28 @@ int hsv_apply_fused_chain(hsv_state* s, const hsv_gate* gates, int num_gates, co
   // skip the tiles with a 1 in its slot (the first parts run on a small corner
   // of the state)
   const uint64_t all_q = (n == 64) ? ~0ull : ((1ull << n) - 1);
+  // The parts' step groups. Below kPlanBytes of state a pass is shorter than
+  // the host's search for the next part's (2 to 3 ms): all of them are then
+  // searched on the device at once, before the first pass. (Not in the
+  // no-allocation form, which has no pinned memory to exchange them through;
+  // the groups are the same.)
+  constexpr uint64_t kPlanBytes = 8ull << 30;
+  std::vector<std::vector<std::vector<int>>> groups(num_parts);
+  if (s->len * s->elem() <= kPlanBytes && !s->fused_scratch.fixed) {
+    if (int rc = ensure_host_partial(s)) return rc;
+    std::vector<std::vector<uint64_t>> masks(num_parts);
+    size_t g0 = 0;
+    for (int p = 0; p < num_parts; g0 += part_sizes[p], ++p)
+      for (size_t g = g0; g < g0 + part_sizes[p]; ++g) {
+        uint64_t m = 0;
+        for (int q = 0; q < n; ++q)
+          if (gate_qubits(Ls[g]) >> q & 1) m |= 1ull << layout[p][q];
+        if (m) masks[p].push_back(m);
+      }
+    std::string err;
+    if (int rc = fused_plan_steps(s->stream, &s->fused_scratch, s->host_partial, sizeof(double) * 2 * kSumBlocks, masks, 5, &groups, &err))
+      return fail(rc, err);
+  }
   uint64_t support = s->support & all_q;
   s->support = ~0ull;  // until the state is back in the standard layout
   off = 0;
@@ -1555,7 +1577,7 @@ int hsv_apply_fused_chain(hsv_state* s, const hsv_gate* gates, int num_gates, co
     if (int rc = begin_timed(s)) return rc;
     std::string err;
     if (int rc = fused_part_bf_layout(s->amp, n, s->dtype, s->stream, &s->fused_scratch, part, tile[p],
-                                      layout[p].data(), layout[p + 1].data(), live, s->bf, &err, pieces)) {
+                                      layout[p].data(), layout[p + 1].data(), live, s->bf, &err, pieces, &groups[p])) {
       // close this part's timing pair, then bring the parts applied so far
       // back to the standard layout; a failed restore is reported too
       std::string msg = "part " + std::to_string(p) + ": " + err;

@@ -382,3 +382,42 @@ def test_gate_list_stops_at_the_gate_that_fails():
             assert e.value.code == -1
             assert capi.counters()["gates"] == before + 6
             assert np.array_equal(s.read(), r.read())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("circuit,n,k,reps", [("layered", 13, 12, 1), ("layered", 16, 13, 1), ("layered", 20, 14, 1),
+                                              ("qft", 14, 13, 1), ("qft", 18, 12, 2), ("one", 14, 13, 3),
+                                              ("one", 14, 13, 6), ("one", 14, 13, 12)])
+def test_device_step_groups_equal_the_hosts(circuit, n, k, reps):
+    """The chain, whose parts' steps are searched on the device, against its
+    no-allocation form, whose steps the host searches: the same steps give the
+    same bits. Parts of a few gates, of more than 64, of 128 and more (left to
+    the host), layout changes between parts."""
+    from hisvsim_amd import capi
+    from hisvsim_amd.circuit import Gate, qft, random_layered
+    rng = np.random.default_rng(n)
+    if circuit == "layered":
+        gs = random_layered(n, 5, n)
+    elif circuit == "qft":
+        gs = [Gate("U3", (q,), (), (0.3 + q, 0.2, 0.9)) for q in range(n)] + qft(n) * reps
+    else:  # one part on 13 of the qubits
+        gs = _some_gates(rng, list(range(13)), 9 * reps) + [Gate("RZZ", (0, q), (), (0.1 * q,)) for q in range(1, 13)]
+    if circuit == "one":
+        parts, lows = [gs], [list(range(5))]
+    else:
+        parts, lows = capi.chain_parts(gs, k, 5, 13, beam=(4, 4))
+    a = _stored(n, "complex128", 2)
+    with capi.State(n) as s, capi.State(n) as r:
+        for start in (None, a):
+            for x in (s, r):
+                x.reset()
+                if start is not None:
+                    x.write(start)
+            try:
+                r.apply_fused_chain(parts, lows, "bf16split", noalloc=True)
+            except capi.HsvError as e:      # more than 28 steps: not for that form's scratch
+                assert e.code == -5
+                s.apply_fused_chain(parts, lows, "bf16split")
+                continue
+            s.apply_fused_chain(parts, lows, "bf16split")
+            assert np.array_equal(s.read(), r.read())
