@@ -944,7 +944,7 @@ __global__ __launch_bounds__(part_bf_threads(KT, STREAM_U)) __attribute__((amdgp
 // selection, 0.9 ms in all. With one wave going through all states' extensions
 // and absorbing them again a selection took 200 to 700 us; all levels in one
 // workgroup per part, on 10 of the 256 CUs, 2.5 ms. The whole pass at 27
-// qubits: 34.1 -> 13.8 ms, at 16 qubits 3.0 ms.
+// qubits: 34.1 -> 13.8 ms.
 constexpr int kPlanGates = 128;   // gates of a part, at most (two 64-bit masks)
 constexpr int kPlanQubits = 14;
 constexpr int kPlanSubsets = 2002;  // C(14, 5)
@@ -1214,6 +1214,162 @@ __global__ __launch_bounds__(kPlanSelect) void k_plan_select(const PlanPart* __r
   }
 }
 
+// ---- the steps' matrices on the device -----------------------------------------
+// What the host does otherwise before each pass, 0.3 to 0.9 ms a part: 28 us a
+// step for the check that its matrix is unitary, 7 us for its BF16 fragments,
+// up to 0.4 ms for the part's swizzle. For all parts at once instead: 13 and 24
+// us for the 65 steps of a 27-qubit QFT, bound by latency (one workgroup a
+// step, a part).
+__host__ __device__ inline uint16_t bf16_bits(float f) {
+  // round to nearest even (finite inputs; NaN stays NaN)
+  uint32_t u;
+  __builtin_memcpy(&u, &f, 4);
+  if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40);
+  u += 0x7fffu + ((u >> 16) & 1u);
+  return (uint16_t)(u >> 16);
+}
+__host__ __device__ inline double bf16_value(uint16_t h) {
+  const uint32_t u = (uint32_t)h << 16;
+  float f;
+  __builtin_memcpy(&f, &u, 4);
+  return f;
+}
+// The BF16 fragments of a step's matrix in the MFMA's A-operand order: entry e
+// of lane `lane` in row block rb is U[part_bf_row][part_bf_col]; its pieces are
+// 64 * 8 apart, the real ones first.
+__host__ __device__ inline int part_bf_row(int rb, int lane) {
+  const int mm = lane % 16;
+  return 16 * rb + 4 * (mm % 4) + mm / 4;
+}
+__host__ __device__ inline int part_bf_col(int lane, int e) { return lane / 16 + 4 * e; }
+__host__ __device__ inline void part_bf_pieces(double re, double im, int pieces, uint16_t* frag) {
+  // each piece the BF16 of what the previous ones leave of the FP64 entry
+  for (int k = 0; k < pieces; ++k) {
+    const uint16_t pr = bf16_bits((float)re), pi = bf16_bits((float)im);
+    frag[size_t(k) * 64 * 8] = pr;
+    frag[size_t(pieces + k) * 64 * 8] = pi;
+    re -= bf16_value(pr);
+    im -= bf16_value(pi);
+  }
+}
+
+// One workgroup per step. uerr: max |U^H U - I|, a NaN left out as in
+// unitarity_error; -1 when an entry is not finite or huge (the host
+// then decides).
+constexpr int kStepThreads = 256;
+__global__ __launch_bounds__(kStepThreads) void k_part_steps(const double2* __restrict__ U, int pieces,
+                                                             uint16_t* __restrict__ frags, double* __restrict__ uerr) {
+  __shared__ double2 u[32 * 32];
+  __shared__ double worst[kStepThreads];
+  __shared__ int bad;
+  const int t = threadIdx.x;
+  if (t == 0) bad = 0;
+  __syncthreads();
+  for (int i = t; i < 32 * 32; i += kStepThreads) {
+    u[i] = U[size_t(blockIdx.x) * 1024 + i];
+    if (!(fabs(u[i].x) < 1e100 && fabs(u[i].y) < 1e100)) bad = 1;
+  }
+  __syncthreads();
+  double w = 0;
+  for (int p = t; p < 32 * 32; p += kStepThreads) {
+    const int i = p >> 5, j = p & 31;
+    double x = 0, y = 0;
+    for (int r = 0; r < 32; ++r) {
+      const double2 a = u[r * 32 + i], b = u[r * 32 + j];
+      x += a.x * b.x + a.y * b.y;
+      y += a.x * b.y - a.y * b.x;
+    }
+    if (i == j) x -= 1.0;
+    w = fmax(w, sqrt(x * x + y * y));
+  }
+  worst[t] = w;
+  __syncthreads();
+  for (int h = kStepThreads / 2; h; h >>= 1) {
+    if (t < h) worst[t] = fmax(worst[t], worst[t + h]);
+    __syncthreads();
+  }
+  if (t == 0) uerr[blockIdx.x] = bad ? -1.0 : worst[0];
+  uint16_t* f = frags + size_t(blockIdx.x) * 2 * 2 * pieces * 64 * 8;
+  for (int i = t; i < 2 * 64 * 8; i += kStepThreads) {
+    const int e = i & 7, lane = i >> 3 & 63, rb = i >> 9;
+    const double2 v = u[part_bf_row(rb, lane) * 32 + part_bf_col(lane, e)];
+    part_bf_pieces(v.x, v.y, pieces, f + (size_t(rb) * 2 * pieces * 64 + lane) * 8 + e);
+  }
+}
+
+// The LDS swizzle of a part (choose_part_swizzle, with the same choice): its
+// 2000 candidates over the threads of a workgroup, each thread two that follow
+// each other in the generator's sequence, from its state before them.
+struct PartSwizzleKey { int cbit[4]; int rbit0; };
+struct SwizzlePart {
+  int KT, first, count;  // its keys
+};
+constexpr int kSwizzleTries = 2000, kSwizzleThreads = 1024, kSwizzleEach = 2;
+static_assert(kSwizzleThreads * kSwizzleEach >= kSwizzleTries, "a thread for each candidate");
+__host__ __device__ inline void swizzle_candidate(uint64_t* rng, int KT, uint32_t* cand) {
+  uint64_t r = *rng;
+  for (int c = 0; c < 14; ++c) {
+    r ^= r << 13;
+    r ^= r >> 7;
+    r ^= r << 17;
+    cand[c] = c < 4 ? 0u : (c == 4 ? uint32_t(r & 15u) : (c < KT ? uint32_t(r & 31u) : 0u));
+  }
+  *rng = r;
+}
+__global__ __launch_bounds__(kSwizzleThreads) void k_part_swizzle(const SwizzlePart* __restrict__ parts,
+                                                                  const PartSwizzleKey* __restrict__ keys,
+                                                                  const uint64_t* __restrict__ rng,
+                                                                  uint32_t* __restrict__ nimg) {
+  const SwizzlePart P = parts[blockIdx.x];
+  __shared__ uint32_t img[14][kSwizzleThreads + 1];  // a thread's candidate: a column
+  __shared__ int best[kSwizzleThreads];              // score * 4096 + 4095 - (its place in the sequence)
+  const int t = threadIdx.x;
+  int mine = -1;
+  uint64_t r = t * kSwizzleEach < kSwizzleTries ? rng[t] : 0;
+  // the sequence: no swizzle at all, then the candidates
+  for (int e = -1; e < kSwizzleEach; ++e) {
+    if (e < 0 ? t != 0 : t * kSwizzleEach + e >= kSwizzleTries) continue;
+    uint32_t cand[14] = {0};
+    if (e >= 0) swizzle_candidate(&r, P.KT, cand);
+#pragma unroll
+    for (int c = 0; c < 14; ++c) img[c][t] = (c < 5 ? 1u << c : 0u) ^ cand[c];
+    int sc = 0;
+    for (int k = P.first; k < P.first + P.count; ++k) {
+      uint32_t v[5];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = img[keys[k].cbit[j]][t];
+      v[4] = img[keys[k].rbit0][t];
+      // independent: no sum of some of them is 0
+      uint32_t sum[32];
+      bool four = true, five = true;
+      sum[0] = 0;
+#pragma unroll
+      for (int m = 1; m < 32; ++m) {
+        sum[m] = sum[m & (m - 1)] ^ v[__builtin_ctz(m)];
+        five = five && (sum[m] & 31u);
+        if (m < 16) four = four && (sum[m] & 15u);
+      }
+      sc += 2 * four + five;
+    }
+    mine = max(mine, sc * 4096 + 4095 - (t * kSwizzleEach + e + 1));
+  }
+  best[t] = mine;
+  __syncthreads();
+  for (int h = kSwizzleThreads / 2; h; h >>= 1) {
+    if (t < h) best[t] = max(best[t], best[t + h]);
+    __syncthreads();
+  }
+  if (t == 0) {
+    const int at = 4095 - (best[0] & 4095) - 1;  // -1: no swizzle
+    uint32_t cand[14] = {0};
+    if (at >= 0) {
+      uint64_t q = rng[at / kSwizzleEach];
+      for (int e = 0; e <= at % kSwizzleEach; ++e) swizzle_candidate(&q, P.KT, cand);
+    }
+    for (int c = 0; c < 14; ++c) nimg[blockIdx.x * 14 + c] = cand[c];
+  }
+}
+
 namespace {
 
 // the highest `count` slots of an outer mask (the tile kernels' fast slots)
@@ -1279,21 +1435,6 @@ int fused_unitary(int n, const std::vector<Lowered>& gates, std::vector<int>* qu
 }
 
 namespace {
-
-// Round-to-nearest-even FP32 -> BF16 (finite inputs; NaN stays NaN).
-uint16_t bf16_rne(float f) {
-  uint32_t u;
-  std::memcpy(&u, &f, 4);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
-}
-double bf16_value(uint16_t h) {
-  const uint32_t u = (uint32_t)h << 16;
-  float f;
-  std::memcpy(&f, &u, 4);
-  return f;
-}
 
 int ensure_scratch(DeviceScratch* scratch, size_t bytes, hipStream_t stream, std::string* err) {
   if (scratch->bytes >= bytes) return HSV_OK;
@@ -1391,7 +1532,7 @@ int rank_gf2(uint32_t* v, int n) {
   return r;
 }
 
-struct PartSwizzleKey { int cbit[4]; int rbit0; };
+constexpr uint64_t kSwizzleSeed = 0x9E3779B97F4A7C15ull;
 
 void choose_part_swizzle(int KT, const std::vector<PartSwizzleKey>& keys, uint32_t nimg[14]) {
   int best = -1;
@@ -1412,12 +1553,9 @@ void choose_part_swizzle(int KT, const std::vector<PartSwizzleKey>& keys, uint32
   uint32_t cand[14] = {0};
   std::memcpy(nimg, cand, sizeof(cand));
   best = score(cand);
-  uint64_t rng = 0x9E3779B97F4A7C15ull;
-  for (int it = 0; it < 2000 && best < best_possible; ++it) {
-    for (int c = 0; c < 14; ++c) {
-      rng ^= rng << 13; rng ^= rng >> 7; rng ^= rng << 17;
-      cand[c] = c < 4 ? 0u : (c == 4 ? uint32_t(rng & 15u) : (c < KT ? uint32_t(rng & 31u) : 0u));
-    }
+  uint64_t rng = kSwizzleSeed;
+  for (int it = 0; it < kSwizzleTries && best < best_possible; ++it) {
+    swizzle_candidate(&rng, KT, cand);
     const int sc = score(cand);
     if (sc > best) { best = sc; std::memcpy(nimg, cand, sizeof(cand)); }
   }
@@ -1440,18 +1578,13 @@ void launch_part_bf(void* amp, const unsigned char* dev, size_t tabs_off, size_t
                      reinterpret_cast<const bf8*>(dev + frag_off), nsteps, ntiles, outer, top, tpw);
 }
 
-// A part of 8..14 qubits on the BF16-split path (see k_part_bf).
-// tile_qubits: the (logical) qubits the tile must hold, at least those of
-// the gates. Logical qubit q sits in slot phys[q] (q when phys is null) and
-// the store leaves it in slot phys_after[q] (unchanged when null): a layout
-// change that must keep every qubit outside the tile where it is.
-// pieces: BF16 pieces per value (2, or 3 for FP32-class products; 3 takes
-// 12- and 13-qubit tiles).
-int part_apply_bf(void* amp, int n, int dtype, hipStream_t stream, DeviceScratch* scratch,
-                  const std::vector<Lowered>& gates, uint64_t tile_qubits, const int* phys,
-                  const int* phys_after, uint64_t live_slots, const BfTune& bf, std::string* err, int pieces,
-                  const std::vector<std::vector<int>>* planned = nullptr) {
-  int tpw = bf.part_tpw;
+// fused_part_prepare and fused_part_launch for a part of 8 to 14 qubits (see
+// k_part_bf); phys null: logical qubit q sits in slot q, phys_after null: it
+// stays there.
+int part_prepare_bf(int n, const std::vector<Lowered>& gates, uint64_t tile_qubits, const int* phys,
+                    const int* phys_after, int pieces, const std::vector<std::vector<int>>* planned, FusedPart* P,
+                    std::string* err) {
+  *P = FusedPart();
   int ph[64], pa[64], inv[64];
   for (int q = 0; q < n; ++q) ph[q] = phys ? phys[q] : q;
   for (int q = 0; q < n; ++q) {
@@ -1467,7 +1600,7 @@ int part_apply_bf(void* amp, int n, int dtype, hipStream_t stream, DeviceScratch
   // 512-byte runs: a part that fits 12 qubits only without them takes a
   // 13-qubit tile.
   const uint64_t low5 = (1ull << std::min(n, 5)) - 1;
-  const int KT = std::max(12, std::min(14, __builtin_popcountll(pmask | low5)));
+  const int KT = P->KT = std::max(12, std::min(14, __builtin_popcountll(pmask | low5)));
   if (K > 14) {
     *err = "the bf16 fused path takes parts of at most 14 qubits";
     return HSV_ERR_LIMIT;
@@ -1482,7 +1615,7 @@ int part_apply_bf(void* amp, int n, int dtype, hipStream_t stream, DeviceScratch
   }
   uint64_t tmask = pmask;
   for (int b = 0; b < n && __builtin_popcountll(tmask) < KT; ++b) tmask |= 1ull << b;
-  int slot[14], sslot[14];
+  int *slot = P->slot, *sslot = P->sslot;
   uint64_t smask = 0;
   for (int b = 0, j = 0; b < 64 && j < KT; ++b)
     if (tmask >> b & 1) {
@@ -1516,9 +1649,10 @@ int part_apply_bf(void* amp, int n, int dtype, hipStream_t stream, DeviceScratch
     qm.push_back(m);
     gl.push_back(&L);
   }
-  bool moves = false;
-  for (int j = 0; j < KT; ++j) moves = moves || sslot[j] != slot[j];
-  if (qm.empty() && !moves) return HSV_OK;  // identities only
+  P->tmask = tmask;
+  for (int j = 0; j < KT; ++j) P->moves = P->moves || sslot[j] != slot[j];
+  P->nothing = qm.empty() && !P->moves;  // identities only
+  if (P->nothing) return HSV_OK;
   // the steps: groups of <= 5 qubits, as few as a beam of 16 finds
   std::vector<std::vector<int>> groups;
   if (!qm.empty()) groups = planned && !planned->empty() ? *planned : step_groups(qm, 5, kPlanWidth);
@@ -1526,75 +1660,87 @@ int part_apply_bf(void* amp, int n, int dtype, hipStream_t stream, DeviceScratch
     *err = "a gate acts on more than 5 qubits: the wide bf16 fused path cannot take it";
     return HSV_ERR_LIMIT;
   }
-  const int ns = (int)groups.size();
-  std::vector<PartBfStep> steps(ns);
-  std::vector<PartSwizzleKey> keys(ns);
-  const int nsets = 2 * pieces;   // real pieces, then imaginary pieces
-  const size_t step_frag_bytes = size_t(2) * nsets * 64 * 16;
-  std::vector<uint16_t> frags(size_t(ns) * 2 * nsets * 64 * 8);
-  for (int s = 0; s < ns; ++s) {
+  P->steps.resize(groups.size());
+  for (size_t s = 0; s < groups.size(); ++s) {
+    FusedPart::Step& S = P->steps[s];
     uint64_t gm = 0;
     std::vector<Lowered> sg;
     for (int i : groups[s]) { gm |= qm[i]; sg.push_back(*gl[i]); }
     for (int b = 0; b < KT && __builtin_popcountll(gm) < 5; ++b) gm |= 1ull << b;  // pad: U (x) I
-    int rbit[5], cbit[9];
     std::vector<int> qubits;
     for (int b = 0, r = 0, c = 0; b < KT; ++b) {
-      if (gm >> b & 1) { rbit[r++] = b; qubits.push_back(inv[slot[b]]); }
-      else cbit[c++] = b;
+      if (gm >> b & 1) { S.rbit[r++] = b; qubits.push_back(inv[slot[b]]); }
+      else S.cbit[c++] = b;
     }
-    std::vector<cd> U;
-    build_fused(sg, qubits, &U);
-    const double uerr = unitarity_error(U, 32);
+    build_fused(sg, qubits, &S.U);
+  }
+  return HSV_OK;
+}
+
+// A part's keys for the swizzle: its steps' columns, and the store gather of a
+// layout change, which reads a quarter-wave's 16 positions along load bits
+// sig^-1(0..3): its banks count like a step's columns. sig_inv: tile bit j's
+// qubit moves to tile bit sig[j] (the tile position of its new slot); store
+// position u reads load position sig^-1(u).
+std::vector<PartSwizzleKey> part_keys(const FusedPart& P, int* sig_inv) {
+  std::vector<PartSwizzleKey> keys;
+  for (const FusedPart::Step& S : P.steps)
+    keys.push_back(PartSwizzleKey{{S.cbit[0], S.cbit[1], S.cbit[2], S.cbit[3]}, S.rbit[0]});
+  for (int j = 0; j < P.KT; ++j)
+    for (int k = 0; k < P.KT; ++k)
+      if (P.slot[k] == P.sslot[j]) sig_inv[k] = j;
+  if (P.moves) keys.push_back(PartSwizzleKey{{sig_inv[0], sig_inv[1], sig_inv[2], sig_inv[3]}, sig_inv[4]});
+  return keys;
+}
+
+// the tables of a part before its fragments
+size_t part_tables_bytes(size_t ns) {
+  return (2 * sizeof(PartBfTables) + sizeof(PartBfStep) * ns + 255) & ~size_t(255);
+}
+
+int part_launch_bf(void* amp, int n, int dtype, hipStream_t stream, DeviceScratch* scratch, const FusedPart& P,
+                   uint64_t live_slots, const BfTune& bf, int pieces, std::string* err) {
+  if (P.nothing) return HSV_OK;
+  int tpw = bf.part_tpw;
+  const int KT = P.KT, ns = (int)P.steps.size();
+  const uint64_t tmask = P.tmask;
+  const int* slot = P.slot;
+  std::vector<PartBfStep> steps(ns);
+  const int nsets = 2 * pieces;   // real pieces, then imaginary pieces
+  const size_t step_frag_bytes = size_t(2) * nsets * 64 * 16;
+  std::vector<uint16_t> frags(P.checked ? 0 : size_t(ns) * 2 * nsets * 64 * 8);
+  for (int s = 0; s < ns; ++s) {
+    const FusedPart::Step& F = P.steps[s];
+    const double uerr = P.checked && P.uerr[s] >= 0 ? P.uerr[s] : unitarity_error(F.U, 32);
     if (!(uerr <= 1e-10)) {
       *err = "fused step matrix is not unitary (max |U^H U - I| = " + std::to_string(uerr) + ")";
       return HSV_ERR_UNITARY;
     }
     PartBfStep& S = steps[s];
     std::memset(&S, 0, sizeof(S));
-    keys[s] = PartSwizzleKey{{cbit[0], cbit[1], cbit[2], cbit[3]}, rbit[0]};
     for (int r = 0; r < 32; ++r)
       for (int b = 0; b < 5; ++b)
-        if (r >> b & 1) S.rt[r] |= (uint16_t)(1u << rbit[b]);
+        if (r >> b & 1) S.rt[r] |= (uint16_t)(1u << F.rbit[b]);
     const int ncb = KT - 5;
     for (int v = 0; v < 32; ++v)
       for (int j = 0; j < 5; ++j) {
         if (!(v >> j & 1)) continue;
-        if (j < 4 && j < ncb && v < 16) S.ctl[v] |= (uint16_t)(1u << cbit[j]);
-        if (4 + j < ncb) S.cth[v] |= (uint16_t)(1u << cbit[4 + j]);
+        if (j < 4 && j < ncb && v < 16) S.ctl[v] |= (uint16_t)(1u << F.cbit[j]);
+        if (4 + j < ncb) S.cth[v] |= (uint16_t)(1u << F.cbit[4 + j]);
       }
-    for (int rb = 0; rb < 2; ++rb)
+    for (int rb = 0; rb < 2 && !P.checked; ++rb)
       for (int lane = 0; lane < 64; ++lane)
         for (int e = 0; e < 8; ++e) {
-          const int mm = lane % 16;
-          const int row = 16 * rb + 4 * (mm % 4) + mm / 4;
-          const int col = lane / 16 + 4 * e;
-          const cd u = U[size_t(row) * 32 + col];
-          const size_t f = size_t((s * 2 + rb) * nsets) * 64 + lane;
-          // each piece the BF16 of what the previous ones leave of the
-          // FP64 entry
-          double re = u.real(), im = u.imag();
-          for (int k = 0; k < pieces; ++k) {
-            const uint16_t pr = bf16_rne((float)re), pi = bf16_rne((float)im);
-            frags[(f + size_t(k) * 64) * 8 + e] = pr;
-            frags[(f + size_t(pieces + k) * 64) * 8 + e] = pi;
-            re -= bf16_value(pr);
-            im -= bf16_value(pi);
-          }
+          const cd u = F.U[size_t(part_bf_row(rb, lane)) * 32 + part_bf_col(lane, e)];
+          part_bf_pieces(u.real(), u.imag(), pieces, &frags[(size_t((s * 2 + rb) * nsets) * 64 + lane) * 8 + e]);
         }
   }
-  // tile bit j's qubit moves to tile bit sig[j] (the tile position of its new
-  // slot); store position u reads load position sig^-1(u)
-  int sig_inv[14];
-  for (int j = 0; j < KT; ++j)
-    for (int k = 0; k < KT; ++k)
-      if (slot[k] == sslot[j]) sig_inv[k] = j;
-  // the store gather of a layout change reads a quarter-wave's 16 positions
-  // along load bits sig^-1(0..3): its banks count like a step's columns
-  if (moves) keys.push_back(PartSwizzleKey{{sig_inv[0], sig_inv[1], sig_inv[2], sig_inv[3]}, sig_inv[4]});
   // swizzle the steps' LDS offsets (h is linear: XOR of the bits' images)
+  int sig_inv[14];
+  const std::vector<PartSwizzleKey> keys = part_keys(P, sig_inv);
   uint32_t nimg[14];
-  choose_part_swizzle(KT, keys, nimg);
+  if (P.checked) std::memcpy(nimg, P.nimg, sizeof(nimg));
+  else choose_part_swizzle(KT, keys, nimg);
   auto hmap = [&](uint32_t t) {
     uint32_t h = 0;
     for (int c = 4; c < KT; ++c)
@@ -1641,13 +1787,13 @@ int part_apply_bf(void* amp, int n, int dtype, hipStream_t stream, DeviceScratch
   const int max_steps = stream_u ? part_bf_max_steps(KT, pieces)
                                  : (int)std::min<size_t>(kPartBfMaxSteps, (160 * 1024 - static_lds) / step_frag_bytes);
   const size_t steps_off = 2 * sizeof(PartBfTables);
-  const size_t frag_off = (steps_off + sizeof(PartBfStep) * ns + 255) & ~size_t(255);
-  const size_t bytes = frag_off + frags.size() * 2;
+  const size_t own_off = part_tables_bytes(ns), bytes = own_off + frags.size() * 2;
+  const size_t frag_off = P.checked ? P.frag_off : own_off;
   std::vector<unsigned char> host(bytes);
   std::memcpy(host.data(), &T0, sizeof(T0));
   std::memcpy(host.data() + sizeof(T0), &T, sizeof(T));
   std::memcpy(host.data() + steps_off, steps.data(), sizeof(PartBfStep) * ns);
-  std::memcpy(host.data() + frag_off, frags.data(), frags.size() * 2);
+  if (!frags.empty()) std::memcpy(host.data() + own_off, frags.data(), frags.size() * 2);
   if (int rc = ensure_scratch(scratch, bytes, stream, err)) return rc;
   if (hipMemcpyAsync(scratch->ptr, host.data(), bytes, hipMemcpyHostToDevice, stream) != hipSuccess) {
     *err = "fused upload failed";
@@ -1698,6 +1844,14 @@ int part_apply_bf(void* amp, int n, int dtype, hipStream_t stream, DeviceScratch
     return HSV_ERR_DEVICE;
   }
   return HSV_OK;
+}
+
+int part_apply_bf(void* amp, int n, int dtype, hipStream_t stream, DeviceScratch* scratch,
+                  const std::vector<Lowered>& gates, uint64_t tile_qubits, const int* phys, const int* phys_after,
+                  uint64_t live_slots, const BfTune& bf, std::string* err, int pieces) {
+  FusedPart P;
+  if (int rc = part_prepare_bf(n, gates, tile_qubits, phys, phys_after, pieces, nullptr, &P, err)) return rc;
+  return part_launch_bf(amp, n, dtype, stream, scratch, P, live_slots, bf, pieces, err);
 }
 
 // The FP64 path on tiles (k_fused_tile). *taken = false, and nothing done, when
@@ -1843,9 +1997,9 @@ int fused_apply_bf(void* amp, int n, int dtype, hipStream_t stream, int num_cu, 
           const int row = 16 * rb + (swizzle ? 4 * (mm % 4) + mm / 4 : mm);
           const int col = 32 * ks + (swizzle ? g + 4 * e : 8 * g + e);
           const cd u = Um[size_t(row) * D + col];
-          const uint16_t rh = bf16_rne((float)u.real()), ih = bf16_rne((float)u.imag());
-          const uint16_t rl = bf16_rne((float)(u.real() - bf16_value(rh)));
-          const uint16_t il = bf16_rne((float)(u.imag() - bf16_value(ih)));
+          const uint16_t rh = bf16_bits((float)u.real()), ih = bf16_bits((float)u.imag());
+          const uint16_t rl = bf16_bits((float)(u.real() - bf16_value(rh)));
+          const uint16_t il = bf16_bits((float)(u.imag() - bf16_value(ih)));
           const size_t frag = size_t((rb * KS + ks) * 4) * 64;  // first of the 4 sets, in 8-element units
           hf[(frag + 0 * 64 + lane) * 8 + e] = rh;
           hf[(frag + 1 * 64 + lane) * 8 + e] = rl;
@@ -1923,16 +2077,105 @@ int fused_apply_bf(void* amp, int n, int dtype, hipStream_t stream, int num_cu, 
 
 }  // namespace
 
+int fused_part_prepare(int n, const std::vector<Lowered>& gates, uint64_t tile_qubits, const int* phys,
+                       const int* phys_after, int pieces, const std::vector<std::vector<int>>* groups, FusedPart* part,
+                       std::string* err) {
+  return part_prepare_bf(n, gates, tile_qubits, phys, phys_after, pieces, groups, part, err);
+}
+
+int fused_part_launch(void* amp, int n, int dtype, hipStream_t stream, DeviceScratch* scratch, const FusedPart& part,
+                      uint64_t live_slots, const BfTune& bf, int pieces, std::string* err) {
+  return part_launch_bf(amp, n, dtype, stream, scratch, part, live_slots, bf, pieces, err);
+}
+
 int fused_part_bf_layout(void* amp, int n, int dtype, hipStream_t stream, DeviceScratch* scratch,
                          const std::vector<Lowered>& gates, uint64_t tile_qubits, const int* phys,
                          const int* phys_after, uint64_t live_slots, const BfTune& bf, std::string* err,
-                         int pieces, const std::vector<std::vector<int>>* groups) {
+                         int pieces) {
   return part_apply_bf(amp, n, dtype, stream, scratch, gates, tile_qubits, phys, phys_after, live_slots, bf, err,
-                       pieces, groups);
+                       pieces);
+}
+
+int fused_parts_check(hipStream_t stream, DeviceScratch* scratch, void* host, size_t host_bytes, FusedPart* parts,
+                      int count, int pieces, std::string* err) {
+  // the answers in host: 14 swizzle images a part, then an error a step
+  std::vector<SwizzlePart> sw;
+  std::vector<PartSwizzleKey> keys;
+  std::vector<cd> U;
+  std::vector<int> which;
+  size_t ns = 0, tables = 0;
+  for (int p = 0; p < count; ++p) {
+    const FusedPart& P = parts[p];
+    if (P.steps.empty()) continue;
+    if ((sw.size() + 1) * 14 * sizeof(uint32_t) + 8 + (ns + P.steps.size()) * sizeof(double) > host_bytes) break;
+    int sig_inv[14];
+    const std::vector<PartSwizzleKey> k = part_keys(P, sig_inv);
+    sw.push_back(SwizzlePart{P.KT, (int)keys.size(), (int)k.size()});
+    keys.insert(keys.end(), k.begin(), k.end());
+    for (const FusedPart::Step& S : P.steps) U.insert(U.end(), S.U.begin(), S.U.end());
+    which.push_back(p);
+    ns += P.steps.size();
+    tables = std::max(tables, part_tables_bytes(P.steps.size()));
+  }
+  // parts without steps (a layout change alone) have tables too
+  tables = std::max(tables, part_tables_bytes(0));
+  if (which.empty()) return HSV_OK;
+  std::vector<uint64_t> rng(kSwizzleThreads);
+  uint64_t r = kSwizzleSeed;
+  uint32_t cand[14];
+  for (size_t t = 0; t < rng.size(); ++t) {
+    rng[t] = r;
+    for (int e = 0; e < kSwizzleEach; ++e) swizzle_candidate(&r, 14, cand);
+  }
+  // scratch: tables of the part under way | fragments | matrices | generator
+  // states | parts | keys
+  const size_t step_frag = size_t(2) * 2 * pieces * 64 * 16, u_off = tables + ns * step_frag,
+               rng_off = u_off + U.size() * sizeof(cd), sw_off = rng_off + rng.size() * sizeof(uint64_t),
+               key_off = sw_off + sw.size() * sizeof(SwizzlePart), end = key_off + keys.size() * sizeof(PartSwizzleKey);
+  std::vector<unsigned char> up(end - u_off);
+  std::memcpy(up.data(), U.data(), U.size() * sizeof(cd));
+  std::memcpy(up.data() + (rng_off - u_off), rng.data(), rng.size() * sizeof(uint64_t));
+  std::memcpy(up.data() + (sw_off - u_off), sw.data(), sw.size() * sizeof(SwizzlePart));
+  std::memcpy(up.data() + (key_off - u_off), keys.data(), keys.size() * sizeof(PartSwizzleKey));
+  if (int rc = ensure_scratch(scratch, end, stream, err)) {
+    if (rc != HSV_ERR_ALLOC) return rc;
+    (void)hipGetLastError();  // no room on the card: the host's way
+    err->clear();
+    return HSV_OK;
+  }
+  auto* dev = static_cast<unsigned char*>(scratch->ptr);
+  auto* nimg = static_cast<uint32_t*>(host);
+  auto* uerr = reinterpret_cast<double*>(static_cast<unsigned char*>(host) +
+                                         ((sw.size() * 14 * sizeof(uint32_t) + 7) & ~size_t(7)));
+  if (hipMemcpyAsync(dev + u_off, up.data(), up.size(), hipMemcpyHostToDevice, stream) != hipSuccess) {
+    *err = "fused upload failed";
+    return HSV_ERR_DEVICE;
+  }
+  hipLaunchKernelGGL(k_part_steps, (unsigned)ns, kStepThreads, 0, stream, reinterpret_cast<const double2*>(dev + u_off),
+                     pieces, reinterpret_cast<uint16_t*>(dev + tables), uerr);
+  hipLaunchKernelGGL(k_part_swizzle, (unsigned)sw.size(), kSwizzleThreads, 0, stream,
+                     reinterpret_cast<const SwizzlePart*>(dev + sw_off),
+                     reinterpret_cast<const PartSwizzleKey*>(dev + key_off),
+                     reinterpret_cast<const uint64_t*>(dev + rng_off), nimg);
+  if (hipGetLastError() != hipSuccess || hipStreamSynchronize(stream) != hipSuccess) {
+    *err = "the step check failed on the device";
+    return HSV_ERR_DEVICE;
+  }
+  size_t s0 = 0;
+  for (size_t w = 0; w < which.size(); ++w) {
+    FusedPart& P = parts[which[w]];
+    P.checked = true;
+    P.uerr.assign(uerr + s0, uerr + s0 + P.steps.size());
+    std::memcpy(P.nimg, nimg + w * 14, sizeof(P.nimg));
+    P.frag_off = tables + s0 * step_frag;
+    s0 += P.steps.size();
+  }
+  return HSV_OK;
 }
 
 int fused_plan_steps(hipStream_t stream, DeviceScratch* scratch, void* host, size_t host_bytes,
-                     const std::vector<std::vector<uint64_t>>& masks, int k, std::vector<std::vector<std::vector<int>>>* groups, std::string* err) {
+                     const std::vector<std::vector<uint64_t>>& masks, int k,
+                     std::vector<std::vector<std::vector<int>>>* groups, std::string* err) {
   groups->assign(masks.size(), {});
   struct Wanted {
     size_t part;

@@ -1543,14 +1543,22 @@ int hsv_apply_fused_chain(hsv_state* s, const hsv_gate* gates, int num_gates, co
   // skip the tiles with a 1 in its slot (the first parts run on a small corner
   // of the state)
   const uint64_t all_q = (n == 64) ? ~0ull : ((1ull << n) - 1);
-  // The parts' step groups. Below kPlanBytes of state a pass is shorter than
-  // the host's search for the next part's (2 to 3 ms): all of them are then
-  // searched on the device at once, before the first pass. (Not in the
-  // no-allocation form, which has no pinned memory to exchange them through;
-  // the groups are the same.)
-  constexpr uint64_t kPlanBytes = 8ull << 30;
+  // The parts' step groups and matrices. On the host the search takes 2 to 5 ms
+  // a part and the checks 0.3 to 0.9; both are done on the device instead: the
+  // groups of all parts before the first pass, the rest for kAhead parts at a
+  // time. The first parts run on a small corner of the state whatever its
+  // size, so this pays for all (QFT, 3 BF16 pieces: 16 qubits 1.4 ms where the
+  // groups alone left 3.0, 27 qubits 13.9 -> 11.6 ms; layered circuit, 2
+  // pieces, 16 GiB: 105.8 -> 104.7). Later, above kAheadBytes of state, the
+  // host prepares a part while the pass before it runs (1 ms at 4 GiB), and no
+  // stop for the device's answers is made. (Not in the no-allocation form,
+  // which has no pinned memory to exchange them through; groups and tables are
+  // the same.)
+  constexpr uint64_t kAheadBytes = 4ull << 30;
+  constexpr int kAhead = 16;
+  const bool ahead = !s->fused_scratch.fixed, small_state = s->len * s->elem() <= kAheadBytes;
   std::vector<std::vector<std::vector<int>>> groups(num_parts);
-  if (s->len * s->elem() <= kPlanBytes && !s->fused_scratch.fixed) {
+  if (ahead) {
     if (int rc = ensure_host_partial(s)) return rc;
     std::vector<std::vector<uint64_t>> masks(num_parts);
     size_t g0 = 0;
@@ -1562,9 +1570,20 @@ int hsv_apply_fused_chain(hsv_state* s, const hsv_gate* gates, int num_gates, co
         if (m) masks[p].push_back(m);
       }
     std::string err;
-    if (int rc = fused_plan_steps(s->stream, &s->fused_scratch, s->host_partial, sizeof(double) * 2 * kSumBlocks, masks, 5, &groups, &err))
+    if (int rc = fused_plan_steps(s->stream, &s->fused_scratch, s->host_partial, sizeof(double) * 2 * kSumBlocks,
+                                  masks, 5, &groups, &err))
       return fail(rc, err);
   }
+  std::vector<FusedPart> plans(kAhead);
+  std::vector<std::string> plan_err(kAhead);
+  std::vector<int> plan_rc(kAhead, HSV_OK);
+  size_t prepared = 0;  // gates
+  auto prepare = [&](int p) {
+    const std::vector<Lowered> part(Ls.begin() + prepared, Ls.begin() + prepared + part_sizes[p]);
+    prepared += part_sizes[p];
+    plan_rc[p % kAhead] = fused_part_prepare(n, part, tile[p], layout[p].data(), layout[p + 1].data(), pieces,
+                                             &groups[p], &plans[p % kAhead], &plan_err[p % kAhead]);
+  };
   uint64_t support = s->support & all_q;
   s->support = ~0ull;  // until the state is back in the standard layout
   off = 0;
@@ -1574,10 +1593,22 @@ int hsv_apply_fused_chain(hsv_state* s, const hsv_gate* gates, int num_gates, co
     uint64_t live = 0;
     for (int q = 0; q < n; ++q)
       if (support >> q & 1) live |= 1ull << layout[p][q];
-    if (int rc = begin_timed(s)) return rc;
     std::string err;
-    if (int rc = fused_part_bf_layout(s->amp, n, s->dtype, s->stream, &s->fused_scratch, part, tile[p],
-                                      layout[p].data(), layout[p + 1].data(), live, s->bf, &err, pieces, &groups[p])) {
+    int prc = HSV_OK;
+    if (!ahead || (p >= kAhead && !small_state)) {
+      prepare(p);
+    } else if (p % kAhead == 0) {
+      const int count = std::min(kAhead, num_parts - p);
+      for (int i = 0; i < count; ++i) prepare(p + i);
+      prc = fused_parts_check(s->stream, &s->fused_scratch, s->host_partial, sizeof(double) * 2 * kSumBlocks,
+                              plans.data(), count, pieces, &err);
+    }
+    if (int rc = begin_timed(s)) return rc;
+    if (!prc && (prc = plan_rc[p % kAhead])) err = plan_err[p % kAhead];
+    if (!prc)
+      prc = fused_part_launch(s->amp, n, s->dtype, s->stream, &s->fused_scratch, plans[p % kAhead], live, s->bf, pieces,
+                              &err);
+    if (const int rc = prc) {
       // close this part's timing pair, then bring the parts applied so far
       // back to the standard layout; a failed restore is reported too
       std::string msg = "part " + std::to_string(p) + ": " + err;

@@ -421,3 +421,36 @@ def test_device_step_groups_equal_the_hosts(circuit, n, k, reps):
                 continue
             s.apply_fused_chain(parts, lows, "bf16split")
             assert np.array_equal(s.read(), r.read())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["bf16split", "bf16x3"])
+@pytest.mark.parametrize("count,bad", [(1, None), (16, None), (17, None), (33, None), (33, 0), (33, 20)])
+def test_chain_parts_checked_ahead_equal_the_hosts(mode, count, bad):
+    """Parts prepared several at a time on the device against the no-allocation
+    form, whose parts are prepared one by one on the host: the same bits, also
+    of what ran before a part with a matrix that is not unitary."""
+    from hisvsim_amd import capi
+    from hisvsim_amd.circuit import Gate
+    n, rng = 16, np.random.default_rng(count)
+    parts, lows = [], [list(range(5))]
+    for p in range(count):
+        qs = sorted(set(lows[p]) | set(int(q) for q in rng.permutation(n)[:6]))
+        part = _some_gates(rng, qs, 12) + [Gate("H", (q,), (), ()) for q in qs]
+        if p == bad:
+            part.append(Gate("C2", (qs[0], qs[1]), (), tuple(complex(x) for x in rng.standard_normal(16))))
+        parts.append(part)
+        lows.append(sorted(int(q) for q in rng.permutation(qs)[:5]))
+    a = _stored(n, "complex128", 2)
+    with capi.State(n) as s, capi.State(n) as r:
+        codes = []
+        for x, noalloc in ((s, False), (r, True)):
+            x.write(a)
+            try:
+                x.apply_fused_chain(parts, lows[:count], mode, noalloc=noalloc)
+                codes.append(0)
+            except capi.HsvError as e:
+                codes.append((e.code, str(e).split(" (max")[0]))
+        assert codes[0] == codes[1]
+        assert codes[0] == 0 if bad is None else codes[0][0] == -6
+        assert np.array_equal(s.read(), r.read())
