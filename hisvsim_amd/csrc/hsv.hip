@@ -1160,7 +1160,7 @@ static int permute_in_place(hsv_state* s, const int* new_slot, bool renorm = fal
                          norm_out, scale);
     HIPCHK(hipGetLastError());
     if (norm_out) {
-      hipLaunchKernelGGL(k_norm_scale, 1, 64, 0, s->stream, s->partial, grid, s->partial + 2 * kRedBlocks - 2);
+      hipLaunchKernelGGL(k_norm_scale, 1, 256, 0, s->stream, s->partial, grid, s->partial + 2 * kRedBlocks - 2);
       HIPCHK(hipGetLastError());
     }
   }

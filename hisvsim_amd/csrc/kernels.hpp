@@ -838,12 +838,33 @@ __global__ __launch_bounds__(kSwapThreads) void k_swap_tiles(typename VecT<R>::t
 }
 
 // sum of the partials (in order) and the renormalisation factor: out[0] =
-// norm^2, out[1] = 1 / norm (1 for a zero state, which stays unchanged)
-static __global__ __launch_bounds__(64) void k_norm_scale(const double* __restrict__ partials, int count,
-                                                         double* __restrict__ out) {
+// norm^2, out[1] = 1 / norm (1 for a zero state, which stays unchanged). Bound
+// by the serial sum; the partials come through LDS, loaded by all lanes at
+// once (15 us for 2048 of them, 110 when the adding lane waits for each
+// load).
+static __global__ __launch_bounds__(256) void k_norm_scale(const double* __restrict__ partials, int count,
+                                                          double* __restrict__ out) {
+  constexpr int kChunk = 2048;
+  __shared__ double part[kChunk];
+  double t = 0.0;
+  for (int c0 = 0; c0 < count; c0 += kChunk) {
+    const int cnt = count - c0 < kChunk ? count - c0 : kChunk;
+    for (int i = threadIdx.x; i < cnt; i += 256) part[i] = partials[c0 + i];
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      int i = 0;
+      for (; i + 32 <= cnt; i += 32) {
+        double v[32];
+#pragma unroll
+        for (int j = 0; j < 32; ++j) v[j] = part[i + j];
+#pragma unroll
+        for (int j = 0; j < 32; ++j) t += v[j];
+      }
+      for (; i < cnt; ++i) t += part[i];
+    }
+    __syncthreads();
+  }
   if (threadIdx.x == 0) {
-    double t = 0.0;
-    for (int i = 0; i < count; ++i) t += partials[i];
     out[0] = t;
     out[1] = t > 0.0 ? 1.0 / sqrt(t) : 1.0;
   }
