@@ -1310,7 +1310,7 @@ int hsv_dtype(const hsv_state* s) { return s ? s->dtype : HSV_ERR_ARG; }
 
 int hsv_reset(hsv_state* s) {
   if (!s) return fail(HSV_ERR_ARG, "null handle");
-  const int grid = grid_for(s->len, 256, 1u << 16);
+  const int grid = grid_for(s->len * s->elem(), kZeroRun, 1u << 20);
   if (s->dtype == HSV_C128)
     hipLaunchKernelGGL((k_zero_state<double>), grid, 256, 0, s->stream, amp_as<double>(s), s->len);
   else

