@@ -112,6 +112,18 @@ def exchange_permutation(n: int, m: int = 3):
     return new_slot
 
 
+def full_passes(parts, n: int):
+    """Which passes of a path in the standard layout run over the whole state:
+    from |0...0> every path skips what an untouched qubit outside the part's
+    own keeps zero, so a pass counts as full when the part's qubits and those
+    touched before it are all of the state's."""
+    touched, full = set(), []
+    for part in parts:
+        touched |= {x for g in part for x in g.qubits()}
+        full.append(len(touched) == n)
+    return full
+
+
 def chain_full_passes(parts, lows, n: int):
     """Which chain passes run over the whole state. Starting from |0...0>,
     hsv_apply_fused_chain skips the tiles with a 1 in a slot whose qubit no
@@ -379,12 +391,16 @@ def main() -> int:
             partial = {"passes": int(len(full) - sum(full)),
                        "ms": float(launches[:, [i for i, f in enumerate(full) if not f]].sum(axis=1).mean())}
             launches = launches[:, [i for i, f in enumerate(full) if f]]
-        kern_ms = float(launches.mean())
-        if args.mode == "pergate":
+        elif args.mode == "pergate":
             # the dominant kernel is the dense U3 sweep over the whole state;
             # CZ sweeps move a quarter of it and would skew a per-launch mean
-            dense = np.array([g.name == "U3" for g in gates])
-            kern_ms = float(launches[:, dense].mean())
+            full = full_passes([[g] for g in gates], n)
+            launches = launches[:, [i for i, g in enumerate(gates) if g.name == "U3" and full[i]]]
+        elif args.mode != "permute" and per_step == len(parts):
+            full = full_passes(parts, n)
+            if any(full):
+                launches = launches[:, [i for i, f in enumerate(full) if f]]
+        kern_ms = float(launches.mean())
         passes = per_step
         log(f"[bench] TTS {tts:.3f} s, {passes} passes/step, mean full pass {kern_ms:.3f} ms"
             + (f", {partial['passes']} partial passes from |0...0> in {partial['ms']:.1f} ms" if partial else ""))
@@ -407,10 +423,11 @@ def main() -> int:
 
         per_gate = None
         if args.mode != "permute" and args.pergate_layers > 0:
-            # per-gate sample: first layers of the same circuit
+            # per-gate sample: first layers of the same circuit, on the state
+            # the timed path left (from |0...0> the sweeps would skip what is
+            # still zero)
             per_layer = n + n // 2
             sample = gates[: per_layer * args.pergate_layers]
-            s.reset()
             s.synchronize()
             s.set_timing(True)
             s.kernel_times()
@@ -481,8 +498,8 @@ def main() -> int:
         achieved = flops / (kern_ms * 1e-3)
         roof = {"bound": "mfma", "achieved": achieved / 1e12, "peak": peak / 1e12, "unit": "TFLOP/s",
                 "frac": achieved / peak, "traffic": measured_traffic("k_fused", n, args.mode, k),
-                "kernel": "k_fused",
-                "per_launch": f"8 x 2^k x 2^{n} algorithmic flops (k={kk}) / {kern_ms:.3f} ms",
+                "kernel": "k_fused_tile or k_fused",   # the first where its 4-qubit steps are faster
+                "per_launch": f"8 x 2^k x 2^{n} flops of the dense product (k={kk}) / {kern_ms:.3f} ms",
                 "hbm_gbs": 2 * S * 2 ** n / (kern_ms * 1e-3) / 1e9}
 
     verify = None if args.no_verify else verify_small(args.mode, k, depth, partitioner=args.partitioner,

@@ -171,15 +171,9 @@ class QAOABatch:
 
     def bytes_per_run(self, chunk_bits: int = 12) -> int:
         """HBM bytes of one run as the schedule moves them, 8 B per complex64
-        amplitude: the initial write, per layer one read and one write of
-        the state in stage A (the ZZ layer and RX on the chunk_bits low
-        qubits) and, for instances wider than that, one more in stage B (RX
-        on the high qubits), and the read of the cost reduction."""
-        tot = 0
-        for i in self.instances:
-            passes = 0.5 + i.p * (1 + (i.n > chunk_bits)) + 0.5
-            tot += int(passes * 2 * 8 * 2 ** i.n)
-        return tot
+        amplitude: one write of an instance that fits a chunk; of a wider one
+        the first pass' write and p passes that read and write it."""
+        return sum(8 * 2 ** i.n * (1 + 2 * i.p * (i.n > chunk_bits)) for i in self.instances)
 
     def gate_updates_per_run(self) -> int:
         """Gate-amplitude updates of one run: every gate (H layer, ZZ per edge,
@@ -280,8 +274,8 @@ def main(argv=None) -> int:
                "amplitudes": b.total_amplitudes(),
                "roofline": {"bound": "hbm", "achieved": gbs, "peak": 8000.0, "unit": "GB/s", "frac": gbs / 8000.0,
                             "bytes_per_batch": nbytes,
-                            "per_batch": "state bytes x passes of the schedule (init write, stage A and B read + "
-                                         "write per layer, cost read), 8 B per complex64 amplitude"},
+                            "per_batch": "state bytes x passes of the schedule (a write, then a read and a write per "
+                                         "layer for instances wider than a chunk), 8 B per complex64 amplitude"},
                "gate_amp_updates_per_s": b.gate_updates_per_run() / (mean_ms * 1e-3),
                "p1_instances": sum(1 for x in insts if x.p == 1), "p1_max_abs_err": err,
                "tuning": tuning["best"] if tuning else (load_tuning() or {}).get("best"),
