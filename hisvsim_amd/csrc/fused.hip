@@ -1846,11 +1846,30 @@ int part_launch_bf(void* amp, int n, int dtype, hipStream_t stream, DeviceScratc
   return HSV_OK;
 }
 
+// host: pinned memory for the device's answers: the part is prepared on the
+// device, with the same steps and tables; null: on the host.
 int part_apply_bf(void* amp, int n, int dtype, hipStream_t stream, DeviceScratch* scratch,
                   const std::vector<Lowered>& gates, uint64_t tile_qubits, const int* phys, const int* phys_after,
-                  uint64_t live_slots, const BfTune& bf, std::string* err, int pieces) {
+                  uint64_t live_slots, const BfTune& bf, std::string* err, int pieces, void* host = nullptr,
+                  size_t host_bytes = 0) {
+  std::vector<std::vector<std::vector<int>>> groups(1);
+  if (host) {
+    std::vector<std::vector<uint64_t>> masks(1);
+    for (const Lowered& L : gates) {
+      if (L.kind == K_IDENT) continue;
+      uint64_t m = 0;
+      for (int i = 0; i < L.nt + L.nc; ++i) {
+        const int q = i < L.nt ? L.t[i] : L.c[i - L.nt];
+        m |= 1ull << (phys ? phys[q] : q);
+      }
+      masks[0].push_back(m);
+    }
+    if (int rc = fused_plan_steps(stream, scratch, host, host_bytes, masks, 5, &groups, err)) return rc;
+  }
   FusedPart P;
-  if (int rc = part_prepare_bf(n, gates, tile_qubits, phys, phys_after, pieces, nullptr, &P, err)) return rc;
+  if (int rc = part_prepare_bf(n, gates, tile_qubits, phys, phys_after, pieces, &groups[0], &P, err)) return rc;
+  if (host)
+    if (int rc = fused_parts_check(stream, scratch, host, host_bytes, &P, 1, pieces, err)) return rc;
   return part_launch_bf(amp, n, dtype, stream, scratch, P, live_slots, bf, pieces, err);
 }
 
@@ -2280,7 +2299,8 @@ int fused_plan_steps(hipStream_t stream, DeviceScratch* scratch, void* host, siz
 }
 
 int fused_apply(void* amp, int n, int dtype, hipStream_t stream, int num_cu, DeviceScratch* scratch,
-                const std::vector<Lowered>& gates, int mode, uint64_t live, std::string* err, const BfTune& bf) {
+                const std::vector<Lowered>& gates, int mode, uint64_t live, std::string* err, const BfTune& bf,
+                void* pinned, size_t pinned_bytes) {
   if (mode != HSV_FUSED_F64 && mode != HSV_FUSED_F32SPLIT && mode != HSV_FUSED_BF16SPLIT &&
       mode != HSV_FUSED_BF16X3) {
     *err = "unknown fused mode";
@@ -2295,7 +2315,8 @@ int fused_apply(void* amp, int n, int dtype, hipStream_t stream, int num_cu, Dev
       for (int i = 0; i < L.nt; ++i) pmask |= 1ull << L.t[i];
       for (int i = 0; i < L.nc; ++i) pmask |= 1ull << L.c[i];
     }
-    return part_apply_bf(amp, n, dtype, stream, scratch, gates, pmask, nullptr, nullptr, live, bf, err, 3);
+    return part_apply_bf(amp, n, dtype, stream, scratch, gates, pmask, nullptr, nullptr, live, bf, err, 3, pinned,
+                         pinned_bytes);
   }
   if (mode == HSV_FUSED_BF16SPLIT) {
     uint64_t pmask = 0;
@@ -2305,7 +2326,8 @@ int fused_apply(void* amp, int n, int dtype, hipStream_t stream, int num_cu, Dev
       for (int i = 0; i < L.nc; ++i) pmask |= 1ull << L.c[i];
     }
     if (__builtin_popcountll(pmask) > 7)
-      return part_apply_bf(amp, n, dtype, stream, scratch, gates, pmask, nullptr, nullptr, live, bf, err, 2);
+      return part_apply_bf(amp, n, dtype, stream, scratch, gates, pmask, nullptr, nullptr, live, bf, err, 2, pinned,
+                           pinned_bytes);
   }
   if (mode == HSV_FUSED_F64 || mode == HSV_FUSED_F32SPLIT) {
     // identities count towards a part's 7 qubits

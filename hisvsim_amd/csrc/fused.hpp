@@ -41,10 +41,12 @@ struct BfTune {
 // Applies the fused unitary of `gates` to the n-qubit state at `amp`
 // (dtype HSV_C128 or HSV_C64) on `stream`. mode: hsv_fused_mode.
 // `num_cu` sizes the persistent grids of the FP64 / FP32-split kernels.
-// live: as in fused_part_bf_layout. Returns 0 or a negative hsv_status.
+// live: as in fused_part_launch. pinned: host memory through which a wide BF16
+// part is prepared on the device, or null. Returns 0 or a negative
+// hsv_status.
 int fused_apply(void* amp, int n, int dtype, hipStream_t stream, int num_cu, DeviceScratch* scratch,
                 const std::vector<Lowered>& gates, int mode, uint64_t live, std::string* err,
-                const BfTune& bf = BfTune());
+                const BfTune& bf = BfTune(), void* pinned = nullptr, size_t pinned_bytes = 0);
 
 // One part on the BF16-split wide-part kernel (a 12- to 14-qubit tile that
 // holds slots 0-4), laid out for its launch.

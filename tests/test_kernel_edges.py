@@ -467,3 +467,34 @@ def test_reset_fills_every_amplitude(n, dtype):
         s.reset()
         a = s.read()
     assert a[0] == 1 and not a[1:].any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["bf16split", "bf16x3"])
+@pytest.mark.parametrize("n,k", [(13, 9), (16, 12), (24, 12)])
+def test_wide_parts_prepared_on_an_idle_stream(mode, n, k):
+    """A wide part prepared on the device (nothing queued before it) and on
+    the host (behind earlier work): the same bits; a matrix that is not unitary
+    is refused either way."""
+    from hisvsim_amd import capi
+    from hisvsim_amd.circuit import Gate
+    rng = np.random.default_rng(n)
+    parts = [_some_gates(rng, sorted({int(q) for q in rng.permutation(n)[:k - 3]} | {0, 1, 2}), 3 * k) for _ in range(3)]
+    bad = parts[0] + [Gate("C2", (0, 1), (), tuple(complex(x) for x in rng.standard_normal(16)))]
+    a = _stored(n, "complex128", 2)
+    with capi.State(n) as s, capi.State(n) as r:
+        s.write(a)
+        r.write(a)
+        for p in parts:
+            s.synchronize()
+            s.apply_fused(p, mode)
+        for _ in range(20):  # work to queue behind
+            r.apply_gate(Gate("X", (n - 1,)))
+        for p in parts:
+            r.apply_fused(p, mode)
+        assert np.array_equal(s.read(), r.read())
+        for _ in range(2):
+            with pytest.raises(capi.HsvError) as e:
+                s.apply_fused(bad, mode)
+            assert e.value.code == -6
+            s.apply_gate(Gate("X", (0,)))
