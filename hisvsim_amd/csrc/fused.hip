@@ -1874,7 +1874,8 @@ int part_apply_bf(void* amp, int n, int dtype, hipStream_t stream, DeviceScratch
 }
 
 // The FP64 path on tiles (k_fused_tile). *taken = false, and nothing done, when
-// the dense kernel is to run: a gate on more than 4 qubits, more steps than
+// the dense kernel is to run: a matrix that is not finite (a NaN spreads over
+// the product that it is part of), a gate on more than 4 qubits, more steps than
 // the dense product is worth (2^(K - 4) in FP64, which it has the same flops
 // as; half as many again against the FP32-split product, whose three FP32
 // products a flop take 1.5 times FP64's time), a state below a tile, or steps
@@ -1890,6 +1891,7 @@ int fused_apply_tile64(void* amp, int n, int dtype, hipStream_t stream, DeviceSc
   uint64_t pmask = 0;
   for (const Lowered& L : gates) {
     if (L.kind == K_IDENT) continue;
+    if (!finite_matrix(L)) return HSV_OK;
     uint64_t m = 0;
     for (int i = 0; i < L.nt; ++i) m |= 1ull << L.t[i];
     for (int i = 0; i < L.nc; ++i) m |= 1ull << L.c[i];

@@ -235,6 +235,12 @@ void dense_of(const Lowered& L, cd* m) {
   }
 }
 
+bool finite_matrix(const Lowered& L) {
+  for (const cd& x : L.m)
+    if (!std::isfinite(x.real()) || !std::isfinite(x.imag())) return false;
+  return true;
+}
+
 void build_fused(const std::vector<Lowered>& gates, const std::vector<int>& qubits,
                  std::vector<cd>* Uout) {
   const int k = (int)qubits.size();

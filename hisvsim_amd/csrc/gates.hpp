@@ -45,6 +45,9 @@ int lower(const hsv_gate& g, Lowered* out, std::string* err);
 // The dense matrix of a lowered gate (2x2 or 4x4, row-major).
 void dense_of(const Lowered& L, cd* m /* 16 */);
 
+// Whether every entry of the gate's matrix is finite.
+bool finite_matrix(const Lowered& L);
+
 // Builds the 2^k x 2^k unitary (row-major, FP64) of a sequence of lowered
 // gates acting on `qubits` (sorted ascending; local bit i <-> qubits[i]).
 void build_fused(const std::vector<Lowered>& gates, const std::vector<int>& qubits,

@@ -129,11 +129,21 @@ uint64_t gate_qubits(const Lowered& L) {
   return m;
 }
 // Adds a gate's qubits to the state's support; all of them for a matrix with
-// an entry that is not finite, whose products with zeros are not zero.
-void touch(hsv_state* s, const Lowered& L) {
+// an entry that is not finite, whose products with zeros are not zero: then
+// false, and the pass that applies it may skip nothing.
+bool touch(hsv_state* s, const Lowered& L) {
   s->support |= gate_qubits(L);
-  for (const cd& x : L.m)
-    if (!std::isfinite(x.real()) || !std::isfinite(x.imag())) s->support = ~0ull;
+  if (finite_matrix(L)) return true;
+  s->support = ~0ull;
+  return false;
+}
+// The same for a pass that applies all of Ls at once; returns the qubits whose
+// zeros it may rely on: the support before it (it has its own in its tile).
+uint64_t touch_all(hsv_state* s, const std::vector<Lowered>& Ls) {
+  uint64_t live = s->support;
+  for (const Lowered& L : Ls)
+    if (!touch(s, L)) live = ~0ull;
+  return live;
 }
 
 int check_gate_qubits(const hsv_state* s, const Lowered& L) {
@@ -1369,8 +1379,7 @@ int hsv_apply_part(hsv_state* s, const hsv_gate* gates, int num_gates, int opt_s
     for (int i = 0; i < L.nc; ++i) part |= 1ull << L.c[i];
   }
   if (opt_slots) part |= (s->n >= 4 ? 0xFull : ((1ull << s->n) - 1));  // execute.hpp:184-199
-  const uint64_t live = s->support;  // before this part: it has its own qubits in its tile
-  for (const Lowered& L : Ls) touch(s, L);
+  const uint64_t live = touch_all(s, Ls);
   // part_kernel 2: every part whose qubits and slots 0-4 fit a tile takes
   // the FP64 tile kernel (it pads the tile with the lowest free slots itself)
   const int kt = tile_part_bits(s);
@@ -1405,8 +1414,7 @@ int hsv_apply_fused(hsv_state* s, const hsv_gate* gates, int num_gates, int mode
   if (!s || (num_gates > 0 && !gates) || num_gates < 0) return fail(HSV_ERR_ARG, "bad arguments");
   std::vector<Lowered> Ls;
   if (int rc = lower_all(gates, num_gates, &Ls, s)) return rc;
-  const uint64_t live = s->support;
-  for (const Lowered& L : Ls) touch(s, L);
+  const uint64_t live = touch_all(s, Ls);
   // With nothing left to run on the stream, the device would wait while the
   // host prepares a wide BF16 part (1 to 5 ms): it prepares the part itself.
   // Otherwise the host does, while the pass before runs. First part of a
@@ -1609,6 +1617,8 @@ int hsv_apply_fused_chain(hsv_state* s, const hsv_gate* gates, int num_gates, co
   for (int p = 0; p < num_parts; ++p) {
     const std::vector<Lowered> part(Ls.begin() + off, Ls.begin() + off + part_sizes[p]);
     off += part_sizes[p];
+    for (const Lowered& L : part)
+      if (!finite_matrix(L)) support = all_q;  // as in touch()
     uint64_t live = 0;
     for (int q = 0; q < n; ++q)
       if (support >> q & 1) live |= 1ull << layout[p][q];

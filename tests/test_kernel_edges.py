@@ -498,3 +498,45 @@ def test_wide_parts_prepared_on_an_idle_stream(mode, n, k):
                 s.apply_fused(bad, mode)
             assert e.value.code == -6
             s.apply_gate(Gate("X", (0,)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("path", ["gates", "part", "reg", "lds", "f64", "f64dense", "f32split", "bf16split", "bf16col",
+                                  "bf16wide", "bf16x3", "chain", "chain3"])
+def test_matrices_that_are_not_finite_reach_the_whole_state(path):
+    """A gate with a NaN entry on a state whose other qubits are still |0>:
+    its products with those zeros are NaN, so the NaNs are where the same call
+    leaves them on a state that was written (nothing known to be zero); and so
+    after one more gate on an untouched qubit."""
+    from hisvsim_amd import capi
+    from hisvsim_amd.circuit import Gate
+    n, nan = 15, float("nan")
+    first = [Gate("H", (1,)), Gate("X", (6,), (1,))]
+    bad = [Gate("H", (2,)), Gate("C1", (5,), (), (1, 0, 0, nan)), Gate("RZZ", (2, 5), (), (0.3,)), Gate("H", (8,))]
+    if path == "f64dense":
+        bad.append(Gate("X", (0,), (1, 2, 3, 4)))
+    if path in ("bf16wide", "bf16x3", "chain", "chain3"):
+        bad += [Gate("H", (q,)) for q in (0, 1, 3, 4, 7, 9)]
+    with capi.State(n) as a, capi.State(n) as b:
+        for s in (a, b):
+            s.apply_gates(first)
+        b.write(b.read())
+        for s in (a, b):
+            s.tune("part_kernel", {"reg": 1, "lds": 0}.get(path, 2))
+            if path == "bf16col":
+                s.tune("fused_variant", 1)
+            if path == "gates":
+                s.apply_gates(bad)
+            elif path in ("part", "reg", "lds"):
+                s.apply_part(bad, 0)
+            elif path in ("chain", "chain3"):
+                s.apply_fused_chain([bad, [Gate("H", (10,))]], [list(range(5))] * 2,
+                                    "bf16x3" if path == "chain3" else "bf16split")
+            else:
+                s.apply_fused(bad, {"f64dense": "f64", "bf16col": "bf16split", "bf16wide": "bf16split"}.get(path, path))
+            s.apply_gate(Gate("H", (13,)))
+        x, y = a.read(), b.read()
+    assert np.isnan(y).any()
+    assert np.array_equal(np.isnan(x.real), np.isnan(y.real)) and np.array_equal(np.isnan(x.imag), np.isnan(y.imag))
+    ok = ~np.isnan(y.real) & ~np.isnan(y.imag)
+    assert np.abs(x[ok] - y[ok]).max(initial=0.0) <= 1e-12
