@@ -1809,10 +1809,11 @@ int hsv_expect_pauli(hsv_state* s, uint64_t x_mask, uint64_t z_mask, double* out
   if (int rc = s->dtype == HSV_C128 ? pauli_t<double>(s, x_mask, z_mask, &t) : pauli_t<float>(s, x_mask, z_mask, &t))
     return rc;
   // with X or Y: 2 t (ny even) or 2i t (ny odd), ny = number of Y factors,
-  // times i^ny: real, 2 t for ny = 0, 3 and -2 t for ny = 1, 2 (mod 4)
+  // times i^ny: real, 2 t for ny = 0, 3 and -2 t for ny = 1, 2 (mod 4); the
+  // imaginary part is 0, or NaN with t
   const int ny = __builtin_popcountll(x_mask & z_mask) & 3;
   out2[0] = !x_mask ? t : (ny == 0 || ny == 3) ? 2 * t : -2 * t;
-  out2[1] = 0.0;
+  out2[1] = t - t;
   return HSV_OK;
 }
 

@@ -205,7 +205,8 @@ int hsv_project(hsv_state* s, uint64_t qubit_mask, uint64_t values, double* p_ou
 /* <psi|P|psi> for the Pauli string P with X on the qubits of x_mask only, Z
  * on z_mask only and Y on both (bit q = qubit q), FP64 accumulation. The
  * reference has no expectation read-out; its tests measure instead. out2 =
- * (re, im); im is rounding noise for a Hermitian P. */
+ * (re, im); im is 0 (P is Hermitian), or NaN where the state has a NaN or an
+ * infinity. */
 int hsv_expect_pauli(hsv_state* s, uint64_t x_mask, uint64_t z_mask, double* out2);
 
 /* Host-only introspection (no device needed; not in the reference).

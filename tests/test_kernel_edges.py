@@ -540,3 +540,23 @@ def test_matrices_that_are_not_finite_reach_the_whole_state(path):
     assert np.array_equal(np.isnan(x.real), np.isnan(y.real)) and np.array_equal(np.isnan(x.imag), np.isnan(y.imag))
     ok = ~np.isnan(y.real) & ~np.isnan(y.imag)
     assert np.abs(x[ok] - y[ok]).max(initial=0.0) <= 1e-12
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_pauli_sums_that_are_not_finite_have_no_zero_part(value, dtype):
+    """<P> of a state with a NaN or an infinity: neither part is a number;
+    the imaginary part of a finite state's is 0."""
+    import ctypes
+    from hisvsim_amd import capi
+    n = 13
+    a = _stored(n, dtype, 3)
+    out = (ctypes.c_double * 2)()
+    with capi.State(n, dtype) as s:
+        for state, finite in ((a, True), (np.where(np.arange(2 ** n) == 1234, value, a), False)):
+            s.write(state)
+            for x, z in ((0, 3), (1, 0), (1, 1), (1 << (n - 1), 5), (6, 6)):
+                capi._check(capi.lib().hsv_expect_pauli(s.handle, x, z, out))
+                assert np.isfinite(out[0]) == finite
+                assert out[1] == 0 if finite else np.isnan(out[1])
