@@ -560,3 +560,26 @@ def test_pauli_sums_that_are_not_finite_have_no_zero_part(value, dtype):
                 capi._check(capi.lib().hsv_expect_pauli(s.handle, x, z, out))
                 assert np.isfinite(out[0]) == finite
                 assert out[1] == 0 if finite else np.isnan(out[1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,n", [("complex128", 21), ("complex64", 22)])
+def test_read_outs_keep_what_each_workgroup_adds(dtype, n):
+    """One amplitude with all but 1.8e-13 of the mass, the rest spread over the
+    workgroups in pieces below half an ulp of 1: a sum of the workgroups'
+    partials one after another drops them all. At most 2 roundings per level of
+    the sums (a thread's items, lanes, waves, workgroups: 32 levels) of 2^-53."""
+    from hisvsim_amd import capi
+    a = np.zeros(2 ** n, complex)
+    a[0] = 1.0
+    a[256:2 ** 19:256] = np.sqrt(0.9e-16)
+    a = a if dtype == "complex128" else a.astype(np.complex64).astype(complex)
+    p = np.abs(a) ** 2
+    rest = p[1:].sum()
+    tol = 32 * 2.0 ** -53
+    top = 1 << (n - 1)
+    with capi.State(n, dtype) as s:
+        s.write(a)
+        assert abs((s.norm2() - 1.0) - rest) <= tol
+        assert abs((s.probability(n - 1, 0) - 1.0) - rest) <= tol
+        assert abs((s.expectation((0, top)) - 1.0) - rest) <= tol
