@@ -78,8 +78,8 @@ def _module():
     global _native
     if _native is None:
         try:
-            from . import load_module
-            _native = load_module()
+            from . import own_module
+            _native = own_module() or False
         except ImportError:
             _native = False
     return _native

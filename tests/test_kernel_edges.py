@@ -1,6 +1,8 @@
 """Kernels and dispatch rules at the sizes where they can go wrong: tile edges,
 remainders, the smallest and the largest of a rule's range. Each against the
 restatements under oracle/ or plain numpy in 64 bits."""
+import os
+
 import numpy as np
 import pytest
 
@@ -583,3 +585,28 @@ def test_read_outs_keep_what_each_workgroup_adds(dtype, n):
         assert abs((s.norm2() - 1.0) - rest) <= tol
         assert abs((s.probability(n - 1, 0) - 1.0) - rest) <= tol
         assert abs((s.expectation((0, top)) - 1.0) - rest) <= tol
+
+
+def test_gate_records_leave_the_module_path_alone():
+    """Building gate records neither adds the package's folder to sys.path
+    (its module names would hide a program's own) nor takes another module of
+    the pybind module's name for it."""
+    import subprocess
+    import sys
+    code = """
+import sys, types
+path = list(sys.path)
+if {other}:
+    sys.modules["svsimulator_py_wrapper"] = types.ModuleType("svsimulator_py_wrapper")
+from hisvsim_amd import capi
+from hisvsim_amd.circuit import Gate
+arr = capi.gate_array([Gate("H", (3,))])
+assert bytes(arr[0]) == bytes(capi.to_hsv_gate(Gate("H", (3,))))
+assert sys.path == path, sys.path
+import hisvsim_amd
+if not {other}:
+    assert hisvsim_amd.load_module()._fill_gates
+"""
+    for other in (False, True):
+        subprocess.run([sys.executable, "-c", code.format(other=other)], check=True, timeout=300,
+                       cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
