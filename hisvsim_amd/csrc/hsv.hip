@@ -722,6 +722,18 @@ int ensure_host_partial(hsv_state* s) {
   return HSV_OK;
 }
 
+// Whether the stream runs out of work within `us` microseconds.
+bool drains_within(hsv_state* s, double us) {
+  const auto t0 = std::chrono::steady_clock::now();
+  for (;;) {
+    const hipError_t e = hipStreamQuery(s->stream);
+    if (e == hipSuccess) return true;
+    (void)hipGetLastError();  // work left is no failure
+    if (e != hipErrorNotReady) return false;
+    if (std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count() >= us) return false;
+  }
+}
+
 template <typename R, int MODE>
 int reduce_t(hsv_state* a, hsv_state* b, double* out0, double* out1) {
   if (int rc = ensure_host_partial(a)) return rc;
@@ -1430,10 +1442,7 @@ int hsv_apply_fused(hsv_state* s, const hsv_gate* gates, int num_gates, int mode
     uint64_t mask = 0;
     for (const Lowered& L : Ls) mask |= gate_qubits(L);
     if (__builtin_popcountll(mask) > 7) {
-      idle = hipStreamQuery(s->stream) == hipSuccess;
-      (void)hipGetLastError();  // work left is no failure
-      if (idle)
-        if (int rc = ensure_host_partial(s)) return rc;
+      idle = drains_within(s, 0.0) && !ensure_host_partial(s);
     }
   }
   if (int rc = begin_timed(s)) return rc;
@@ -1583,29 +1592,38 @@ int hsv_apply_fused_chain(hsv_state* s, const hsv_gate* gates, int num_gates, co
   // stop for the device's answers is made. (Not in the no-allocation form,
   // which has no pinned memory to exchange them through; groups and tables are
   // the same.)
+  // The device can only answer once it is through with what is queued before
+  // the chain, so that is waited for as long as a reset of the state takes
+  // (what a chain usually follows), and no longer than the host's own search
+  // would keep the caller; behind more work the host prepares every part while
+  // that runs, and the call returns before it is done (27 qubits complex64, 4
+  // parts behind 21 ms of sweeps: in 9.5 ms, 22 when it waits).
   constexpr uint64_t kAheadBytes = 4ull << 30;
   constexpr int kAhead = 16;
-  const bool ahead = !s->fused_scratch.fixed, small_state = s->len * s->elem() <= kAheadBytes;
+  const bool small_state = s->len * s->elem() <= kAheadBytes;
+  const double wait_us = std::min(2000.0 * num_parts, 500.0 + double(s->len * s->elem()) / 5e6);
+  bool ahead = num_parts > 0 && !s->fused_scratch.fixed;
+  std::vector<std::vector<uint64_t>> masks(ahead ? num_parts : 0);
+  size_t g0 = 0;
+  for (int p = 0; p < (int)masks.size(); g0 += part_sizes[p], ++p)
+    for (size_t g = g0; g < g0 + part_sizes[p]; ++g) {
+      uint64_t m = 0;
+      for (uint64_t q = gate_qubits(Ls[g]); q; q &= q - 1) m |= 1ull << layout[p][__builtin_ctzll(q)];
+      if (m) masks[p].push_back(m);
+    }
+  ahead = ahead && drains_within(s, wait_us) && !ensure_host_partial(s);
   std::vector<std::vector<std::vector<int>>> groups(num_parts);
   // a part's timed interval has its preparation in it, the first one's also the
   // search for all
   if (num_parts > 0)
     if (int rc = begin_timed(s)) return rc;
   if (ahead) {
-    if (int rc = ensure_host_partial(s)) return rc;
-    std::vector<std::vector<uint64_t>> masks(num_parts);
-    size_t g0 = 0;
-    for (int p = 0; p < num_parts; g0 += part_sizes[p], ++p)
-      for (size_t g = g0; g < g0 + part_sizes[p]; ++g) {
-        uint64_t m = 0;
-        for (int q = 0; q < n; ++q)
-          if (gate_qubits(Ls[g]) >> q & 1) m |= 1ull << layout[p][q];
-        if (m) masks[p].push_back(m);
-      }
     std::string err;
     if (int rc = fused_plan_steps(s->stream, &s->fused_scratch, s->host_partial, sizeof(double) * 2 * kSumBlocks,
-                                  masks, 5, &groups, &err))
+                                  masks, 5, &groups, &err)) {
+      (void)end_timed(s);
       return fail(rc, err);
+    }
   }
   std::vector<FusedPart> plans(kAhead);
   std::vector<std::string> plan_err(kAhead);

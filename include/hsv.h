@@ -136,7 +136,10 @@ int hsv_apply_fused(hsv_state* s, const hsv_gate* gates, int num_gates, int mode
  * found before any pass; a part that fails later (a gate on more than 5
  * qubits) leaves the parts before it applied, in the standard layout.
  * A qubit that no gate has touched since the state was |0...0> is |0>
- * everywhere, so the first passes skip the tiles with a 1 in such a qubit. */
+ * everywhere, so the first passes skip the tiles with a 1 in such a qubit.
+ * The parts' steps are searched on the device, and the call waits for that,
+ * when the handle has nothing queued, or not more than a reset takes; behind
+ * more work they are searched on the host while that runs. */
 int hsv_apply_fused_chain(hsv_state* s, const hsv_gate* gates, int num_gates, const int* part_sizes,
                           int num_parts, const int* lows, int mode);
 
