@@ -713,9 +713,14 @@ int launch_tile_part(hsv_state* s, const std::vector<Lowered>& Ls, uint64_t part
                                  : launch_tile_part_t<R, KT - 1, 256>(s, Ls, part_mask, live);
 }
 
+// The read-outs' pinned memory: a kernel's partials (or what a search on the
+// device is asked and answers), or the masses of kWalkHostLen amplitudes for the
+// measurement walk and, behind them, the first of those amplitudes.
+constexpr uint64_t kWalkHostLen = 1ull << 14;
+static_assert(2 * kSumBlocks <= kWalkHostLen, "pinned memory");
 int ensure_host_partial(hsv_state* s) {
   if (s->host_partial) return HSV_OK;
-  if (hipHostMalloc(reinterpret_cast<void**>(&s->host_partial), sizeof(double) * 2 * kSumBlocks, 0) != hipSuccess) {
+  if (hipHostMalloc(reinterpret_cast<void**>(&s->host_partial), sizeof(double) * (kWalkHostLen + 1), 0) != hipSuccess) {
     s->host_partial = nullptr;
     return fail(HSV_ERR_ALLOC, "cannot allocate reduction scratch");
   }
@@ -820,7 +825,9 @@ int pauli_t(hsv_state* s, uint64_t x, uint64_t z, double* out) {
 // The measurement walk: the reference's sequential walk over cumulative
 // probabilities (state_vector.hpp:946-972) inside the chunks the samples land
 // in, the other chunks passed by their mass. States of kWalkHostLen
-// amplitudes or less are read back whole and walked here; on wider ones the
+// amplitudes or less are fetched whole (their masses, by a kernel that writes
+// pinned memory: a copy to a vector took 20 us or 110, depending on where
+// the heap has it) and walked here; on wider ones the
 // chunks' serial sums and the samples' places come from the device (see
 // k_walk_sums), bit for bit the walk's, and only the sub-blocks that its
 // integers do not cover (the first one from cum = 0, a change of binade, an
@@ -832,7 +839,6 @@ int pauli_t(hsv_state* s, uint64_t x, uint64_t z, double* out) {
 // product state at 18 / 28 qubits 10 shots 0.21 -> 0.09 / 2.3 -> 1.2 ms, 1000
 // shots 3.2 -> 0.14 / 11.4 -> 1.2 ms.
 constexpr double kWalkDeviceUs = 60.0;
-constexpr uint64_t kWalkHostLen = 1ull << 14;
 
 struct Walk {
   hsv_state* s;
@@ -858,22 +864,39 @@ struct Walk {
     while (sp < samples() && u[sp] < cum + p) place(sp++, pos);
     cum += p;
   }
-  // the walk over `len` amplitudes from `base`, at `a`, fetched or read back
-  int serial(uint64_t base, uint64_t len, const double* a = nullptr) {
-    for (size_t f = 0; !a && f < fetched.size(); ++f) {
-      if (fetched[f] != base || len != fetch_len) continue;
-      for (uint64_t i = 0; i < len && sp < samples(); ++i) step(fetched_mass[f * len + i], base + i);
+  // the walk over `len` amplitudes from `base`, given their masses
+  void over(const double* mass, uint64_t base, uint64_t len) {
+    for (uint64_t i = 0; i < len && sp < samples(); ++i) step(mass[i], base + i);
+  }
+  // the same, fetched before, fetched now or (more than kWalkHostLen) read back
+  int serial(uint64_t base, uint64_t len) {
+    for (size_t f = 0; f < fetched.size(); ++f)
+      if (fetched[f] == base && len == fetch_len) {
+        over(fetched_mass + f * len, base, len);
+        return HSV_OK;
+      }
+    if (len <= kWalkHostLen) {
+      if (int rc = s->dtype == HSV_C128 ? masses<double>(base, len) : masses<float>(base, len)) return rc;
+      over(s->host_partial, base, len);
       return HSV_OK;
     }
-    if (!a) {
-      amps.resize(2 * len);
-      if (int rc = hsv_read(s, base, len, amps.data())) return rc;
-      a = amps.data();
-    }
+    amps.resize(2 * len);
+    if (int rc = hsv_read(s, base, len, amps.data())) return rc;
     for (uint64_t i = 0; i < len && sp < samples(); ++i) {
-      const double x = a[2 * i], y = a[2 * i + 1];
+      const double x = amps[2 * i], y = amps[2 * i + 1];
       step(x * x + y * y, base + i);
     }
+    return HSV_OK;
+  }
+  // |a|^2 of up to kWalkHostLen amplitudes, to host_partial
+  template <typename R>
+  int masses(uint64_t base, uint64_t len) {
+    auto* at = reinterpret_cast<uint64_t*>(s->host_partial + kWalkHostLen);
+    *at = base;
+    hipLaunchKernelGGL((k_walk_fetch<R>), (unsigned)((len + 255) / 256), 256, 0, s->stream, amp_as<R>(s), len, at,
+                       s->host_partial);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(s->stream));
     return HSV_OK;
   }
   // whether the walk's next `sum0` / `sum1` ulps (lower / upper binade of the
@@ -1063,11 +1086,10 @@ struct Walk {
     std::vector<double> mass(blocks);
     for (int b = 0; b < blocks; ++b) mass[b] = s->host_partial[2 * b];
     if (s->len > kWalkHostLen) return s->dtype == HSV_C128 ? device<double>(mass) : device<float>(mass);
-    std::vector<double> a(2 * s->len);
-    if (int rc = hsv_read(s, 0, s->len, a.data())) return rc;
+    if (int rc = s->dtype == HSV_C128 ? masses<double>(0, s->len) : masses<float>(0, s->len)) return rc;
     for (int b = 0; b < blocks && sp < samples(); ++b) {
       if (!(u[sp] < cum + mass[b])) { cum += mass[b]; continue; }
-      if (int rc = serial(uint64_t(b) * chunk, chunk, a.data() + 2 * uint64_t(b) * chunk)) return rc;
+      over(s->host_partial + uint64_t(b) * chunk, uint64_t(b) * chunk, chunk);
     }
     return HSV_OK;
   }

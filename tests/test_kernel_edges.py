@@ -641,3 +641,25 @@ def test_chain_behind_queued_work_does_not_wait_for_it():
             if x is s:
                 assert called < 0.5 * total, (called, total)
         assert s.max_abs_diff(r) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+@pytest.mark.parametrize("n", [1, 2, 8, 9, 11, 13, 14, 15, 24, 25])
+def test_few_shots_walk_the_serial_sum(n, dtype):
+    """One shot and three, walked on the host: in the state fetched whole (up to
+    14 qubits), in a chunk fetched (up to 24) or found on the device: the
+    outcomes of the reference's walk, which passes the other chunks by their
+    masses (a uniform in the middle of an amplitude's share, so that the
+    masses' own rounding does not matter)."""
+    from hisvsim_amd import capi
+    a = _stored(n, dtype, n)
+    p = a.real * a.real + a.imag * a.imag
+    cum = np.cumsum(p)
+    rng = np.random.default_rng(n)
+    with capi.State(n, dtype) as s:
+        s.write(a)
+        for shots in (1, 3):
+            at = np.sort(rng.choice(np.flatnonzero(p > 0.3 * 2.0 ** -n), shots))
+            got = s.measure(list(range(n)), cum[at] - p[at] / 2) @ (1 << np.arange(n))
+            assert np.array_equal(got, at)
