@@ -831,7 +831,7 @@ int pauli_t(hsv_state* s, uint64_t x, uint64_t z, double* out) {
 // chunks' serial sums and the samples' places come from the device (see
 // k_walk_sums), bit for bit the walk's, and only the sub-blocks that its
 // integers do not cover (the first one from cum = 0, a change of binade, an
-// exact tie) are read back and walked here. A chunk read back and walked
+// exact tie) are fetched and walked here. A chunk fetched and walked
 // costs about 12 us and 2 ns an amplitude, the device's two launches and
 // waits about 60 us: kWalkDeviceUs is where they meet. Shots of the whole
 // register of a complex128 state, every walked chunk read back and walked
@@ -849,7 +849,6 @@ struct Walk {
   uint64_t chunk;                // amplitudes per chunk
   int sp = 0;                    // samples placed
   double cum = 0;
-  std::vector<double> amps = {};
   std::vector<uint64_t> fetched = {};   // sub-blocks of fetch_len amplitudes whose masses are at hand
   uint64_t fetch_len = 0;
   const double* fetched_mass = nullptr;
@@ -868,23 +867,17 @@ struct Walk {
   void over(const double* mass, uint64_t base, uint64_t len) {
     for (uint64_t i = 0; i < len && sp < samples(); ++i) step(mass[i], base + i);
   }
-  // the same, fetched before, fetched now or (more than kWalkHostLen) read back
+  // the same, fetched before or now, kWalkHostLen at a time
   int serial(uint64_t base, uint64_t len) {
     for (size_t f = 0; f < fetched.size(); ++f)
       if (fetched[f] == base && len == fetch_len) {
         over(fetched_mass + f * len, base, len);
         return HSV_OK;
       }
-    if (len <= kWalkHostLen) {
-      if (int rc = s->dtype == HSV_C128 ? masses<double>(base, len) : masses<float>(base, len)) return rc;
-      over(s->host_partial, base, len);
-      return HSV_OK;
-    }
-    amps.resize(2 * len);
-    if (int rc = hsv_read(s, base, len, amps.data())) return rc;
-    for (uint64_t i = 0; i < len && sp < samples(); ++i) {
-      const double x = amps[2 * i], y = amps[2 * i + 1];
-      step(x * x + y * y, base + i);
+    for (uint64_t i = 0; i < len && sp < samples(); i += kWalkHostLen) {
+      const uint64_t cnt = std::min(kWalkHostLen, len - i);
+      if (int rc = s->dtype == HSV_C128 ? masses<double>(base + i, cnt) : masses<float>(base + i, cnt)) return rc;
+      over(s->host_partial, base + i, cnt);
     }
     return HSV_OK;
   }
