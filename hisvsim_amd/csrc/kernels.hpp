@@ -379,13 +379,13 @@ __global__ __launch_bounds__(kRedBlock) void k_reduce(const typename VecT<R>::ty
 }
 
 // The one-state read-outs below go through the state in 16-byte units (one
-// complex128 or two complex64 amplitudes), four loads in flight per thread on
+// complex128 or two complex64 amplitudes), eight loads in flight per thread on
 // a grid that fills the chip (kSumBlocks workgroups, 8 per CU), and load only
 // what the result depends on. They are bound by HBM: a two-qubit
-// XX or YY term of a 28-qubit complex64 state (2.1 GB) takes 366 us (5.9
+// XX or YY term of a 28-qubit complex64 state (2.1 GB) takes 362 us (5.9
 // TB/s; with one thread per amplitude, every pair read twice, 610), a ZZ term
-// 398; P(0) of a 31-qubit complex128 state (17 GB of its 34) 3.7 ms against
-// 4.8 with the whole state's loop.
+// 358; P(0) of a 31-qubit complex128 state (17 GB of its 34) 2.8 ms, 5.0 with
+// the whole state's loop; its norm 5.6, with one amplitude per thread 5.8.
 constexpr int kSumBlocks = 2048;
 
 template <typename R>
@@ -410,23 +410,40 @@ __device__ __forceinline__ uint64_t insert_zero(uint64_t w, int pv) {
   return ((w ^ lo) << 1) | lo;
 }
 
-// f(w) summed over w < count, as partial[2 * block]. count and the grid are
-// powers of two, so with 4 * 256 * grid <= count every thread has the same
-// number of groups of four; smaller counts run on one block.
-template <typename F>
-__device__ __forceinline__ void sum_items(uint64_t count, double* __restrict__ partial, F f) {
-  const uint64_t stride = uint64_t(gridDim.x) * kRedBlock;
-  uint64_t w = uint64_t(blockIdx.x) * kRedBlock + threadIdx.x;
-  double s[4] = {0.0, 0.0, 0.0, 0.0};
-  if (count >= 4 * stride) {
-    for (; w < count; w += 4 * stride) {
+// f(w) summed over w < count, as partial[2 * block]. In large states a
+// workgroup takes groups of GROUP * 256 consecutive items (32 KB with eight
+// 16-byte loads a thread), so the chip reads a narrow front of the state: items
+// a whole grid apart, 8 MB, cost 9 to 13 % there (norm of a 28-qubit complex128
+// state 782 us, so 690; the highest qubit's P(0) 402 and 349). States that the
+// L2 holds keep the grid-wide steps, which other sweeps have too: what one
+// workgroup reads is then in its own XCD's L2 (renormalisation at 20 qubits 20
+// us, 25 with the near ones). count and the grid are powers of two, so with 4 *
+// 256 * grid <= count every thread has the same number of groups; smaller
+// counts run on one block.
+template <int GROUP, typename F>
+__device__ __forceinline__ double sum_groups(uint64_t count, uint64_t first, uint64_t step, F f) {
+  double s[GROUP] = {};
+  const uint64_t round = uint64_t(gridDim.x) * (GROUP * kRedBlock);
+  for (uint64_t w = first; w < count; w += round) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) s[j] += f(w + j * stride);
-    }
-  } else {
-    for (; w < count; w += stride) s[0] += f(w);
+    for (int j = 0; j < GROUP; ++j) s[j] += f(w + j * step);
   }
-  double t = (s[0] + s[1]) + (s[2] + s[3]);
+#pragma unroll
+  for (int h = GROUP / 2; h; h /= 2)
+#pragma unroll
+    for (int j = 0; j < h; ++j) s[j] += s[j + h];
+  return s[0];
+}
+template <int GROUP, typename F>
+__device__ __forceinline__ void sum_items(uint64_t count, double* __restrict__ partial, F f) {
+  const uint64_t grid = uint64_t(gridDim.x) * kRedBlock, far = uint64_t(blockIdx.x) * kRedBlock + threadIdx.x;
+  double t;
+  if (count >= 8 * grid)
+    t = sum_groups<GROUP>(count, uint64_t(blockIdx.x) * (GROUP * kRedBlock) + threadIdx.x, kRedBlock, f);
+  else if (count >= 4 * grid)
+    t = sum_groups<4>(count, far, grid, f);
+  else
+    t = sum_groups<1>(count, far, grid, f);
   for (int m = 32; m >= 1; m >>= 1) t += __shfl_xor(t, m);
   __shared__ double r[kRedBlock / 64];
   if ((threadIdx.x & 63) == 0) r[threadIdx.x >> 6] = t;
@@ -444,7 +461,7 @@ __global__ __launch_bounds__(kRedBlock) void k_mass0(const typename VecT<R>::typ
                                                      int qubit, double* __restrict__ partial) {
   const int pv = qubit - Unit<R>::LOG;  // the qubit's bit of the unit index
   const bool inside = Unit<R>::N == 2 && qubit == 0;
-  sum_items(count, partial, [&](uint64_t w) {
+  sum_items<8>(count, partial, [&](uint64_t w) {
     const Unit<R> x = load_unit<R>(a, insert_zero(w, qubit < 0 ? -1 : pv));
     double p = x.mass(0);
     if constexpr (Unit<R>::N == 2) p += inside ? 0.0 : x.mass(1);
@@ -463,7 +480,7 @@ __global__ __launch_bounds__(kRedBlock) void k_mass0(const typename VecT<R>::typ
 template <typename R>
 __global__ __launch_bounds__(kRedBlock) void k_pauli_z(const typename VecT<R>::type* __restrict__ a, uint64_t count,
                                                        uint64_t zmask, double* __restrict__ partial) {
-  sum_items(count, partial, [&](uint64_t u) {
+  sum_items<8>(count, partial, [&](uint64_t u) {
     const Unit<R> x = load_unit<R>(a, u);
     double p = x.mass(0);
     if constexpr (Unit<R>::N == 2) p += (zmask & 1) ? -x.mass(1) : x.mass(1);
@@ -483,7 +500,7 @@ __global__ __launch_bounds__(kRedBlock) void k_pauli_x(const typename VecT<R>::t
                                                        double* __restrict__ partial) {
   const uint64_t xu = xmask >> Unit<R>::LOG, zu = zmask >> Unit<R>::LOG;
   if (xu == 0) {  // x = 1 on complex64: both partners in one unit
-    sum_items(count, partial, [&](uint64_t u) {
+    sum_items<8>(count, partial, [&](uint64_t u) {
       const Unit<R> p = load_unit<R>(a, u);
       const double t = conj_part(p.a[Unit<R>::N - 1], p.a[0], imag);
       return (__popcll(u & zu) & 1) ? -t : t;
@@ -491,7 +508,7 @@ __global__ __launch_bounds__(kRedBlock) void k_pauli_x(const typename VecT<R>::t
     return;
   }
   const int pv = 63 - __clzll(xu);
-  sum_items(count, partial, [&](uint64_t w) {
+  sum_items<4>(count, partial, [&](uint64_t w) {
     const uint64_t u = insert_zero(w, pv);
     const Unit<R> p = load_unit<R>(a, u), q = load_unit<R>(a, u ^ xu);
     double t;

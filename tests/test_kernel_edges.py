@@ -663,3 +663,24 @@ def test_few_shots_walk_the_serial_sum(n, dtype):
             at = np.sort(rng.choice(np.flatnonzero(p > 0.3 * 2.0 ** -n), shots))
             got = s.measure(list(range(n)), cum[at] - p[at] / 2) @ (1 << np.arange(n))
             assert np.array_equal(got, at)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+@pytest.mark.parametrize("n", [21, 22, 23, 24])
+def test_read_outs_where_the_groups_grow(n, dtype):
+    """States around the sizes from which a thread sums eight items at a time
+    instead of four: norm, P(0) and strings with X on the lowest, a middle and
+    the highest qubit against numpy; 2^-53 per level of the sums, 40 of them,
+    and as much again in numpy's."""
+    from hisvsim_amd import capi
+    from oracle.oracle import pauli_expectation
+    a = _stored(n, dtype, n)
+    p = np.abs(a) ** 2
+    with capi.State(n, dtype) as s:
+        s.write(a)
+        assert abs(s.norm2() - p.sum()) <= 1e-14
+        for q in (0, 1, n // 2, n - 1):
+            assert abs(s.probability(q, 0) - p.reshape(-1, 2, 2 ** q)[:, 0].sum()) <= 1e-14
+        for x, z in ((0, 5), (1, 0), (1 << (n // 2), 3), (1 << (n - 1), 1 << (n - 1)), (3, 2 ** n - 1)):
+            assert abs(s.expectation((x, z)) - pauli_expectation(a, x, z).real) <= 1e-14, (x, z)
