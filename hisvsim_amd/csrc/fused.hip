@@ -1902,9 +1902,12 @@ int fused_apply_tile64(void* amp, int n, int dtype, hipStream_t stream, DeviceSc
   const int K = std::max(4, __builtin_popcountll(pmask));
   // one workgroup per tile: its 2^(n - 12) * 512 threads must fit 32 bits
   if (n < 12 || n > 34 || K > 7 || qm.empty()) return HSV_OK;
-  const std::vector<std::vector<int>> groups = step_groups(qm, 4, 16);
+  // the search ends where it exceeds what is worth it (120 gates on 7 qubits:
+  // 0.2 of the 4.9 ms that preparing the dense product takes, 0.3 to its end)
+  const int worth = std::min(kTileStepsMax, (split ? 3 : 2) << (K - 4) >> 1);
+  const std::vector<std::vector<int>> groups = step_groups(qm, 4, 16, worth);
   const int ns = (int)groups.size();
-  if (ns == 0 || ns > std::min(kTileStepsMax, (split ? 3 : 2) << (K - 4) >> 1)) return HSV_OK;
+  if (ns == 0) return HSV_OK;
   uint64_t tmask = pmask;
   for (int b = 0; b < n && __builtin_popcountll(tmask) < 12; ++b) tmask |= 1ull << b;
   int slot[12];

@@ -288,7 +288,7 @@ void build_fused(const std::vector<Lowered>& gates, const std::vector<int>& qubi
 double unitarity_error(const std::vector<cd>& U, int dim) {
   double worst = 0;
   for (int i = 0; i < dim; ++i)
-    for (int j = 0; j < dim; ++j) {
+    for (int j = i; j < dim; ++j) {  // U^H U is Hermitian, to the last bit
       cd s = 0.0;
       for (int r = 0; r < dim; ++r) s += std::conj(U[r * dim + i]) * U[r * dim + j];
       if (i == j) s -= 1.0;

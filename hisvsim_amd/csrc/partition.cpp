@@ -15,7 +15,7 @@
 #include "partition.hpp"
 
 namespace hsv {
-std::vector<std::vector<int>> step_groups(const std::vector<uint64_t>& qm, int k, int width);
+std::vector<std::vector<int>> step_groups(const std::vector<uint64_t>& qm, int k, int width, int max_groups);
 }
 
 namespace {
@@ -245,7 +245,7 @@ int chain_beam(const std::vector<uint64_t>& qm, int k, int low, int lookahead, i
 
 namespace hsv {
 
-std::vector<std::vector<int>> step_groups(const std::vector<uint64_t>& qm, int k, int width) {
+std::vector<std::vector<int>> step_groups(const std::vector<uint64_t>& qm, int k, int width, int max_groups) {
   const int ng = (int)qm.size();
   std::vector<std::vector<int>> out;
   if (ng == 0) return out;
@@ -338,6 +338,7 @@ std::vector<std::vector<int>> step_groups(const std::vector<uint64_t>& qm, int k
       if (!dup) next.push_back(std::move(c));
       if ((int)next.size() >= width) break;
     }
+    if (max_groups > 0 && (int)next[0].sets.size() >= max_groups) return {};  // gates are left
     beam.swap(next);
   }
 }
