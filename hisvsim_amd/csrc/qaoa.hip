@@ -11,8 +11,8 @@
 // instance of n <= L qubits runs whole in one chunk of LDS. A wider one takes
 // p + 1 passes over its state, each on chunks of up to 2^13 amplitudes:
 //  * even passes ("low"): contiguous chunks over the L low qubits;
-//  * odd passes ("high"): chunks over the n - L high qubits and as many of the
-//    lowest ones as fit.
+//  * odd passes ("high"): chunks over the n - L high qubits and some of the
+//    lowest ones.
 // D_l needs RX of layer l - 1 done on every qubit, but can be applied in any
 // chunk, and RX on different qubits commute. So pass k finishes layer k - 1 on
 // its own half of the qubits (the pass before did the other half), applies
@@ -60,12 +60,20 @@ int qfail(int code, const std::string& m) {
 constexpr int kMaxEdges = 64;
 constexpr int kMaxQaoaQubits = 26;
 // High chunks hold an instance's hb = n - L high qubits and its lowest
-// low_contig(hb, L) qubits (contiguous runs of 2^that amplitudes), kStageBBits
-// qubits in all where L leaves that many: at least kLowContig of them (64-byte
-// runs).
+// low_contig(hb, L, threads) qubits (contiguous runs of 2^that amplitudes): 16
+// amplitudes a thread, kStageBBits qubits in all at most, at least kLowContig
+// low ones (64-byte runs). Fewer threads take smaller chunks, not longer loops,
+// so that a small batch has more of them to run at once: 16 instances of 20
+// qubits in 256 threads 503 -> 337 us, 8 of 12 to 14 qubits 135 -> 116 (128
+// threads 211 -> 161); a batch that fills the chip, 512 of 12 to 22 qubits,
+// 14.8 -> 15.0 ms for the shorter runs.
 constexpr int kLowContig = 3;
 constexpr int kStageBBits = 13;
-inline int low_contig(int hb, int L) { return std::min(kStageBBits - hb, L); }
+inline int low_contig(int hb, int L, int threads) {
+  int bits = 4;
+  while ((1 << (bits - 4)) < threads) ++bits;
+  return std::min(std::max(std::min(kStageBBits, bits) - hb, kLowContig), L);
+}
 
 struct alignas(8) cf { float x, y; };
 
@@ -631,7 +639,7 @@ int build_graph(hsv_qaoa_batch* b) {
     Inst& I = b->inst[id];
     const bool whole = I.n <= L;
     const int hb = whole ? 0 : I.n - L;
-    I.lc = whole ? I.n : low_contig(hb, L);
+    I.lc = whole ? I.n : low_contig(hb, L, b->nt);
     I.bits[0] = std::min(I.n, L);
     I.bits[1] = whole ? I.n : I.lc + hb;
     I.part_off = (int)parts;
@@ -783,7 +791,7 @@ int hsv_qaoa_tune(hsv_qaoa_batch* b, const char* key, int value) {
   else if (k == "threads" && (value == 128 || value == 256 || value == 512)) b->nt = value;
   else if (k == "grid_per_cu" && value >= 1 && value <= 64) b->grid_per_cu = value;
   else return qfail(HSV_ERR_ARG, "unknown QAOA tuning key or value: " + k);
-  // stage B holds the high qubits plus the low ones; keep it within 64 KB of LDS
+  // a high chunk holds the high qubits and kLowContig low ones: within 64 KB of LDS
   int maxn = 0;
   for (const Inst& I : b->inst) maxn = std::max(maxn, I.n);
   if (kLowContig + maxn - b->L > kStageBBits) return qfail(HSV_ERR_LIMIT, "chunk_bits too small for the widest instance");

@@ -684,3 +684,23 @@ def test_read_outs_where_the_groups_grow(n, dtype):
             assert abs(s.probability(q, 0) - p.reshape(-1, 2, 2 ** q)[:, 0].sum()) <= 1e-14
         for x, z in ((0, 5), (1, 0), (1 << (n // 2), 3), (1 << (n - 1), 1 << (n - 1)), (3, 2 ** n - 1)):
             assert abs(s.expectation((x, z)) - pauli_expectation(a, x, z).real) <= 1e-14, (x, z)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(12, 128), (10, 128), (13, 256), (12, 256), (13, 512)])
+def test_qaoa_high_chunks_of_every_width(shape):
+    """High chunks from one high qubit to as many as leave the fewest low ones,
+    narrower than, as wide as and wider than 16 amplitudes a thread: one layer
+    against the closed form, at the bar of the batch's tests."""
+    from hisvsim_amd.qaoa import Instance, QAOABatch, expectation_p1, random_3regular
+    bits, threads = shape
+    rng = np.random.default_rng(bits + threads)
+    insts = [Instance(n, random_3regular(n, rng), [float(rng.uniform(0, np.pi))], [float(rng.uniform(0, np.pi))])
+             for n in range(bits, min(bits + 10, 22) + 1)]
+    with QAOABatch(insts) as b:
+        b.tune("chunk_bits", bits)
+        b.tune("threads", threads)
+        got = b.run()
+    for i, inst in enumerate(insts):
+        want = expectation_p1(inst.n, inst.edges, inst.gammas[0], inst.betas[0])
+        assert abs(got[i] - want) <= 1e-5 * max(1.0, abs(want)), inst.n
