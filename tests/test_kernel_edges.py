@@ -704,3 +704,52 @@ def test_qaoa_high_chunks_of_every_width(shape):
     for i, inst in enumerate(insts):
         want = expectation_p1(inst.n, inst.edges, inst.gammas[0], inst.betas[0])
         assert abs(got[i] - want) <= 1e-5 * max(1.0, abs(want)), inst.n
+
+
+def _busy_part(rng, qubits, steps):
+    """Random gates on the qubits, more than `steps` steps of 4 qubits."""
+    from hisvsim_amd import capi
+    gs = []
+    while len(capi.part_steps(gs, 4, 16)) <= steps if gs else True:
+        gs += _some_gates(rng, qubits, 6)
+    return gs
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+@pytest.mark.parametrize("n,k,why", [(8, 4, "small"), (9, 5, "small"), (10, 6, "small"), (11, 7, "small"),
+                                     (12, 5, "five"), (14, 6, "five"), (16, 7, "five"),
+                                     (13, 5, "steps"), (15, 6, "steps"), (17, 7, "steps")])
+def test_fused_f32split_dense_product(n, k, why, dtype):
+    """The FP32-split product where the FP64 steps do not take the part (a
+    state below a tile, a gate on five qubits, more steps than are worth it:
+    1.5 * 2^(k - 4), at most 8), from a written state and from |0...0> with a
+    few qubits touched, against the gates one by one. Each real product is
+    accumulated in FP32 over 3 * 2^k terms of at most the state's norm: error
+    below 1e-6, and on a complex128 state above 1e-12, where FP64 steps would
+    be."""
+    from hisvsim_amd import capi
+    from hisvsim_amd.circuit import Gate
+    rng = np.random.default_rng(100 * n + k)
+    limit = min(8, (3 << (k - 4)) >> 1)
+    with capi.State(n, dtype) as s, capi.State(n) as r:
+        for start in (None, _stored(n, dtype, n)):
+            for _ in range(3):
+                qubits = [int(q) for q in rng.permutation(n)[:k]]
+                if why == "steps":
+                    gs = _busy_part(rng, qubits, limit)
+                else:
+                    gs = [Gate("H", (q,)) for q in qubits] + _some_gates(rng, qubits, 6)
+                if why == "five":
+                    gs.append(Gate("RX", (qubits[0],), tuple(qubits[1:5]), (0.7,)))
+                for x in (s, r):
+                    x.reset()
+                    if start is not None:
+                        x.write(start)
+                    x.apply_gates([Gate("H", (1,)), Gate("RY", (n - 1,), (1,), (0.8,))])
+                s.apply_fused(gs, "f32split")
+                r.apply_gates(gs)
+                err = np.abs(s.read() - r.read()).max()
+                assert err <= 1e-6
+                if dtype == "complex128":
+                    assert err >= 1e-12
