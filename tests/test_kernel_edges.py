@@ -753,3 +753,62 @@ def test_fused_f32split_dense_product(n, k, why, dtype):
                 assert err <= 1e-6
                 if dtype == "complex128":
                     assert err >= 1e-12
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+@pytest.mark.parametrize("seed", range(10))
+def test_every_kernel_skips_only_what_is_zero(seed, dtype):
+    """Gates, parts on each kernel, fused parts of each precision as steps and
+    as one product, both forms of small BF16 parts, wide BF16 parts and chains
+    of several parts, one after another from |0...0>: the same numbers as on a
+    state that is written before each call, where nothing is known to be zero.
+    The tiles that are not skipped run the same arithmetic, but for the
+    three-piece split, whose column signs are hashed from a tile's number in
+    the launch: there to its bar, 1e-6 (and on from the same amplitudes)."""
+    from hisvsim_amd import capi
+    n, rng = 17, np.random.default_rng([seed, 5])
+    ops = ["gates", "part", "reg", "lds", "f64", "f32split", "f64dense", "f32dense", "bf16tile", "bf16col", "bf16rows",
+           "bf16wide", "bf16x3", "chain", "chain3", "permute", "reset"]
+    weight = np.array([2, 2, 1, 1, 2, 2, 2, 2, 2, 2, 2, 2, 2, 2, 2, 1, 1.5])
+    with capi.State(n, dtype) as a, capi.State(n, dtype) as b:
+        for _ in range(16):
+            b.write(b.read())        # forgets what b knows
+            op = str(rng.choice(ops, p=weight / weight.sum()))
+            wide = op in ("bf16wide", "bf16x3")
+            k = int(rng.integers(8, 12)) if wide else int(rng.integers(5, 8))
+            pick = [int(x) for x in rng.permutation(n)[:k]]
+            if wide:
+                pick = sorted(set(pick) | set(range(5)))[:12]
+            if op in ("gates", "part", "reg", "lds"):
+                pick = pick[:int(rng.integers(1, 6))]
+            if op in ("f64dense", "f32dense"):
+                gs = _busy_part(rng, pick, min(8, (3 << (k - 4)) >> 1))
+            elif op in ("chain", "chain3"):
+                gs = [g for _ in range(3) for g in _some_gates(rng, [int(x) for x in rng.permutation(n)[:6]], 5)]
+                parts, lows = capi.chain_parts(gs, 12, 5, 7)
+            else:
+                gs = _some_gates(rng, pick, int(rng.integers(1, 4)))
+            perm = [int(x) for x in rng.permutation(n)]
+            for s in (a, b):
+                s.tune("part_kernel", {"reg": 1, "lds": 0}.get(op, 2))
+                s.tune("fused_variant", {"bf16col": 1, "bf16rows": 0}.get(op, 2))
+                if op == "gates":
+                    s.apply_gates(gs)
+                elif op in ("part", "reg", "lds"):
+                    s.apply_part(gs, 0)
+                elif op in ("chain", "chain3"):
+                    s.apply_fused_chain(parts, lows, "bf16x3" if op == "chain3" else "bf16split")
+                elif op == "permute":
+                    s.permute_qubits(perm)
+                elif op == "reset":
+                    s.reset()
+                else:
+                    mode = {"f64dense": "f64", "f32dense": "f32split"}.get(op, op)
+                    s.apply_fused(gs, mode if mode in ("f64", "f32split", "bf16x3") else "bf16split")
+            x, y = a.read(), b.read()
+            if op in ("bf16x3", "chain3"):
+                assert np.abs(x - y).max() <= 1e-6, op
+                b.write(x)
+            else:
+                assert np.array_equal(x, y), op
