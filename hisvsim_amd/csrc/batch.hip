@@ -476,10 +476,10 @@ void build_tiles(hsv_batch* b, const std::vector<Lowered>& all, std::vector<BSeg
       A->rounds.push_back(Q);
     }
     A->ranges.push_back({(int)(&S - segs->data()), gb, (int)TP.gates.size()});
-    const std::vector<Lowered> fused = fuse_one_qubit_runs(Ls);
     for (size_t i = 0; i < TP.gates.size(); ++i) {
+      const RegGate& G = TP.gates[i];
       A->source.push_back(TP.source[i]);
-      A->sign.push_back(tile_sign_flip(fused[TP.source[i]]));
+      A->sign.push_back(G.kind == GK_PHASE1 && G.m[0] == -1.0 && G.m[1] == 0.0);  // tile_sign_flip
       A->gates.push_back(TP.gates[i]);
       A->m2idx.push_back(TP.m2idx[i] >= 0 ? TP.m2idx[i] + mb : -1);
     }
@@ -489,7 +489,7 @@ void build_tiles(hsv_batch* b, const std::vector<Lowered>& all, std::vector<BSeg
 
 // Writes the arrays into b->d_tile (allocated here when absent), the gate
 // records' matrix pointers into the same buffer.
-int upload_tiles(hsv_batch* b, const TileArrays& A) {
+int upload_tiles(hsv_batch* b, TileArrays&& A) {
   const size_t seg_off = 0;
   const size_t round_off = seg_off + A.segs.size() * sizeof(RegSeg);
   const size_t gate_off = round_off + A.rounds.size() * sizeof(TileRound);
@@ -513,12 +513,13 @@ int upload_tiles(hsv_batch* b, const TileArrays& A) {
     hg[i].m2 = A.m2idx[i] >= 0 ? reinterpret_cast<const double*>(dev + mat_off) + 32 * size_t(A.m2idx[i]) : nullptr;
   }
   if (!A.mat2.empty()) std::memcpy(host.data() + mat_off, A.mat2.data(), A.mat2.size() * sizeof(double));
-  b->tile_gates.assign(hg, hg + A.gates.size());
-  b->tile_m2idx = A.m2idx;
-  b->tile_source = A.source;
-  b->tile_mat2 = A.mat2;
-  b->tile_sign = A.sign;
-  b->tile_ranges = A.ranges;
+  std::copy(hg, hg + A.gates.size(), A.gates.begin());  // with their pointers
+  b->tile_gates = std::move(A.gates);
+  b->tile_m2idx = std::move(A.m2idx);
+  b->tile_source = std::move(A.source);
+  b->tile_mat2 = std::move(A.mat2);
+  b->tile_sign = std::move(A.sign);
+  b->tile_ranges = std::move(A.ranges);
   BCHK(hipMemcpyAsync(b->d_tile, host.data(), bytes, hipMemcpyHostToDevice, b->stream));
   BCHK(hipStreamSynchronize(b->stream));
   return HSV_OK;
@@ -626,7 +627,7 @@ int build(hsv_batch* b) {
     }
     TileArrays A;
     build_tiles(b, all, &b->segs, &A);
-    if (int rc = upload_tiles(b, A)) return rc;
+    if (int rc = upload_tiles(b, std::move(A))) return rc;
     int first = 0;
     for (BSeg& S : b->segs) {
       S.part_first = first;
