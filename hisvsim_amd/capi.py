@@ -266,6 +266,18 @@ def part_steps(gates: Sequence, k: int = 5, width: int = 16):
     return steps
 
 
+def fused_steps(gates: Sequence, n: int, split: bool = False) -> int | None:
+    """The 4-qubit FP64 steps hsv_apply_fused runs a part as (split: mode
+    "f32split"), None where it takes one dense product: the library's rule, on
+    the gates' qubits (host only)."""
+    gates = [g for g in gates if g.name.upper() != "I"]
+    if not gates or not 12 <= n <= 34 or any(len(set(g.qubits())) > 4 for g in gates):
+        return None
+    k = max(4, len({q for g in gates for q in g.qubits()}))
+    steps = len(part_steps(gates, 4)) if k <= 7 else 99
+    return steps if steps <= min(8, (3 if split else 2) << (k - 4) >> 1) else None
+
+
 def fused_unitary(n: int, gates: Sequence):
     """(qubits, U, unitarity_error) of the fused part (host only)."""
     arr = gate_array(gates)

@@ -15,8 +15,9 @@ qubits):
   1-qubit and multi-qubit gate counts, the multi-qubit fraction, min / max /
   spread of the qubit indices, whether it touches the top 3 (high-order)
   qubits, two mode flags, n, and the number of fused blocks the pass
-  applies (0 for the register kernel, 1 for a 5..7-qubit unitary, the
-  5-qubit steps of a wide part).
+  applies (0 for the register kernel, 1 for a BF16-split unitary of 5..7
+  qubits, the 4-qubit steps of an FP64 part or as many as its dense product
+  has the flops of, the 5-qubit steps of a wide part).
 Target: log(ms per pass scaled to a 2^30-amplitude state), so one model
 covers every n (a pass is memory-bound work proportional to 2^n). A chain
 plan adds its layout restore, priced per 2^30 amplitudes by the median of
@@ -57,8 +58,11 @@ def part_features(part: Sequence[Gate], n: int, mode: str, low: Sequence[int] = 
         # the wide-part kernel's tile: 12 or 13 qubits holding slots 0-4
         width = 12 if len(set(qs) | (low5 if mode != "chain" else set())) <= 12 else 13
         blocks = len(capi.part_steps(part)) if part else 0   # the kernel's fused steps
+    elif mode == "fused64":
+        width = max(4, k)
+        blocks = capi.fused_steps(part, n) or 2 ** (width - 4)
     else:
-        width, blocks = max(4 if mode == "fused64" else 5, k), 1
+        width, blocks = max(5, k), 1
     n1 = sum(1 for g in part if len(g.qubits()) == 1)
     n2 = len(part) - n1
     return np.array([

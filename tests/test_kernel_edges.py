@@ -812,3 +812,29 @@ def test_every_kernel_skips_only_what_is_zero(seed, dtype):
                 b.write(x)
             else:
                 assert np.array_equal(x, y), op
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [11, 12, 16])
+def test_fused_steps_says_which_arithmetic_runs(n):
+    """capi.fused_steps, which the benchmark and the cost model price fused
+    parts by, against what ran: an FP32-split part leaves an error of FP32's
+    size exactly where the rule says that it is one dense product."""
+    from hisvsim_amd import capi
+    from hisvsim_amd.circuit import Gate
+    rng = np.random.default_rng(n)
+    a = _stored(n, "complex128", 3)
+    seen = set()
+    with capi.State(n) as s, capi.State(n) as r:
+        for k in (2, 4, 5, 6, 7):
+            for count in (1, 3, 8, 20):
+                qubits = [int(q) for q in rng.permutation(n)[:k]]
+                gs = _some_gates(rng, qubits, count) + [Gate("H", (q,)) for q in qubits] + [Gate("I", (qubits[0],))]
+                for x in (s, r):
+                    x.write(a)
+                s.apply_fused(gs, "f32split")
+                r.apply_gates(gs)
+                dense = capi.fused_steps(gs, n, True) is None
+                seen.add(dense)
+                assert (np.abs(s.read() - r.read()).max() >= 1e-12) == dense, (k, count)
+    assert seen == ({True} if n < 12 else {True, False})
