@@ -24,9 +24,10 @@ ARCH = os.environ.get("HSV_OFFLOAD_ARCH", "gfx950")
 # -packed-fp32-ops keeps the compiler from emitting packed FP32 VALU ops.
 HIP_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Wall", "-Wno-unused-function", "-Wno-unused-value",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-I", os.path.join(ROOT, "include")]
-# The chain planner's inner loops run 10 to 15 % slower where they straddle a
+# The chain planner's inner loops run 5 to 15 % slower where they straddle a
 # 32-byte line, which otherwise depends on the size of the code linked before
-# them (n = 30, 540 gates, one core: 2.7 s aligned, 3.2 s not).
+# them (n = 30, 540 gates, one core: 2.7 to 2.9 s aligned, 3.0 to 3.2 s not,
+# where an earlier library happened to have them aligned).
 CXX_FLAGS = ["-O3", "-falign-functions=64", "-falign-loops=32", "-falign-jumps=32", "-std=c++17", "-fPIC",
              "-pthread", "-Wall", "-I", os.path.join(ROOT, "include")]
 
