@@ -492,15 +492,37 @@ def main() -> int:
             products = 6 if args.mode == "fusedbf16x3" else 3
             roof["mfma_frac_executed"] = products * per_pass / (kern_ms * 1e-3) / BF16_MFMA_PEAK
     else:
-        kk = max(4, min(7, k))
-        flops = 8 * 2 ** kk * 2 ** n
-        peak = FP64_MFMA_PEAK if args.mode == "fused64" else FP32_MFMA_PEAK
-        achieved = flops / (kern_ms * 1e-3)
-        roof = {"bound": "mfma", "achieved": achieved / 1e12, "peak": peak / 1e12, "unit": "TFLOP/s",
-                "frac": achieved / peak, "traffic": measured_traffic("k_fused", n, args.mode, k),
-                "kernel": "k_fused_tile or k_fused",   # the first where its 4-qubit steps are faster
-                "per_launch": f"8 x 2^k x 2^{n} flops of the dense product (k={kk}) / {kern_ms:.3f} ms",
-                "hbm_gbs": 2 * S * 2 ** n / (kern_ms * 1e-3) / 1e9}
+        # parts of up to 7 qubits: 4-qubit FP64 steps on a tile (128 flops per
+        # amplitude and step) where the library takes them, else one dense
+        # product of 8 x 2^k flops at the mode's own rate
+        split = args.mode == "fused32"
+        timed = parts
+        if per_step == len(parts):
+            full = full_passes(parts, n)
+            timed = [p for p, f in zip(parts, full) if f] or parts   # the passes kern_ms averages
+        steps = [capi.fused_steps(p, n, split) for p in timed]
+        dense_peak = FP32_MFMA_PEAK if split else FP64_MFMA_PEAK
+        widths = [max(4, len({q for g in p for q in g.qubits()})) for p in timed]
+        at_peak = [128 * s * 2 ** n / FP64_MFMA_PEAK if s else 8 * 2 ** w * 2 ** n / dense_peak
+                   for s, w in zip(steps, widths)]
+        mfma = float(np.mean(at_peak)) / (kern_ms * 1e-3)
+        tiles = [s for s in steps if s]
+        flops = float(np.mean([128 * s if s else 8 * 2 ** w for s, w in zip(steps, widths)])) * 2 ** n
+        hbm_gbs = 2 * S * 2 ** n / (kern_ms * 1e-3) / 1e9
+        hbm = hbm_gbs / HBM_PEAK_GBS
+        kernel = "k_fused_tile" if len(tiles) == len(steps) else "k_fused_tile and k_fused" if tiles else "k_fused"
+        roof = {"bound": "hbm" if hbm >= mfma else "mfma", "kernel": kernel,
+                "traffic": measured_traffic(kernel.split()[0], n, args.mode, k),
+                "parts_as_steps": len(tiles), "parts_dense": len(steps) - len(tiles),
+                "steps_per_part": float(np.mean(tiles)) if tiles else None,
+                "mfma_frac": mfma, "mfma_tflops": flops / (kern_ms * 1e-3) / 1e12, "hbm_gbs": hbm_gbs,
+                "per_launch": f"{2 * S * 2 ** n} B (read + write of the state) and {flops:.3g} flops of the parts' "
+                              f"steps and products on average / {kern_ms:.3f} ms"}
+        if hbm >= mfma:
+            roof.update({"achieved": hbm_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": hbm})
+        else:
+            roof.update({"achieved": mfma * FP64_MFMA_PEAK / 1e12, "peak": FP64_MFMA_PEAK / 1e12, "unit": "TFLOP/s",
+                         "frac": mfma})
 
     verify = None if args.no_verify else verify_small(args.mode, k, depth, partitioner=args.partitioner,
                                                       layout=args.layout, dtype=args.dtype)
