@@ -16,8 +16,8 @@
 //  * HSV_FUSED_F64: v_mfma_f64_16x16x4_f64, FP64 products and accumulation;
 //    most parts as 4-qubit steps on a tile (k_fused_tile, below).
 //  * HSV_FUSED_F32SPLIT: the same FP64 steps where they are the faster way
-//    (15 parts of 6 qubits at 25 qubits 9.6 -> 4.3 ms with their read-outs), and
-//    the more exact one; other parts v_mfma_f32_16x16x4_f32 on hi/lo FP32 splits of U and
+//    (15 parts of 6 qubits at 25 qubits, read-outs included, 9.6 -> 4.3 ms; 3.0
+//    since zero tiles are skipped), and the more exact one; other parts v_mfma_f32_16x16x4_f32 on hi/lo FP32 splits of U and
 //    X (x = hi + lo, hi = fp32(x), lo = fp32(x - hi)); each real product is
 //    hi*hi + hi*lo + lo*hi, accumulated in FP32; the result is stored back in
 //    the state's precision.
@@ -944,7 +944,7 @@ __global__ __launch_bounds__(part_bf_threads(KT, STREAM_U)) __attribute__((amdgp
 // selection, 0.9 ms in all. With one wave going through all states' extensions
 // and absorbing them again a selection took 200 to 700 us; all levels in one
 // workgroup per part, on 10 of the 256 CUs, 2.5 ms. The whole pass at 27
-// qubits: 34.1 -> 13.8 ms.
+// qubits: 34.1 -> 13.8 ms (11.5 with the steps' matrices from the device too).
 constexpr int kPlanGates = 128;   // gates of a part, at most (two 64-bit masks)
 constexpr int kPlanQubits = 14;
 constexpr int kPlanSubsets = 2002;  // C(14, 5)

@@ -85,7 +85,8 @@ struct hsv_state {
   // them after a write): every amplitude with a 1 in another qubit is zero,
   // so the passes skip the tiles, and the gate sweeps the upper part of the
   // state, that hold only such amplitudes: a 31-qubit circuit of 4 layers from
-  // |0...0>, 11 parts and read-outs, takes 126 ms instead of 215.
+  // |0...0>, 11 parts and read-outs, 215 ms without, 126 with (122 since the
+  // read-outs read neighbouring items).
   uint64_t support = ~0ull;
   DeviceScratch fused_scratch;       // fused unitary + offset tables
   // hsv_measure on the device (made at its first use): the walked chunks'
