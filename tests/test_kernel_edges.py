@@ -666,8 +666,8 @@ def test_few_shots_walk_the_serial_sum(n, dtype):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
-@pytest.mark.parametrize("n", [21, 22, 23, 24])
+@pytest.mark.parametrize("n,dtype", [(21, "complex128"), (22, "complex128"), (23, "complex128"), (22, "complex64"),
+                                     (23, "complex64"), (24, "complex64")])
 def test_read_outs_where_the_groups_grow(n, dtype):
     """States around the sizes from which a thread sums eight items at a time
     instead of four: norm, P(0) and strings with X on the lowest, a middle and
